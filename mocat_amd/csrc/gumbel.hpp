@@ -1,0 +1,135 @@
+// Gumbel-max draws by whole wavefronts: argmax_j gumbel_j + logit_j, the first maximum, as
+// random.categorical (mocat/src/ssm/filtering.py:196-199, mocat/src/ssm/backward.py:20-39). The draws are
+// elements of a jax.random bits array (halves layout), gumbel = -log(-log(uniform(tiny, 1))).
+//
+// What bounds it: one threefry block per one or two draws (about 70 integer operations a block), then the
+// two accurate logarithms of each draw. Most draws cannot win, and a bound shows it without the logarithms:
+// with f the draw's uniform, -log(f) >= 1 - f, so gumbel <= -log(1 - f), and 1 - f is exact in FP32. The
+// bound takes one v_log_f32 and a margin (1e-4, above the error of v_log_f32 and of both logf's: a draw's
+// Gumbel is at most 16); adding the logit rounds monotonically, so a candidate whose bound is below the
+// best value seen by the wave is below it too, and is dropped without changing the result. A candidate that
+// is not dropped, a few per row (the chance of a new best falls as one over the draws seen), takes the exact
+// value. A NaN logit is never dropped; a row that met one is drawn again without the bound.
+#pragma once
+#include "common.hpp"
+
+namespace mocat {
+
+constexpr float kGumbelTiny = 1.17549435e-38f;  // float32 tiny: the lower end of jax's gumbel uniforms
+constexpr uint32_t kNoIndex = 0xffffffffu;
+
+MOCAT_DEV float gumbel_exact(uint32_t bits) { return -logf(-logf(uniform_from_bits(bits, kGumbelTiny, 1.f))); }
+
+MOCAT_DEV float gumbel_upper(uint32_t bits) {
+  const float om = 2.0f - __uint_as_float((bits >> 9) | 0x3F800000u);  // 1 - f, in [2^-23, 1]
+  return fmaf(-0.69314718f, __builtin_amdgcn_logf(om), 1e-4f);
+}
+
+// One row's running maximum: each lane keeps the best candidate it evaluated, `top` is the wave's.
+// offer() is called by the whole wave (act: the lane holds a candidate).
+template <bool PRUNE>
+struct GumbelRow {
+  float best = -INFINITY, top = -INFINITY;
+  uint32_t bi = kNoIndex;
+  bool nan = false;
+
+  MOCAT_DEV void offer(bool act, uint32_t j, uint32_t bits, float logit) {
+    const bool c = act && !(PRUNE && gumbel_upper(bits) + logit < top);
+    if (PRUNE && __ballot(c) == 0ull) return;
+    if (c) {
+      const float v = gumbel_exact(bits) + logit;
+      nan = nan || isnan(v);
+      if (bi == kNoIndex || v > best || (v == best && j < bi)) {
+        best = v;
+        bi = j;
+      }
+    }
+    if (PRUNE) top = wave_max(best);
+  }
+
+  // the maximum over the wave, the lower index on ties (first maximum); kNoIndex without candidates
+  MOCAT_DEV uint32_t first_max() const {
+    float b = best;
+    uint32_t i = bi;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+      const float ob = __shfl_xor(b, o, kWave);
+      const uint32_t oi = (uint32_t)__shfl_xor((int)i, o, kWave);
+      if (oi != kNoIndex && (i == kNoIndex || ob > b || (ob == b && oi < i))) {
+        b = ob;
+        i = oi;
+      }
+    }
+    return i;
+  }
+  MOCAT_DEV bool met_nan() const { return __any(nan) != 0; }
+};
+
+// Row m of gumbel(k, (rows, n)) (elements m n + j of S = rows n), any S.
+template <class Logit>
+MOCAT_DEV uint32_t gumbel_row(Key k, uint32_t S, uint32_t off, uint32_t n, int lane, Logit logit) {
+  auto draw = [&](auto& row) {
+    for (uint64_t j0 = 0; j0 < n; j0 += kWave) {
+      const bool act = j0 + (uint64_t)lane < n;
+      const uint32_t j = (uint32_t)j0 + (uint32_t)lane, jc = act ? j : n - 1u;
+      row.offer(act, j, bits_at(k, S, off + jc), logit(jc));
+    }
+  };
+  GumbelRow<true> row;
+  draw(row);
+  if (!row.met_nan()) return row.first_max();
+  GumbelRow<false> all;
+  draw(all);
+  return all.first_max();
+}
+
+// Rows m and m + rows / 2 of gumbel(k, (rows, n)) for an even number of rows: element m n + j and the same
+// element of the other row are the two words of one threefry block.
+template <class Logit>
+MOCAT_DEV void gumbel_row_pair(Key k, uint32_t S, uint32_t off, uint32_t n, int lane, Logit logit, uint32_t& first,
+                               uint32_t& second) {
+  const uint32_t h = S >> 1;
+  auto draw = [&](auto& a, auto& b) {
+    for (uint64_t j0 = 0; j0 < n; j0 += kWave) {
+      const bool act = j0 + (uint64_t)lane < n;
+      const uint32_t j = (uint32_t)j0 + (uint32_t)lane, jc = act ? j : n - 1u;
+      uint32_t w0 = off + jc, w1 = off + jc + h;
+      threefry2x32(k.a, k.b, w0, w1);
+      const float l = logit(jc);
+      a.offer(act, j, w0, l);
+      b.offer(act, j, w1, l);
+    }
+  };
+  GumbelRow<true> a, b;
+  draw(a, b);
+  first = a.first_max();
+  second = b.first_max();
+  if (!a.met_nan() && !b.met_nan()) return;
+  GumbelRow<false> fa, fb;
+  draw(fa, fb);
+  first = fa.first_max();
+  second = fb.first_max();
+}
+
+// Rows of random.categorical(key, lw, (rows,)) by one wave: unit u of the ceil(rows / 2) that cover them
+// is the rows u and u + rows / 2 when rows is even (they share their threefry blocks), else 2u and 2u + 1.
+MOCAT_DEV void categorical_unit(const float* __restrict__ lw, uint32_t n, uint32_t rows, Key key, uint32_t u, int lane,
+                                int32_t* __restrict__ idx) {
+  const uint32_t S = n * rows;
+  auto logit = [&](uint32_t j) { return lw[j]; };
+  if ((rows & 1u) == 0u) {
+    uint32_t a, b;
+    gumbel_row_pair(key, S, u * n, n, lane, logit, a, b);
+    if (lane == 0) {
+      idx[u] = (int32_t)a;
+      idx[u + rows / 2] = (int32_t)b;
+    }
+    return;
+  }
+  for (uint32_t r = 2u * u; r < 2u * u + 2u && r < rows; ++r) {
+    const uint32_t a = gumbel_row(key, S, r * n, n, lane, logit);
+    if (lane == 0) idx[r] = (int32_t)a;
+  }
+}
+
+}  // namespace mocat

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "gumbel.hpp"
 
 using namespace mocat;
 
@@ -547,24 +548,6 @@ MOCAT_DEV void resample_block(WeightFn weight, int64_t n, Key key, int method, u
   __syncthreads();
 }
 
-// random.categorical(key, lw, shape=(n_out,)): argmax_i lw_i + gumbel(key, (n_out, n))[j, i]
-// (first maximum wins), gumbel = -log(-log(uniform(minval=tiny, maxval=1))).
-MOCAT_DEV int32_t categorical_row(const float* __restrict__ lw, int64_t n, Key key, uint32_t S, int64_t j) {
-  float best = -INFINITY;
-  int32_t bi = 0;
-  for (int64_t i = 0; i < n; ++i) {
-    const float u = uniform_from_bits(bits_at(key, S, (uint32_t)(j * n + i)), 1.17549435e-38f, 1.f);
-    const float g = -logf(-logf(u)) + lw[i];
-    if (g > best || (i == 0)) {
-      if (i == 0 || g > best) {
-        best = g;
-        bi = (int32_t)i;
-      }
-    }
-  }
-  return bi;
-}
-
 // ---------------------------------------------------------------- the persistent filter kernel
 struct PfArgs {
   const mocat_pf_filter* filters;
@@ -694,8 +677,8 @@ __global__ __launch_bounds__(NT) void pf_kernel(PfArgs a) {
       const double lse_res = res ? logn : lse;
       if (res) {
         if (a.resampling == 2) {
-          const uint32_t S = (uint32_t)(n * n);
-          for (int64_t j = tid; j < n; j += NT) anc[j] = categorical_row(lwa, n, ik, S, j);
+          for (uint32_t u = tid / kWave; u < (uint32_t)((n + 1) / 2); u += NW)
+            categorical_unit(lwa, (uint32_t)n, (uint32_t)n, ik, u, tid & (kWave - 1), anc);
           __syncthreads();
         } else {
           const float m = (float)(lse);  // any finite shift works: weights are rescaled exactly
@@ -841,37 +824,14 @@ __global__ __launch_bounds__(256) void resample_search_kernel(const uint64_t* __
     idx[j] = ancestor_at(csum, n, W, k, method, u_sys, j);
 }
 
-// random.categorical(key, lw, shape=(n_out,)): one wave per output j, the lanes over the n Gumbel
-// draws of row j (elements j n + i of the (n_out, n) bits array); each lane keeps its first maximum,
-// and a butterfly takes the larger value, the lower index on ties (the first maximum overall).
+// random.categorical(key, lw, shape=(n_out,)): one wave per unit of two outputs, the lanes over the n
+// Gumbel draws of each row of the (n_out, n) matrix.
 __global__ __launch_bounds__(256) void categorical_kernel(const float* __restrict__ lw, int64_t n, int64_t n_out,
                                                           const uint32_t* key, int32_t* idx) {
   const Key k{key[0], key[1]};
-  const uint32_t S = (uint32_t)(n * n_out);
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
-  for (int64_t j = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; j < n_out; j += waves) {
-    float best = -INFINITY;
-    int64_t bi = -1;
-    for (int64_t i = lane; i < n; i += kWave) {
-      const float u = uniform_from_bits(bits_at(k, S, (uint32_t)(j * n + i)), 1.17549435e-38f, 1.f);
-      const float g = -logf(-logf(u)) + lw[i];
-      if (bi < 0 || g > best) {
-        best = g;
-        bi = i;
-      }
-    }
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, kWave);
-      const int64_t oi = (int64_t)__shfl_xor((long long)bi, o, kWave);
-      if (oi >= 0 && (bi < 0 || ob > best || (ob == best && oi < bi))) {
-        best = ob;
-        bi = oi;
-      }
-    }
-    if (lane == 0) idx[j] = (int32_t)bi;
-  }
+  const int64_t units = (n_out + 1) / 2, waves = (int64_t)gridDim.x * (blockDim.x / kWave);
+  for (int64_t u = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; u < units; u += waves)
+    categorical_unit(lw, (uint32_t)n, (uint32_t)n_out, k, (uint32_t)u, threadIdx.x & (kWave - 1), idx);
 }
 
 // ---------------------------------------------------------------- large filters: grid-wide launches per step
@@ -884,7 +844,8 @@ __global__ __launch_bounds__(256) void categorical_kernel(const float* __restric
 //              weights (resampling steps only);
 //   lf_csum    per chunk: the chunk's threefry blocks of the step's split(key, n) (every step), then
 //              offset = sum of the earlier chunks' totals, plus an inclusive block scan;
-//   lf_step    per chunk: ancestor (binary search in the exact prefix sums, or Gumbel-max), then
+//   lf_cat     categorical resampling only: the Gumbel-max rows, one wave per two of them;
+//   lf_step    per chunk: ancestor (binary search in the exact prefix sums, or lf_cat's), then
 //              propagate, weight, outputs and the chunk accumulators of step t+1.
 // The weights are shifted by float(lse) and quantised with the shift of the largest weight exactly as
 // in pf_kernel, so for the same log-weights and key the ancestors are the same.
@@ -958,6 +919,7 @@ struct LfArgs {
   int64_t* bounds;   // [n_chunks] systematic: ancestor of each chunk's first target
   StepKey* skeys;    // [key_slot + t] per filter
   uint32_t* bar;     // persistent kernel: [0] barrier arrivals, [1] abort flag (zeroed by the init launch)
+  int32_t* anc;      // [n_chunks * CH] categorical: the step's ancestors, per filter from chunk0 * CH
   uint32_t* pkeys;   // [n_chunks * CH * 2] the step's split(step key, n), flat, per filter from chunk0 * CH * 2;
                      // null for the optimal proposal (its noise is not drawn from per-particle keys)
 };
@@ -1529,6 +1491,24 @@ __global__ __launch_bounds__(LT) void lf_csum_kernel(LfArgs a, int64_t t) {
   lf_csum_chunk(a, t, blockIdx.x, s, cs);
 }
 
+// Categorical resampling of step t: the Gumbel-max rows of chunk c, block `sub` of its kCatBlocks taking
+// one unit of two rows per wave. The n^2 draws are spread over every workgroup of the launch (a thread
+// that walked its particle's n draws alone took 88 ms for 100 steps of 1024 particles in one workgroup).
+constexpr int kCatBlocks = CH / 2 / LW;
+MOCAT_DEV void lf_cat_block(const LfArgs& a, int64_t t, int64_t c, int sub) {
+  const LfDesc& F = a.cdesc[c];
+  if (t >= F.T || !a.st[F.slot].res) return;
+  const int64_t u = (c - F.chunk0) * (CH / 2) + sub * LW + threadIdx.x / kWave;
+  if (u >= (F.n + 1) / 2) return;
+  const StepKey& sk = a.skeys[F.key_slot + t];
+  categorical_unit(lf_lw_prev(a, t) + F.state_offset, (uint32_t)F.n, (uint32_t)F.n, Key{sk.k[0], sk.k[1]}, (uint32_t)u,
+                   threadIdx.x & (kWave - 1), a.anc + F.chunk0 * CH);
+}
+
+__global__ __launch_bounds__(LT) void lf_cat_kernel(LfArgs a, int64_t t) {
+  lf_cat_block(a, t, blockIdx.x, blockIdx.y);
+}
+
 // dst[k] = src(k) for k < count, by the whole workgroup, U loads per thread issued before their stores.
 template <int U, class Src>
 MOCAT_DEV void stage_lds(uint64_t* dst, int64_t count, Src src) {
@@ -1699,7 +1679,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
   if (res && a.resampling == 2) {
 #pragma unroll
     for (int pk = 0; pk < PPT; ++pk)
-      if (live[pk]) srcs[pk] = categorical_row(lwa, n, ik, (uint32_t)(n * n), srcs[pk]);
+      if (live[pk]) srcs[pk] = a.anc[F.chunk0 * CH + srcs[pk]];
   } else if (res) {
     uint64_t tg[PPT];
 #pragma unroll
@@ -1990,6 +1970,8 @@ __global__ __launch_bounds__(LT) void lf_persist_kernel(LfArgs a, int64_t max_T,
       __syncthreads();
       lf_csum_call(a, t, c, s, buf);
     }
+    if (a.resampling == 2)
+      for (int64_t k = blockIdx.x; k < as * kCatBlocks; k += G) lf_cat_block(a, t, k / kCatBlocks, (int)(k % kCatBlocks));
     if (!lf_grid_sync(a.bar, ++k, max_polls)) return;
     for (int64_t c = blockIdx.x; c < as; c += G) {
       __syncthreads();
@@ -2150,6 +2132,7 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
     for (int64_t t = 1; t < max_T; ++t) {
       hipLaunchKernelGGL((lf_prep_kernel<GRAD>), grid(t - 1), blk, 0, q, a, t);
       hipLaunchKernelGGL(lf_csum_kernel, grid(t), blk, 0, q, a, t);
+      if (a.resampling == 2) hipLaunchKernelGGL(lf_cat_kernel, dim3(grid(t).x, kCatBlocks), blk, 0, q, a, t);
       hipLaunchKernelGGL((lf_step_kernel<Model, D, DY, GRAD>), grid(t), blk, cend_bytes, q, a, t, cend_slots);
     }
     hipLaunchKernelGGL((lf_prep_kernel<GRAD>), grid(max_T - 1), blk, 0, q, a, max_T);  // the last step's statistics
@@ -2196,7 +2179,7 @@ struct LfLayout {
   int cend_slots = 1;  // SG-block end sums the step kernel stages: the largest filter's, up to kChunkEnds
   int64_t n_chunks = 0, max_T = 0;
   int64_t n_tk = 0;  // step-key slots: the sum of T over the flagged filters
-  int64_t o_desc, o_cf, o_m, o_s1, o_s2, o_g, o_tot, o_st, o_cend, o_bnd, o_keys, o_act, o_bar, o_pk, bytes;
+  int64_t o_desc, o_cf, o_m, o_s1, o_s2, o_g, o_tot, o_st, o_cend, o_bnd, o_keys, o_act, o_bar, o_pk, o_anc, bytes;
 };
 
 int64_t lf_align(int64_t v) { return (v + 255) / 256 * 256; }
@@ -2240,6 +2223,8 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters) {
   o = lf_align(o + 8);
   L.o_pk = o;
   o = lf_align(o + L.n_chunks * CH * 8);
+  L.o_anc = o;
+  o = lf_align(o + L.n_chunks * CH * 4);
   L.bytes = o;
   return L;
 }
@@ -2440,7 +2425,7 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
            reinterpret_cast<uint64_t*>(ws + L.o_tot), reinterpret_cast<LfState*>(ws + L.o_st),
            reinterpret_cast<uint64_t*>(ws + L.o_cend), reinterpret_cast<int64_t*>(ws + L.o_bnd),
            reinterpret_cast<StepKey*>(ws + L.o_keys), reinterpret_cast<uint32_t*>(ws + L.o_bar),
-           model == 2 ? nullptr : reinterpret_cast<uint32_t*>(ws + L.o_pk)};
+           reinterpret_cast<int32_t*>(ws + L.o_anc), model == 2 ? nullptr : reinterpret_cast<uint32_t*>(ws + L.o_pk)};
   if (model == 1) {
     if (d != dy) return MOCAT_ERR_ARG;
     if (d != 1 && out_grad) return MOCAT_ERR_ARG;
@@ -2521,7 +2506,7 @@ int mocat_resample_categorical(const float* log_weight, int64_t n, int64_t n_out
                                hipStream_t stream) {
   if (!log_weight || !key || !idx || n <= 0 || n_out <= 0) return MOCAT_ERR_ARG;
   if (n * n_out >= 0xFFFFFFFFll) return MOCAT_ERR_SIZE;
-  const int64_t blocks = (n_out + 3) / 4;  // one wave per output, four per workgroup
+  const int64_t blocks = ((n_out + 1) / 2 + 3) / 4;  // one wave per two outputs, four per workgroup
   hipLaunchKernelGGL(categorical_kernel, dim3((unsigned)(blocks < 65535 ? blocks : 65535)), dim3(256), 0, stream,
                      log_weight, n, n_out, key, idx);
   MOCAT_LAUNCH_CHECK();

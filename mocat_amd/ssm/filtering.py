@@ -415,11 +415,12 @@ def _keys_np(keys):
     return np.stack([_key_np(k) for k in keys]) if len(keys) else np.zeros((0, 2), np.uint32)
 
 
-def _large_flags(ns, Ts, large_n):
+def _large_flags(ns, Ts, large_n, resampling=None):
     """Which filters take the chunked path: those with at least large_n particles (default 4096:
-    above it one workgroup per filter is slower than a few grid-wide launches per time step)."""
+    above it one workgroup per filter is slower than a few grid-wide launches per time step; 256 with
+    categorical resampling, whose n^2 draws per step need the whole GPU)."""
     if large_n is None:
-        large_n = 4096
+        large_n = 256 if resampling == "categorical" else 4096
     return [int(n) >= int(large_n) for n in ns]
 
 
@@ -522,7 +523,7 @@ def _launch(models, ys, keys, ns, ess_threshold, resampling, store, grad=False, 
     F = len(models)
     Ts = [int(np.asarray(y).shape[0]) for y in ys]
     order = sorted(range(F), key=lambda i: -(ns[i] * Ts[i]))  # longest first
-    large = _large_flags(ns, Ts, large_n)
+    large = _large_flags(ns, Ts, large_n, resampling)
     desc = np.zeros(F, FILTER_DTYPE)
     keys_host = _keys_np(keys)
     params, yflat, scales = [], [], []
