@@ -184,7 +184,8 @@ int mocat_pf_run(int model, int d, int dy, const mocat_pf_filter* host_filters, 
  * mocat_pf_run) for those flagged MOCAT_PF_LARGE, spread over the whole GPU: per time step three
  * grid-wide launches over 1024-particle chunks, all flagged filters batched in each (the previous
  * step's statistics, resampling decision and quantised weight totals; exact prefix sums; ancestor
- * search, propagation and weighting). For the same log-weights and key the ancestors equal mocat_pf_run's. host_filters is a
+ * search, propagation and weighting), or one over 256-particle chunks when no flagged filter has more
+ * than 4096 particles (launch modes 0 and 1); categorical resampling adds a launch of its draws. For the same log-weights and key the ancestors equal mocat_pf_run's. host_filters is a
  * host array (the launch sequence depends on n and T); workspace holds
  * mocat_pf_large_workspace_bytes bytes, including T step-key slots per flagged filter (independent of
  * t_offset, which only places out_ess / out_loglik_t and must be >= 0 when either is given).

@@ -849,10 +849,16 @@ __global__ __launch_bounds__(256) void categorical_kernel(const float* __restric
 //              propagate, weight, outputs and the chunk accumulators of step t+1.
 // The weights are shifted by float(lse) and quantised with the shift of the largest weight exactly as
 // in pf_kernel, so for the same log-weights and key the ancestors are the same.
+//
+// Calls whose largest flagged filter has at most kSmallMax particles take one launch per step instead
+// (lf_small_kernel, 256-particle chunks): every workgroup redoes the statistics and the prefix sums of its
+// whole filter, which costs less than two more dependent launches.
 constexpr int LT = 256;          // threads per workgroup
 constexpr int LW = LT / kWave;
 constexpr int PPT = 4;           // particles per thread
 constexpr int CH = LT * PPT;     // particles per chunk (one workgroup)
+constexpr int SCH = LT;          // particles per chunk of the one-launch step: one per thread
+constexpr int kSmallMax = 4096;  // largest filter of the one-launch step
 constexpr int SG = 256;          // prefix-sum search granularity (chunk ends staged in LDS)
 constexpr int kSearchWin = 2048;   // prefix sums of a block's ancestor chunks staged in LDS (16 KB)
 constexpr int kChunkEnds = 4096;   // SG-block end sums staged in LDS (filters up to 2^20 particles);
@@ -1094,7 +1100,8 @@ MOCAT_DEV void lf_store_lse(const LfArgs& a, int64_t c, LseAcc r) {
   }
 }
 
-template <class Model, int D, int DY, bool GRAD>
+// P: particles per thread (chunks of LT * P particles)
+template <class Model, int D, int DY, bool GRAD, int P>
 MOCAT_DEV void lf_init_chunk(const LfArgs& a, int64_t c, LfScratch& s, Model& model) {
   const LfDesc F = a.cdesc[c];
   const int tid = threadIdx.x;
@@ -1124,16 +1131,16 @@ MOCAT_DEV void lf_init_chunk(const LfArgs& a, int64_t c, LfScratch& s, Model& mo
       a.skeys[F.key_slot + t] = sk;
     }
   }
-  float lv[PPT], lt[PPT][3];
-  bool lvalid[PPT];
+  float lv[P], lt[P][3];
+  bool lvalid[P];
 #pragma unroll
-  for (int pk = 0; pk < PPT; ++pk) {
+  for (int pk = 0; pk < P; ++pk) {
     lv[pk] = 0.f;
     lt[pk][0] = lt[pk][1] = lt[pk][2] = 0.f;
     lvalid[pk] = false;
   }
-  for (int pk = 0; pk < PPT; ++pk) {
-    const int64_t i = (c - F.chunk0) * CH + pk * LT + tid;
+  for (int pk = 0; pk < P; ++pk) {
+    const int64_t i = (c - F.chunk0) * (LT * P) + pk * LT + tid;
     if (i >= n) break;
     float eps[D], x[D];
     float l;
@@ -1192,18 +1199,18 @@ MOCAT_DEV void lf_init_chunk(const LfArgs& a, int64_t c, LfScratch& s, Model& mo
   }
   if constexpr (GRAD) {
     double g[3];
-    const LseAcc r = lf_block_lse2g<PPT>(lv, lt, lvalid, s, g);
+    const LseAcc r = lf_block_lse2g<P>(lv, lt, lvalid, s, g);
     lf_store_lse_g(a, c, r, g);
   } else {
-    lf_store_lse(a, c, lf_block_lse2<PPT>(lv, lvalid, s));
+    lf_store_lse(a, c, lf_block_lse2<P>(lv, lvalid, s));
   }
 }
 
-template <class Model, int D, int DY, bool GRAD>
+template <class Model, int D, int DY, bool GRAD, int P>
 __global__ __launch_bounds__(LT) void lf_init_kernel(LfArgs a) {
   __shared__ LfScratch s;
   __shared__ Model model;
-  lf_init_chunk<Model, D, DY, GRAD>(a, blockIdx.x, s, model);
+  lf_init_chunk<Model, D, DY, GRAD, P>(a, blockIdx.x, s, model);
 }
 
 // The prefix sums are integers below 2^52 (exact in FP64), so for a target T >= 0 the test
@@ -1211,6 +1218,63 @@ __global__ __launch_bounds__(LT) void lf_init_kernel(LfArgs a) {
 MOCAT_DEV uint64_t target_floor(double t) { return t > 0.0 ? (uint64_t)floor(t) : 0ull; }
 
 MOCAT_DEV const float* lf_lw_prev(const LfArgs& a, int64_t t) { return ((t - 1) & 1) ? a.lw1 : a.lw0; }
+
+// What a step's combined accumulators say about the next step: the log-sum-exps and ESS, the resampling
+// decision and the weight shift (pf_kernel: m = float(lse), shift from the largest weight exp(lw - m),
+// i.e. exp(max lw - m): the hardware exponential is monotone). They do not depend on the filter state.
+struct LfStats {
+  double lse, ess, logn;
+  float m;
+  int res, shift;
+};
+
+MOCAT_DEV LfStats lf_stats(LseAcc r, int64_t n, float ess_threshold) {
+  LfStats v;
+  double lse2;
+  if (isnan(r.m)) {
+    v.lse = NAN;
+    lse2 = NAN;
+  } else if (r.m == -INFINITY) {
+    v.lse = -INFINITY;
+    lse2 = -INFINITY;
+  } else {
+    v.lse = (double)r.m + log(r.s1);
+    lse2 = 2.0 * (double)r.m + log(r.s2);
+  }
+  v.logn = log((double)n);
+  v.ess = exp(2.0 * v.lse - lse2);
+  v.res = v.ess < (double)ess_threshold * (double)n ? 1 : 0;
+  v.m = (float)v.lse;
+  v.shift = quant_shift(__expf(r.m - v.m), n);
+  return v;
+}
+
+// The filter state and per-step outputs after step tp (one thread of the filter's first chunk).
+template <bool GRAD>
+MOCAT_DEV void lf_update_state(const LfArgs& a, const LfDesc& F, int64_t tp, const LfStats& v, const LseAcc& r,
+                               const double (&gsum)[3]) {
+  LfState st = a.st[F.slot];
+  st.loglik = tp == 0 ? ((F.flags & kPfResume) ? 0.0 : v.lse - v.logn) : st.loglik + v.lse - st.lse_res;
+  if (a.out_ess) a.out_ess[F.t_offset + tp] = (float)v.ess;
+  if (a.out_loglik_t) a.out_loglik_t[F.t_offset + tp] = st.loglik;
+  if constexpr (GRAD) {
+    for (int q = 0; q < 3; ++q) {
+      const double gm = gsum[q] / r.s1;
+      st.gtot[q] = tp == 0 ? gm : st.gtot[q] + gm - (st.res ? 0.0 : st.gprev[q]);
+      st.gprev[q] = gm;
+    }
+  }
+  st.res = v.res;
+  st.lse_res = v.res ? v.logn : v.lse;
+  st.m = v.m;
+  st.shift = v.shift;
+  a.st[F.slot] = st;
+  if (tp == F.T - 1) {
+    a.out_loglik[F.f] = st.loglik;
+    if constexpr (GRAD)
+      for (int q = 0; q < 3; ++q) a.out_grad[(int64_t)F.f * 3 + q] = st.gtot[q];
+  }
+}
 
 // One launch per step t >= 1 (and one after the last step):
 //  * the statistics of step t - 1 (LSE of its weights, ESS, log-likelihood, next resampling decision
@@ -1222,7 +1286,6 @@ MOCAT_DEV const float* lf_lw_prev(const LfArgs& a, int64_t t) { return ((t - 1) 
 template <bool GRAD>
 MOCAT_DEV void lf_prep_chunk(const LfArgs& a, int64_t t, int64_t c, LfScratch& s) {
   const LfDesc F = a.cdesc[c];
-  const int fi = F.slot;
   if (t - 1 >= F.T) return;
   const int64_t n = F.n, nchunk = (n + CH - 1) / CH;
   // the chunk's weights for its quantised total are loaded first: they do not depend on the combine
@@ -1325,52 +1388,11 @@ MOCAT_DEV void lf_prep_chunk(const LfArgs& a, int64_t t, int64_t c, LfScratch& s
     }
     r = LseAcc{anybad ? NAN : M, r1, r2};
   }
-  double lse, lse2;
-  if (isnan(r.m)) {
-    lse = NAN;
-    lse2 = NAN;
-  } else if (r.m == -INFINITY) {
-    lse = -INFINITY;
-    lse2 = -INFINITY;
-  } else {
-    lse = (double)r.m + log(r.s1);
-    lse2 = 2.0 * (double)r.m + log(r.s2);
-  }
-  const double logn = log((double)n);
-  const double ess = exp(2.0 * lse - lse2);
-  // decision and weight shift for step t (pf_kernel: m = float(lse), shift from the largest weight
-  // exp(lw - m), i.e. exp(max lw - m): the hardware exponential is monotone)
-  const int res = ess < (double)a.ess_threshold * (double)n ? 1 : 0;
-  const float m = (float)lse;
-  const int shift = quant_shift(__expf(r.m - m), n);
-  if (c == F.chunk0) {
-    double gm[3] = {0.0, 0.0, 0.0};
-    if constexpr (GRAD)
-      for (int q = 0; q < 3; ++q) gm[q] = gsum[q] / r.s1;
-    if (threadIdx.x == 0) {
-      const int64_t tp = t - 1;
-      LfState st = a.st[fi];
-      st.loglik = tp == 0 ? ((F.flags & kPfResume) ? 0.0 : lse - logn) : st.loglik + lse - st.lse_res;
-      if (a.out_ess) a.out_ess[F.t_offset + tp] = (float)ess;
-      if (a.out_loglik_t) a.out_loglik_t[F.t_offset + tp] = st.loglik;
-      if constexpr (GRAD) {
-        for (int q = 0; q < 3; ++q) {
-          st.gtot[q] = tp == 0 ? gm[q] : st.gtot[q] + gm[q] - (st.res ? 0.0 : st.gprev[q]);
-          st.gprev[q] = gm[q];
-        }
-      }
-      st.res = res;
-      st.lse_res = res ? logn : lse;
-      st.m = m;
-      st.shift = shift;
-      a.st[fi] = st;
-      if (tp == F.T - 1) {
-        a.out_loglik[F.f] = st.loglik;
-        if constexpr (GRAD)
-          for (int q = 0; q < 3; ++q) a.out_grad[(int64_t)F.f * 3 + q] = st.gtot[q];
-      }
-    }
-  }
+  const LfStats v = lf_stats(r, n, a.ess_threshold);
+  if (c == F.chunk0 && threadIdx.x == 0) lf_update_state<GRAD>(a, F, t - 1, v, r, gsum);
+  const bool res = v.res != 0;
+  const float m = v.m;
+  const int shift = v.shift;
   if (t >= F.T || !res || a.resampling == 2) return;
   uint64_t q = 0;
 #pragma unroll
@@ -1872,13 +1894,263 @@ __global__ __launch_bounds__(LT) void lf_step_kernel(LfArgs a, int64_t t, int ce
   lf_step_chunk<Model, D, DY, GRAD>(a, t, cend_slots, blockIdx.x, s, model, win, cend);
 }
 
+// ---------------------------------------------------------------- the one-launch step (n <= kSmallMax)
+// A step of filters up to kSmallMax particles is bound by latency: three dependent launches over four
+// workgroups took 31 us (4096 particles, d = 4; the step kernel 19 of them, four particles per thread).
+// Here a workgroup takes 256 particles, one per thread, and does the whole step: the statistics from the
+// chunk partials of step t - 1 (at most 16, one per lane), the quantised prefix sums of the whole filter
+// in LDS (16 weights per thread), the ancestor of its own particle, propagation, and its partial of step t.
+// Partials alternate between two halves of their arrays, since a workgroup of the same launch may still read
+// the previous step's. The launch of step t also covers filters that ended at T = t (their last statistics).
+
+// The filter's accumulators after step t - 1, in every lane of every wave alike (16 lanes hold the partials,
+// repeated four times over the wave).
+template <bool GRAD>
+MOCAT_DEV LseAcc lf_small_combine(const LfArgs& a, const LfDesc& F, int64_t t, double (&g)[3]) {
+  constexpr int kParts = kSmallMax / SCH;
+  static_assert(kParts == 16, "one partial per lane of a 16-lane group");
+  const int k = threadIdx.x & (kParts - 1);
+  const int nchunk = (int)((F.n + SCH - 1) / SCH);
+  const int64_t cc = ((t - 1) & 1) * a.n_chunks + F.chunk0 + k;
+  const bool have = k < nchunk;
+  float pm = -INFINITY;
+  double s1 = 0.0, s2 = 0.0;
+  g[0] = g[1] = g[2] = 0.0;
+  if (have) {
+    pm = a.part_m[cc];
+    s1 = a.part_s1[cc];
+    s2 = a.part_s2[cc];
+    if constexpr (GRAD)
+      for (int q = 0; q < 3; ++q) g[q] = a.part_g[cc * 3 + q];
+  }
+  const bool bad = __any(isnan(pm)) != 0;
+  float M = isnan(pm) ? -INFINITY : pm;
+#pragma unroll
+  for (int o = kParts / 2; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, kWave));
+  const double f = pm > -INFINITY ? exp((double)pm - (double)M) : 0.0;  // NaN and -inf partials add nothing
+  s1 = f > 0.0 ? s1 * f : 0.0;
+  s2 = f > 0.0 ? s2 * f * f : 0.0;
+  if constexpr (GRAD)
+    for (int q = 0; q < 3; ++q) g[q] = f > 0.0 ? g[q] * f : 0.0;
+#pragma unroll
+  for (int o = kParts / 2; o > 0; o >>= 1) {
+    s1 += __shfl_xor(s1, o, kWave);
+    s2 += __shfl_xor(s2, o, kWave);
+    if constexpr (GRAD)
+      for (int q = 0; q < 3; ++q) g[q] += __shfl_xor(g[q], o, kWave);
+  }
+  return LseAcc{bad ? NAN : M, s1, s2};
+}
+
+// Categorical resampling: the rows of chunk c's kSmallCatBlocks blocks, one unit of two rows per wave; the
+// decision comes from the same combined accumulators as the step kernel's.
+constexpr int kSmallCatBlocks = SCH / 2 / LW;
+__global__ __launch_bounds__(LT) void lf_small_cat_kernel(LfArgs a, int64_t t) {
+  const LfDesc& F = a.cdesc[blockIdx.x];
+  if (t >= F.T) return;
+  const int64_t u = (blockIdx.x - F.chunk0) * (SCH / 2) + blockIdx.y * LW + threadIdx.x / kWave;
+  if (u >= (F.n + 1) / 2) return;
+  double g[3];
+  const LseAcc r = lf_small_combine<false>(a, F, t, g);
+  if (!lf_stats(r, F.n, a.ess_threshold).res) return;
+  const StepKey& sk = a.skeys[F.key_slot + t];
+  categorical_unit(lf_lw_prev(a, t) + F.state_offset, (uint32_t)F.n, (uint32_t)F.n, Key{sk.k[0], sk.k[1]}, (uint32_t)u,
+                   threadIdx.x & (kWave - 1), a.anc + F.chunk0 * SCH);
+}
+
+template <class Model, int D, int DY, bool GRAD>
+__global__ __launch_bounds__(LT) void lf_small_kernel(LfArgs a, int64_t t) {
+  constexpr int TW = 4 * LT;                // weights of one scan tile: four consecutive per thread
+  constexpr int NTILE = kSmallMax / TW;
+  __shared__ LfScratch s;
+  __shared__ Model model;
+  __shared__ uint64_t cs[kSmallMax];        // inclusive prefix sums of the filter's quantised weights
+  __shared__ uint64_t wtot[NTILE][LW];
+  const int64_t c = blockIdx.x;
+  const LfDesc F = a.cdesc[c];
+  if (t - 1 >= F.T) return;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  const int n = (int)F.n, i = (int)(c - F.chunk0) * SCH + tid;
+  const bool live = i < n;
+  const bool odd = (t - 1) & 1, last = t >= F.T;
+  const float* xa = (odd ? a.x1 : a.x0) + F.state_offset * D;
+  float* xb = (odd ? a.x0 : a.x1) + F.state_offset * D;
+  const float* lwa = (odd ? a.lw1 : a.lw0) + F.state_offset;
+  float* lwb = (odd ? a.lw0 : a.lw1) + F.state_offset;
+  // every load that depends on the descriptor only, before the combine
+  const bool sums = a.resampling != 2 && !last;
+  const int ntile = (n + TW - 1) / TW;
+  float wv[NTILE][4];
+#pragma unroll
+  for (int q = 0; q < NTILE; ++q)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int e = q * TW + tid * 4 + k;
+      wv[q][k] = (sums && e < n) ? lwa[e] : 0.f;
+    }
+  const float lwi = (live && !last) ? lwa[i] : 0.f;
+  // read here, as in the other kernels: next to its use the compiler would compile a second transition for
+  // a scale of one, with another contraction
+  float sc = 1.f;
+  if constexpr (Model::kTimeScaled)
+    if (a.step_scale && !last) sc = a.step_scale[F.y_offset / DY + t];
+  StepKey skv{};
+  if (!last) {
+    skv = a.skeys[F.key_slot + t];
+    load_shared_params(model, a.params + F.param_offset);
+  }
+  double gsum[3];
+  const LseAcc r = lf_small_combine<GRAD>(a, F, t, gsum);
+  const LfStats v = lf_stats(r, n, a.ess_threshold);
+  if (c == F.chunk0 && tid == 0) lf_update_state<GRAD>(a, F, t - 1, v, r, gsum);
+  if (last) return;
+  const bool res = v.res != 0;
+  const Key ik{skv.k[0], skv.k[1]};
+  if (res && sums) {
+    uint64_t incl[NTILE], own[NTILE];
+#pragma unroll
+    for (int q = 0; q < NTILE; ++q) {
+      own[q] = 0ull;
+      incl[q] = 0ull;
+      if (q >= ntile) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (q * TW + tid * 4 + k < n) own[q] += quantise(__expf(wv[q][k] - v.m), v.shift);
+      incl[q] = wave_inclusive_scan(own[q]);
+      if (lane == kWave - 1) wtot[q][w] = incl[q];
+    }
+    __syncthreads();
+    uint64_t base = 0ull;
+#pragma unroll
+    for (int q = 0; q < NTILE; ++q) {
+      if (q >= ntile) continue;
+      uint64_t run = base + incl[q] - own[q];
+#pragma unroll
+      for (int k = 0; k < LW; ++k) {
+        const uint64_t tk = wtot[q][k];
+        if (k < w) run += tk;
+        base += tk;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int e = q * TW + tid * 4 + k;
+        if (e < n) {
+          run += quantise(__expf(wv[q][k] - v.m), v.shift);
+          cs[e] = run;
+        }
+      }
+    }
+  }
+  // the particle's noise does not depend on its ancestor
+  float eps[D];
+  if constexpr (Model::kOptimal) {
+    shared_eps<D>(Key{skv.k[2], skv.k[3]}, (uint32_t)(n * D), (uint32_t)(live ? i : 0), eps);
+  } else {
+    const Key ki = split_at(ik, (uint32_t)n, (uint32_t)(live ? i : 0));
+    constexpr uint32_t hD = (D + 1) / 2;
+#pragma unroll
+    for (uint32_t q = 0; q < hD; ++q) {
+      uint32_t w0, w1;
+      bits_pair(ki, D, q, w0, w1);
+      eps[q] = normal_from_bits(w0);
+      if (q + hD < (uint32_t)D) eps[q + hD] = normal_from_bits(w1);
+    }
+  }
+  __syncthreads();
+  int src = i;
+  if (live && res) {
+    if (a.resampling == 2) {
+      src = a.anc[F.chunk0 * SCH + i];
+    } else {
+      const double W = (double)cs[n - 1];
+      const uint64_t tg = target_floor(a.resampling == 0
+                                           ? ((double)i + (double)skv.su) * (W / (double)n)
+                                           : (double)uniform_from_bits(bits_at(ik, (uint32_t)n, (uint32_t)i), 0.f, 1.f) * W);
+      int lo = 0, len = n;
+      while (len > 0) {
+        const int h = len >> 1;
+        if (cs[lo + h] <= tg) {
+          lo += h + 1;
+          len -= h + 1;
+        } else {
+          len = h;
+        }
+      }
+      src = lo < n ? lo : n - 1;
+    }
+  }
+  const float* ycur = a.y + F.y_offset + t * DY;
+  float l = 0.f, gd[1][3] = {{0.f, 0.f, 0.f}};
+  if (live) {
+    float xp[D], xn[D];
+#pragma unroll
+    for (int q = 0; q < D; ++q) xp[q] = xa[(int64_t)src * D + q];
+    const float lw0 = res ? 0.f : lwi;
+    // the tangents are read before the arithmetic: a conditional load between a product and its sum keeps
+    // the two from contracting as they do in the other kernels
+    float tg[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (GRAD) {
+      const float* ta = (odd ? a.tan1 : a.tan0) + F.state_offset * 5;
+      tg[0] = ta[src * 5 + 0];
+      tg[1] = ta[src * 5 + 1];
+#pragma unroll
+      for (int q = 2; q < 5; ++q) tg[q] = res ? 0.f : ta[i * 5 + q];
+    }
+    if constexpr (Model::kOptimal) {
+      l = lw0 - model.step_opt(xp, eps, ycur, xn);
+    } else {
+      if constexpr (Model::kTimeScaled)
+        model.transition_s(xp, eps, xn, sc);
+      else
+        model.transition(xp, eps, xn);
+      if constexpr (GRAD) {
+        float* tb = (odd ? a.tan0 : a.tan1) + F.state_offset * 5;
+        float dldx, dldb;
+        l = lw0 - model.lik_grad(xn, ycur, dldx, dldb);
+        const float dxp = xp[0] + model.phi * tg[0];
+        const float dxs = eps[0] * sc + model.phi * tg[1];
+        gd[0][0] = tg[2] - dldx * dxp;
+        gd[0][1] = tg[3] - dldx * dxs;
+        gd[0][2] = tg[4] - dldb;
+        tb[i * 5 + 0] = dxp;
+        tb[i * 5 + 1] = dxs;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) tb[i * 5 + 2 + q] = gd[0][q];
+      } else {
+        l = lw0 - model.lik(xn, ycur);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < D; ++q) xb[(int64_t)i * D + q] = xn[q];
+    lwb[i] = l;
+    if (F.out_offset >= 0) {
+      const int64_t o = F.out_offset + t * F.n + i;
+      if (a.out_value)
+#pragma unroll
+        for (int q = 0; q < D; ++q) a.out_value[o * D + q] = xn[q];
+      if (a.out_lw) a.out_lw[o] = l;
+      if (a.out_anc) a.out_anc[o] = src;
+    }
+  }
+  const float lv[1] = {l};
+  const bool lvalid[1] = {live};
+  const int64_t po = (t & 1) * a.n_chunks + c;
+  if constexpr (GRAD) {
+    double g[3];
+    const LseAcc acc = lf_block_lse2g<1>(lv, gd, lvalid, s, g);
+    lf_store_lse_g(a, po, acc, g);
+  } else {
+    lf_store_lse(a, po, lf_block_lse2<1>(lv, lvalid, s));
+  }
+}
+
 // Final particles of filters whose last step wrote buffer 1 are copied to buffer 0 (as pf_kernel).
-template <int D>
+template <int D, int P>
 MOCAT_DEV void lf_finish_chunk(const LfArgs& a, int64_t c) {
   const LfDesc F = a.cdesc[c];
   if (!((F.T - 1) & 1)) return;
-  for (int pk = 0; pk < PPT; ++pk) {
-    const int64_t i = (c - F.chunk0) * CH + pk * LT + threadIdx.x;
+  for (int pk = 0; pk < P; ++pk) {
+    const int64_t i = (c - F.chunk0) * (LT * P) + pk * LT + threadIdx.x;
     if (i >= F.n) return;
 #pragma unroll
     for (int q = 0; q < D; ++q) a.x0[(F.state_offset + i) * D + q] = a.x1[(F.state_offset + i) * D + q];
@@ -1886,9 +2158,9 @@ MOCAT_DEV void lf_finish_chunk(const LfArgs& a, int64_t c) {
   }
 }
 
-template <int D>
+template <int D, int P>
 __global__ __launch_bounds__(LT) void lf_finish_kernel(LfArgs a) {
-  lf_finish_chunk<D>(a, blockIdx.x);
+  lf_finish_chunk<D, P>(a, blockIdx.x);
 }
 
 // Grid-wide barrier of the persistent kernel. Every workgroup adds one to the arrival counter after a
@@ -1985,7 +2257,7 @@ __global__ __launch_bounds__(LT) void lf_persist_kernel(LfArgs a, int64_t max_T,
     lf_prep_call<GRAD>(a, max_T, c, s);  // the last step's statistics
   }
   if (!lf_grid_sync(a.bar, ++k, max_polls)) return;
-  for (int64_t c = blockIdx.x; c < a.n_chunks; c += G) lf_finish_chunk<D>(a, c);
+  for (int64_t c = blockIdx.x; c < a.n_chunks; c += G) lf_finish_chunk<D, PPT>(a, c);
 }
 
 // After the persistent kernel: if a barrier gave up, every filter's log-likelihood (and gradient) is NaN.
@@ -2104,7 +2376,7 @@ constexpr int kPersistBlocksPerCu = 4;
 
 template <class Model, int D, int DY, bool GRAD = false>
 int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_t* act_dev,
-                    const std::vector<int32_t>& act, int launch_mode, hipStream_t st) {
+                    const std::vector<int32_t>& act, bool small, int launch_mode, hipStream_t st) {
   const dim3 chunks((unsigned)a.n_chunks), blk(LT);
   // the block-end sums are staged only by the multinomial search
   const size_t cend_bytes = a.resampling == 1 ? (size_t)cend_slots * sizeof(uint64_t) : 0;
@@ -2119,7 +2391,7 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
       return MOCAT_ERR_HIP;
     if (per_cu < 1 || cus < 1) return MOCAT_ERR_SIZE;
     const int64_t G = std::min<int64_t>(a.n_chunks, (int64_t)cus * std::min(per_cu, kPersistBlocksPerCu));
-    hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD>), chunks, blk, 0, st, a);
+    hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD, PPT>), chunks, blk, 0, st, a);
     uint32_t max_polls = kBarrierPolls;
     if (const char* e = std::getenv("MOCAT_PF_BARRIER_POLLS")) max_polls = (uint32_t)std::strtoul(e, nullptr, 10);
     hipLaunchKernelGGL(kern, dim3((unsigned)G), blk, cend_bytes, st, a, max_T, cend_slots, act_dev, max_polls);
@@ -2128,7 +2400,17 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
     return MOCAT_OK;
   }
   auto enqueue = [&](hipStream_t q) {
-    hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD>), chunks, blk, 0, q, a);
+    if (small) {
+      hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD, 1>), chunks, blk, 0, q, a);
+      for (int64_t t = 1; t <= max_T; ++t) {
+        if (a.resampling == 2 && t < max_T)
+          hipLaunchKernelGGL(lf_small_cat_kernel, dim3(grid(t).x, kSmallCatBlocks), blk, 0, q, a, t);
+        hipLaunchKernelGGL((lf_small_kernel<Model, D, DY, GRAD>), grid(t - 1), blk, 0, q, a, t);
+      }
+      hipLaunchKernelGGL((lf_finish_kernel<D, 1>), chunks, blk, 0, q, a);
+      return;
+    }
+    hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD, PPT>), chunks, blk, 0, q, a);
     for (int64_t t = 1; t < max_T; ++t) {
       hipLaunchKernelGGL((lf_prep_kernel<GRAD>), grid(t - 1), blk, 0, q, a, t);
       hipLaunchKernelGGL(lf_csum_kernel, grid(t), blk, 0, q, a, t);
@@ -2136,7 +2418,7 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
       hipLaunchKernelGGL((lf_step_kernel<Model, D, DY, GRAD>), grid(t), blk, cend_bytes, q, a, t, cend_slots);
     }
     hipLaunchKernelGGL((lf_prep_kernel<GRAD>), grid(max_T - 1), blk, 0, q, a, max_T);  // the last step's statistics
-    hipLaunchKernelGGL((lf_finish_kernel<D>), chunks, blk, 0, q, a);
+    hipLaunchKernelGGL((lf_finish_kernel<D, PPT>), chunks, blk, 0, q, a);
   };
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (launch_mode == 1 && hipStreamIsCapturing(st, &cap) != hipSuccess) return MOCAT_ERR_HIP;
@@ -2184,12 +2466,20 @@ struct LfLayout {
 
 int64_t lf_align(int64_t v) { return (v + 255) / 256 * 256; }
 
-LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters) {
+// Whether the flagged filters of a call take the one-launch step.
+bool lf_small(const mocat_pf_filter* filters, int n_filters) {
+  for (int f = 0; f < n_filters; ++f)
+    if ((filters[f].flags & kPfLarge) && filters[f].n > kSmallMax) return false;
+  return true;
+}
+
+LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters, bool small) {
+  const int64_t ch = small ? SCH : CH, parts = small ? 2 : 1;  // partials alternate in the one-launch step
   LfLayout L;
   for (int f = 0; f < n_filters; ++f) {
     if (!(filters[f].flags & kPfLarge)) continue;
     ++L.n_large;
-    L.n_chunks += (filters[f].n + CH - 1) / CH;
+    L.n_chunks += (filters[f].n + ch - 1) / ch;
     L.max_T = std::max<int64_t>(L.max_T, filters[f].T);
     L.n_tk += std::max<int64_t>(filters[f].T, 0);
     L.cend_slots = (int)std::min<int64_t>(kChunkEnds, std::max<int64_t>(L.cend_slots, (filters[f].n + SG - 1) / SG));
@@ -2200,19 +2490,19 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters) {
   L.o_cf = o;
   o = lf_align(o + L.n_chunks * (int64_t)sizeof(LfDesc));
   L.o_m = o;
-  o = lf_align(o + L.n_chunks * 4);
+  o = lf_align(o + parts * L.n_chunks * 4);
   L.o_s1 = o;
-  o = lf_align(o + L.n_chunks * 8);
+  o = lf_align(o + parts * L.n_chunks * 8);
   L.o_s2 = o;
-  o = lf_align(o + L.n_chunks * 8);
+  o = lf_align(o + parts * L.n_chunks * 8);
   L.o_g = o;
-  o = lf_align(o + L.n_chunks * 24);
+  o = lf_align(o + parts * L.n_chunks * 24);
   L.o_tot = o;
   o = lf_align(o + L.n_chunks * 8);
   L.o_st = o;
   o = lf_align(o + (int64_t)L.n_large * (int64_t)sizeof(LfState));
   L.o_cend = o;
-  o = lf_align(o + L.n_chunks * (CH / SG) * 8);
+  o = lf_align(o + L.n_chunks * (ch / SG) * 8);
   L.o_bnd = o;
   o = lf_align(o + L.n_chunks * 8);
   L.o_keys = o;
@@ -2222,9 +2512,9 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters) {
   L.o_bar = o;
   o = lf_align(o + 8);
   L.o_pk = o;
-  o = lf_align(o + L.n_chunks * CH * 8);
+  o = lf_align(o + L.n_chunks * ch * 8);
   L.o_anc = o;
-  o = lf_align(o + L.n_chunks * CH * 4);
+  o = lf_align(o + L.n_chunks * ch * 4);
   L.bytes = o;
   return L;
 }
@@ -2355,7 +2645,9 @@ int mocat_pf_run(int model, int d, int dy, const mocat_pf_filter* host_filters, 
 
 int mocat_pf_large_workspace_bytes(const mocat_pf_filter* host_filters, int n_filters, int64_t* bytes) {
   if (!host_filters || n_filters < 0 || !bytes) return MOCAT_ERR_ARG;
-  *bytes = lf_layout(host_filters, n_filters).bytes;
+  *bytes = lf_layout(host_filters, n_filters, false).bytes;
+  if (lf_small(host_filters, n_filters))  // either path may run (launch_mode 2 keeps the chunks of CH)
+    *bytes = std::max(*bytes, lf_layout(host_filters, n_filters, true).bytes);
   return MOCAT_OK;
 }
 
@@ -2369,7 +2661,9 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
       !out_loglik || resampling < 0 || resampling > 2 || launch_mode < 0 || launch_mode > 2)
     return MOCAT_ERR_ARG;
   if (out_grad && (model != 1 || !tan_ws0 || !tan_ws1)) return MOCAT_ERR_ARG;
-  const LfLayout L = lf_layout(host_filters, n_filters);
+  const bool small = launch_mode != 2 && lf_small(host_filters, n_filters);
+  const int64_t ch = small ? SCH : CH;
+  const LfLayout L = lf_layout(host_filters, n_filters, small);
   if (L.n_large == 0) return MOCAT_OK;
   if (!workspace || workspace_bytes < L.bytes) return MOCAT_ERR_SIZE;
   if (L.n_chunks > 0x7FFFFFFFll || L.n_large > 0x7FFFFFFF) return MOCAT_ERR_SIZE;
@@ -2394,7 +2688,7 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
     if (resampling == 2 && F.n * F.n >= 0xFFFFFFFFll) return MOCAT_ERR_SIZE;
     if (model == 2 && F.n * (int64_t)d > 0xFFFFFFFFll) return MOCAT_ERR_SIZE;
     if (out_grad && (F.flags & kPfResume)) return MOCAT_ERR_ARG;
-    const int64_t nchunk = (F.n + CH - 1) / CH;
+    const int64_t nchunk = (F.n + ch - 1) / ch;
     desc.push_back(LfDesc{F.n, F.T, F.y_offset, F.state_offset, F.out_offset, F.t_offset, chunk0, key_slot,
                           {F.key[0], F.key[1]}, F.param_offset, f, F.flags, (int32_t)desc.size()});
     key_slot += F.T;
@@ -2404,7 +2698,7 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
   // act[t]: chunks of the filters with T > t, t = 0 .. max_T
   std::vector<int32_t> act((size_t)L.max_T + 1, 0);
   for (const LfDesc& F : desc) {
-    const int32_t nchunk = (int32_t)((F.n + CH - 1) / CH);
+    const int32_t nchunk = (int32_t)((F.n + ch - 1) / ch);
     for (int64_t t = 0; t < F.T; ++t) act[(size_t)t] += nchunk;
   }
   char* ws = static_cast<char*>(workspace);
@@ -2429,23 +2723,23 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
   if (model == 1) {
     if (d != dy) return MOCAT_ERR_ARG;
     if (d != 1 && out_grad) return MOCAT_ERR_ARG;
-    if (d == 2) return launch_pf_large<SvD<2>, 2, 2>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
-    if (d == 3) return launch_pf_large<SvD<3>, 3, 3>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
-    if (d == 4) return launch_pf_large<SvD<4>, 4, 4>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
+    if (d == 2) return launch_pf_large<SvD<2>, 2, 2>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
+    if (d == 3) return launch_pf_large<SvD<3>, 3, 3>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
+    if (d == 4) return launch_pf_large<SvD<4>, 4, 4>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
     if (d != 1) return MOCAT_ERR_ARG;
-    return out_grad ? launch_pf_large<Sv, 1, 1, true>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream)
-                    : launch_pf_large<Sv, 1, 1>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
+    return out_grad ? launch_pf_large<Sv, 1, 1, true>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream)
+                    : launch_pf_large<Sv, 1, 1>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
   }
   if (model == 2) {
 #define MOCAT_PF_CASE(DD, YY) \
-  if (d == DD && dy == YY) return launch_pf_large<LgssmOpt<DD, YY>, DD, YY>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
+  if (d == DD && dy == YY) return launch_pf_large<LgssmOpt<DD, YY>, DD, YY>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
     MOCAT_PF_LG_SHAPES
 #undef MOCAT_PF_CASE
     return MOCAT_ERR_ARG;
   }
   if (model != 0) return MOCAT_ERR_ARG;
 #define MOCAT_PF_CASE(DD, YY) \
-  if (d == DD && dy == YY) return launch_pf_large<Lgssm<DD, YY>, DD, YY>(a, L.max_T, L.cend_slots, act_dev, act, launch_mode, stream);
+  if (d == DD && dy == YY) return launch_pf_large<Lgssm<DD, YY>, DD, YY>(a, L.max_T, L.cend_slots, act_dev, act, small, launch_mode, stream);
   MOCAT_PF_LG_SHAPES
 #undef MOCAT_PF_CASE
   return MOCAT_ERR_ARG;

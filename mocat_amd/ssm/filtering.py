@@ -416,11 +416,26 @@ def _keys_np(keys):
 
 
 def _large_flags(ns, Ts, large_n, resampling=None):
-    """Which filters take the chunked path: those with at least large_n particles (default 4096:
-    above it one workgroup per filter is slower than a few grid-wide launches per time step; 256 with
-    categorical resampling, whose n^2 draws per step need the whole GPU)."""
+    """Which filters take the chunked path: those with at least large_n particles, by default the sizes
+    above which one workgroup per filter is slower than grid-wide launches per time step (50 steps, d = 4,
+    one workgroup / chunked, with the call's 0.5 ms on the host):
+    * 128 with categorical resampling, whose n^2 draws per step need the whole GPU (64 particles: 0.90 /
+      0.93 ms, 128: 1.66 / 0.97, 1024: 29.6 / 1.29);
+    * without filters of 4096 or more, 1024 (one filter of 512 particles 0.68 / 0.67 ms, of 1024 0.96 /
+      0.68, of 4095 2.85 / 0.81; 64 of 4095 3.24 / 1.78), unless those of 1024 to 4095 particles fill the
+      GPU with a workgroup each (256 of 4095: 4.93 / 5.21), then 4096;
+    * beside filters of 4096 or more, whose launches they join: 1024, or every filter when those below 1024
+      add fewer chunks than are there (a second stream for a few small filters may share a hardware queue
+      with the first, and the two then run one after the other)."""
     if large_n is None:
-        large_n = 256 if resampling == "categorical" else 4096
+        ns = [int(n) for n in ns]
+        chunks = sum(-(-n // 1024) for n in ns if n >= 4096)
+        if resampling == "categorical":
+            large_n = 128
+        elif chunks:
+            large_n = 1 if sum(n < 1024 for n in ns) <= chunks else 1024
+        else:
+            large_n = 1024 if sum(n for n in ns if n >= 1024) <= 2 ** 19 else 4096
     return [int(n) >= int(large_n) for n in ns]
 
 
@@ -784,8 +799,8 @@ def run_particle_filters(ssm_scenarios, ys, random_keys, ns, ess_threshold: floa
     """Independent bootstrap filters of uneven sizes in one launch. Returns a list of cdicts with
     log_likelihood (FP64), ess (T,), final_value, final_log_weight (and value/log_weight/ancestors when
     store=True). grad=True (stochastic volatility): log_likelihood_grad = d log Z / d(phi, sigma, beta)
-    of the fixed-resampling-index estimator. Filters with at least large_n particles (default 4096)
-    run on the chunked path spread over the whole GPU; the results do not depend on the path.
+    of the fixed-resampling-index estimator. Filters with at least large_n particles (default by
+    _large_flags) run on the chunked path spread over the whole GPU; the results do not depend on the path.
     particle_filter: BootstrapFilter (default) or OptimalNonLinearGaussianParticleFilter.
     schedule: None (large_n as given, stream launches), a dict {"large_n": int, "launch": "stream" |
     "graph" | "persistent"} (or {"large_n": int, "graph": bool}), or "auto": the schedule autotuner (mocat_amd.ssm.schedule) times the candidate schedules on this
