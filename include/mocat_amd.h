@@ -257,6 +257,14 @@ int mocat_resample_categorical(const float* log_weight, int64_t n, int64_t n_out
 int mocat_ffbsi_step(int model, int d, const float* params, const float* particles, const float* log_weight,
                      int64_t n, const float* x_next, int64_t m, const uint32_t* key, int32_t* idx, float* x_out,
                      hipStream_t stream);
+/* backward_simulation_full's loop (mocat/src/ssm/backward.py:210-243): mocat_ffbsi_step for t = T - 2 .. 0 on
+ * particles [T][n][d], log_weight [T][n] and step keys [T][2], writing rows T - 2 .. 0 of idx [T][m] and x_out
+ * [T][m][d] (row T - 1 of x_out is read). The same draws as the steps one by one; workspace holds
+ * mocat_ffbsi_workspace_bytes(model, d, T, n, m) bytes (may be 0). */
+int mocat_ffbsi_workspace_bytes(int model, int d, int64_t T, int64_t n, int64_t m, int64_t* bytes);
+int mocat_ffbsi_run(int model, int d, const float* params, const float* particles, const float* log_weight, int64_t T,
+                    int64_t n, int64_t m, const uint32_t* keys, void* workspace, int64_t workspace_bytes, int32_t* idx,
+                    float* x_out, hipStream_t stream);
 /* ---- Backward simulation by rejection (replaces mocat/src/ssm/backward.py:42-194, one step of the
  * scan in backward_simulation_rejection, :197-207): initial categorical proposals, accept/reject
  * rounds against a shared density bound (raised by the inflation factor when exceeded, which sends

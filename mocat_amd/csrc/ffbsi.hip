@@ -4,13 +4,17 @@
 //   x_t[m] = particles_t[argmax_j(gumbel(key_m, (N,))[j] + log_weight_t[j] - U(particles_t[j] -> x_{t+1}[m]))]
 // (random.categorical: the first maximum wins), U the model's transition potential as mocat's
 // gaussian_potential evaluates it (utils.py:49-105): 0.5 |(x' - A x) @ S|^2 + nlz, S the transition
-// precision square root. One wave per trajectory: the lanes take pairs (j, j + N/2), whose Gumbel bits
-// come out of one threefry block (the halves layout), and keep a running maximum; a butterfly with
-// the lower index winning ties combines them. Work per step: N x M potentials and N x M / 2 threefry
-// blocks.
+// precision square root. One wave per trajectory (or a workgroup, when there are few): the lanes take
+// pairs (j, j + N/2), whose Gumbel bits come out of one threefry block (the halves layout), and keep a
+// running maximum; a butterfly with the lower index winning ties combines them. Work per step: N x M / 2
+// threefry blocks, N x M bounds of the scores, and the potentials and accurate logarithms of the draws that
+// the bounds do not drop (gumbel.hpp; a few per trajectory). Kernel time of a step of 4096 x 4096 without and
+// with the bounds: d = 1 45 and 35 us, d = 4 59 and 39, d = 8 150 and 57 (threefry and bound, about 50
+// operations a pair, are then what is left); 4096 x 1024, d = 4: 28 and, four waves a trajectory, 17.5.
 #include <cmath>
 
 #include "common.hpp"
+#include "gumbel.hpp"
 
 using namespace mocat;
 
@@ -46,6 +50,32 @@ struct LgTrans {
     }
     return 0.5f * s + nlz;
   }
+  // u = x @ S and a = max_k sum_i |x_i S_ik|
+  MOCAT_DEV void project(const float* x, float* u, float& a) const {
+    a = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      float v = 0.f, b = 0.f;
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        v += x[i] * S[i * D + k];
+        b += fabsf(x[i] * S[i * D + k]);
+      }
+      u[k] = v;
+      a = b > a || isnan(b) ? b : a;
+    }
+  }
+  MOCAT_DEV void project_mean(const float* xp, float* u, float& a) const {
+    float ax[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      float m = 0.f;
+#pragma unroll
+      for (int k = 0; k < D; ++k) m += A[i * D + k] * xp[k];
+      ax[i] = m;
+    }
+    project(ax, u, a);
+  }
 };
 
 // stochastic volatility, unit steps (stochastic_volatility.py:78-84): params phi, 1/sigma, nlz
@@ -59,6 +89,14 @@ struct SvTrans {
   MOCAT_DEV float pot(const float* xp, const float* xn) const {
     const float diff = xn[0] - xp[0] * phi;
     return 0.5f * (diff * diff) * (isig * isig) + nlz;
+  }
+  MOCAT_DEV void project(const float* x, float* u, float& a) const {
+    u[0] = x[0] * isig;
+    a = fabsf(u[0]);
+  }
+  MOCAT_DEV void project_mean(const float* xp, float* u, float& a) const {
+    const float m = phi * xp[0];
+    project(&m, u, a);
   }
 };
 
@@ -94,56 +132,51 @@ struct LgTransRt {
   }
 };
 
-constexpr float kTiny = 1.17549435e-38f;  // float32 tiny: the lower end of jax's gumbel uniforms
-
-// argmax_j(gumbel_j + logit(j)) over j < n for one wave (the first maximum): the Gumbel draws are
-// elements off + j of a bits array of size S under key k (off = 0, S = n: gumbel(k, (n,)); off = m n,
-// S = M n: row m of gumbel(k, (M, n))). When off = 0 and S = n, the lanes take pairs (j, j + n/2),
-// whose bits come out of one threefry block.
-template <class Logit>
-MOCAT_DEV int64_t gumbel_argmax_wave(Key k, uint32_t S, uint64_t off, int64_t n, int lane, Logit logit) {
-  float best = -INFINITY;
-  int64_t bi = n;  // no candidate yet
-  auto consider = [&](int64_t j, uint32_t bits) {
-    const float u = uniform_from_bits(bits, kTiny, 1.f);
-    const float v = -logf(-logf(u)) + logit(j);
-    if (bi == n || v > best || (v == best && j < bi)) {
-      best = v;
-      bi = j;
-    }
-  };
-  if (off == 0 && (uint64_t)S == (uint64_t)n) {
-    const uint32_t h = (S + 1u) >> 1;
-    for (int64_t j = lane; j < h; j += kWave) {
-      uint32_t w0, w1;
-      bits_pair(k, S, (uint32_t)j, w0, w1);
-      consider(j, w0);
-      if (j + h < n) consider(j + h, w1);
-    }
-  } else {
-    for (int64_t j = lane; j < n; j += kWave) consider(j, bits_at(k, S, (uint32_t)(off + j)));
-  }
-  // the maximum over the wave, the lower index on ties (first maximum)
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) {
-    const float ob = __shfl_xor(best, o, kWave);
-    const int64_t oi = (int64_t)__shfl_xor((long long)bi, o, kWave);
-    if (oi != n && (bi == n || ob > best || (ob == best && oi < bi))) {
-      best = ob;
-      bi = oi;
-    }
-  }
-  return bi == n ? 0 : bi;  // n >= 1: lane 0 always ends with a candidate
+// Bounds of the logits lw_j - U(x_j -> x'), prepared once per filter particle: U = 0.5 |v|^2 + nlz with
+// v = (x' - A x) @ S = x' @ S - p, p = (A x) @ S, so a pair's bound takes D subtractions and D FMAs from p and
+// x' @ S, and no product with A or S. Rounding: a component of that difference is within
+// delta = kRoundings * 2^-24 (a_j + a_m) of the v that pot() forms, a = max_k sum_i |(A x)_i S_ik| (a_m the same
+// of x'), and (v - delta)^2 >= (1 - kEta) v^2 - delta^2 / kEta, with kEta also above the relative error of the
+// squared norm. The sums' own rounding is below 1e-6 (|lw| + |nlz|). Filter particle j carries its share of these
+// slacks in `lim`; a non-finite state leaves NaN or infinity there, which drops nothing.
+constexpr float kEta = 1e-3f, kRoundings = 64.f;
+MOCAT_DEV float rounding_slack(float a) {
+  const float e = kRoundings * 5.9604645e-8f * a;  // (a_j + a_m)^2 <= 2 (a_j^2 + a_m^2)
+  return e * e / kEta;
 }
 
+// One thread per particle of a block of time points: pre[k] = {p[D], lim}.
 template <class Tr, int D>
+__global__ __launch_bounds__(256) void ffbsi_prep_kernel(const float* __restrict__ params, const float* __restrict__ xs,
+                                                         const float* __restrict__ lw, int64_t count,
+                                                         float* __restrict__ p, float* __restrict__ lim) {
+  Tr tr;
+  tr.load(params, D);
+  for (int64_t k = blockIdx.x * (int64_t)256 + threadIdx.x; k < count; k += (int64_t)gridDim.x * 256) {
+    float pj[D], a;
+    tr.project_mean(xs + k * D, pj, a);
+#pragma unroll
+    for (int q = 0; q < D; ++q) p[k * D + q] = pj[q];
+    const float l = lw[k];
+    lim[k] = l == -INFINITY ? l : l - tr.nlz + 1e-6f * (fabsf(l) + fabsf(tr.nlz)) + (float)D * rounding_slack(a);
+  }
+}
+
+// W waves per trajectory: 1, or all four of a workgroup. p, lim: the prepared bounds of these particles, or
+// null (then lw - nlz bounds a logit).
+template <class Tr, int D, int W>
 __global__ __launch_bounds__(256) void ffbsi_step_kernel(const float* __restrict__ params,
                                                          const float* __restrict__ xs, const float* __restrict__ lw,
+                                                         const float* __restrict__ p, const float* __restrict__ lim,
                                                          int64_t n, const float* __restrict__ xnext, int64_t m_count,
                                                          const uint32_t* __restrict__ key, int32_t* __restrict__ idx,
                                                          float* __restrict__ xout) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t m = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+  constexpr int kWaves = 256 / kWave;
+  static_assert(W == 1 || W == kWaves, "one wave or the whole workgroup per trajectory");
+  __shared__ float wbest[kWaves];
+  __shared__ uint32_t wi[kWaves];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int64_t m = W == 1 ? (int64_t)blockIdx.x * kWaves + w : (int64_t)blockIdx.x;
   if (m >= m_count) return;
   Tr tr;
   tr.load(params, D);
@@ -151,18 +184,57 @@ __global__ __launch_bounds__(256) void ffbsi_step_kernel(const float* __restrict
   float xn[D];
 #pragma unroll
   for (int q = 0; q < D; ++q) xn[q] = xnext[m * D + q];
-  const int64_t bi = gumbel_argmax_wave(km, (uint32_t)n, 0, n, lane,
-                                        [&](int64_t j) { return lw[j] - tr.pot(xs + j * D, xn); });
+  const uint32_t part = W == 1 ? 0u : (uint32_t)w;
+  auto logit = [&](uint32_t j) { return lw[j] - tr.pot(xs + (int64_t)j * D, xn); };
+  float best;
+  uint32_t bi;
+  if (p) {
+    float u[D], a;
+    tr.project(xn, u, a);
+    const float slack = (float)D * rounding_slack(a);
+    auto bound = [&](uint32_t j) {
+      float s = 0.f;
+#pragma unroll
+      for (int q = 0; q < D; ++q) {
+        const float v = u[q] - p[(int64_t)j * D + q];
+        s = fmaf(v, v, s);
+      }
+      return fmaf(-0.5f * (1.f - kEta), s, lim[j] + slack);
+    };
+    bi = gumbel_argmax(km, (uint32_t)n, lane, part, W, bound, logit, &best);
+  } else {
+    bi = gumbel_argmax(km, (uint32_t)n, lane, part, W, [&](uint32_t j) { return lw[j] - tr.nlz; }, logit, &best);
+  }
+  if constexpr (W > 1) {
+    if (lane == 0) {
+      wbest[w] = best;
+      wi[w] = bi;
+    }
+    __syncthreads();
+    best = wbest[0];
+    bi = wi[0];
+    for (int k = 1; k < W; ++k)
+      if (wi[k] != kNoIndex && (bi == kNoIndex || wbest[k] > best || (wbest[k] == best && wi[k] < bi))) {
+        best = wbest[k];
+        bi = wi[k];
+      }
+    if (w != 0) return;
+  }
   if (lane == 0 && idx) idx[m] = (int32_t)bi;
-  if (lane < D) xout[m * D + lane] = xs[bi * D + lane];
+  if (lane < D) xout[m * D + lane] = xs[(int64_t)bi * D + lane];
 }
 
 template <class Tr, int D>
-int launch_ffbsi(const float* params, const float* xs, const float* lw, int64_t n, const float* xnext, int64_t m,
-                 const uint32_t* key, int32_t* idx, float* xout, hipStream_t stream) {
-  const int per = 256 / kWave;
-  hipLaunchKernelGGL((ffbsi_step_kernel<Tr, D>), dim3((unsigned)((m + per - 1) / per)), dim3(256), 0, stream, params,
-                     xs, lw, n, xnext, m, key, idx, xout);
+int launch_ffbsi(const float* params, const float* xs, const float* lw, const float* p, const float* lim, int64_t n,
+                 const float* xnext, int64_t m, const uint32_t* key, int32_t* idx, float* xout, hipStream_t stream) {
+  // with at most two waves per SIMD a wave's chain of threefry blocks is the bound: four share it
+  const bool split = m <= 2048 && n >= 512;
+  if (split)
+    hipLaunchKernelGGL((ffbsi_step_kernel<Tr, D, 4>), dim3((unsigned)m), dim3(256), 0, stream, params, xs, lw, p, lim, n,
+                       xnext, m, key, idx, xout);
+  else
+    hipLaunchKernelGGL((ffbsi_step_kernel<Tr, D, 1>), dim3((unsigned)((m + 3) / 4)), dim3(256), 0, stream, params, xs,
+                       lw, p, lim, n, xnext, m, key, idx, xout);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }
@@ -207,7 +279,8 @@ __global__ __launch_bounds__(256) void ffbsi_step_rt_kernel(int d, const float* 
     }
     return 0.5f * s + nlz;
   };
-  const int64_t bi = gumbel_argmax_wave(km, (uint32_t)n, 0, n, lane, [&](int64_t j) { return lw[j] - pot(j); });
+  const int64_t bi = gumbel_argmax(km, (uint32_t)n, lane, 0u, 1u, [&](int64_t j) { return lw[j] - nlz; },
+                                   [&](int64_t j) { return lw[j] - pot(j); });
   if (lane == 0 && idx) idx[m] = (int32_t)bi;
   if (lane < d) xout[m * d + lane] = xs[bi * d + lane];
 }
@@ -253,8 +326,8 @@ __global__ __launch_bounds__(256) void rej_init_kernel(const float* __restrict__
   Tr tr;
   tr.load(params, (int)DD);
   const Key kt{key[0], key[1]};
-  const int64_t bi = gumbel_argmax_wave(split_at(kt, 3, 0), (uint32_t)(M * n), (uint64_t)m * (uint64_t)n, n, lane,
-                                        [&](int64_t j) { return lw[j]; });
+  const int64_t bi = gumbel_row(split_at(kt, 3, 0), (uint32_t)(M * n), (uint32_t)(m * n), (uint32_t)n, lane,
+                                [&](int64_t j) { return lw[j]; });
   if (lane == 0) {
     idx[m] = (int32_t)bi;
     b.dens[m] = expf(-tr.pot(xs + bi * DD, xnext + m * DD));
@@ -361,7 +434,8 @@ __global__ __launch_bounds__(256) void rej_round_kernel(const float* __restrict_
   tr.load(params, (int)DD);
   const Key k{b.keys[2 * m], b.keys[2 * m + 1]};
   const Key kr = split_at(k, 3, 0), kc = split_at(k, 3, 1), ku = split_at(k, 3, 2);
-  const int64_t bi = gumbel_argmax_wave(kc, (uint32_t)n, 0, n, lane, [&](int64_t j) { return lw[j]; });
+  const int64_t bi = gumbel_argmax(kc, (uint32_t)n, lane, 0u, 1u, [&](int64_t j) { return lw[j]; },
+                                   [&](int64_t j) { return lw[j]; });
   if (lane == 0) {
     const float dd = expf(-tr.pot(xs + bi * DD, xnext + m * DD));
     const float u = uniform_from_bits(bits_at(ku, 1, 0), 0.f, 1.f);
@@ -395,10 +469,12 @@ __global__ __launch_bounds__(256) void rej_final_kernel(const float* __restrict_
       float xn[D];
 #pragma unroll
       for (int q = 0; q < D; ++q) xn[q] = xnext[m * D + q];
-      bi = gumbel_argmax_wave(k, (uint32_t)n, 0, n, lane, [&](int64_t j) { return lw[j] - tr.pot(xs + j * D, xn); });
+      bi = gumbel_argmax(k, (uint32_t)n, lane, 0u, 1u, [&](int64_t j) { return lw[j] - tr.nlz; },
+                         [&](int64_t j) { return lw[j] - tr.pot(xs + j * D, xn); });
     } else {
       const float* xn = xnext + m * DD;
-      bi = gumbel_argmax_wave(k, (uint32_t)n, 0, n, lane, [&](int64_t j) { return lw[j] - tr.pot(xs + j * DD, xn); });
+      bi = gumbel_argmax(k, (uint32_t)n, lane, 0u, 1u, [&](int64_t j) { return lw[j] - tr.nlz; },
+                         [&](int64_t j) { return lw[j] - tr.pot(xs + j * DD, xn); });
     }
     if (lane == 0) idx[m] = (int32_t)bi;
   } else {
@@ -446,6 +522,59 @@ int64_t rej_layout(int64_t M, RejBuffers* b, char* base) {
                          reinterpret_cast<int32_t*>(entered), reinterpret_cast<float*>(dens),
                          reinterpret_cast<RejState*>(st)};
   return o;
+}
+
+// (model, d) of the compiled transitions; the linear-Gaussian model runs at any d <= kRtMaxDim without bounds
+#define MOCAT_FFBSI_SHAPES(CASE)                                             \
+  if (model == 1 && d == 1) CASE(SvTrans, 1);                                \
+  if (model == 0 && d == 1) CASE(LgTrans<1>, 1);                             \
+  if (model == 0 && d == 2) CASE(LgTrans<2>, 2);                             \
+  if (model == 0 && d == 3) CASE(LgTrans<3>, 3);                             \
+  if (model == 0 && d == 4) CASE(LgTrans<4>, 4);                             \
+  if (model == 0 && d == 5) CASE(LgTrans<5>, 5);                             \
+  if (model == 0 && d == 8) CASE(LgTrans<8>, 8);
+
+int ffbsi_step_dispatch(int model, int d, const float* params, const float* particles, const float* log_weight,
+                        const float* p, const float* lim, int64_t n, const float* x_next, int64_t m,
+                        const uint32_t* key, int32_t* idx, float* x_out, hipStream_t stream) {
+#define MOCAT_FFBSI_CASE(TR, DD) \
+  return launch_ffbsi<TR, DD>(params, particles, log_weight, p, lim, n, x_next, m, key, idx, x_out, stream)
+  MOCAT_FFBSI_SHAPES(MOCAT_FFBSI_CASE)
+#undef MOCAT_FFBSI_CASE
+  if (model != 0 || d < 1 || d > kRtMaxDim) return MOCAT_ERR_ARG;
+  const int per = 256 / kWave;
+  hipLaunchKernelGGL(ffbsi_step_rt_kernel, dim3((unsigned)((m + per - 1) / per)), dim3(256), 0, stream, d, params,
+                     particles, log_weight, n, x_next, m, key, idx, x_out);
+  MOCAT_LAUNCH_CHECK();
+  return MOCAT_OK;
+}
+
+template <class Tr, int D>
+int launch_ffbsi_prep(const float* params, const float* xs, const float* lw, int64_t count, float* p, float* lim,
+                      hipStream_t stream) {
+  const int64_t blocks = (count + 255) / 256;
+  hipLaunchKernelGGL((ffbsi_prep_kernel<Tr, D>), dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+                     params, xs, lw, count, p, lim);
+  MOCAT_LAUNCH_CHECK();
+  return MOCAT_OK;
+}
+
+int ffbsi_prep_dispatch(int model, int d, const float* params, const float* xs, const float* lw, int64_t count,
+                        float* p, float* lim, hipStream_t stream) {
+#define MOCAT_FFBSI_CASE(TR, DD) return launch_ffbsi_prep<TR, DD>(params, xs, lw, count, p, lim, stream)
+  MOCAT_FFBSI_SHAPES(MOCAT_FFBSI_CASE)
+#undef MOCAT_FFBSI_CASE
+  return MOCAT_ERR_ARG;
+}
+
+// Time points whose bounds are prepared together (up to 64 MB of workspace); 0: no bounds, for a dimension
+// without a compiled transition and for so few trajectories that preparing costs what it saves.
+int64_t ffbsi_step_bytes(int d, int64_t n) { return n * (d + 1) * (int64_t)sizeof(float); }
+int64_t ffbsi_block(int model, int d, int64_t T, int64_t n, int64_t m) {
+  const bool compiled = model == 1 ? d == 1 : (d >= 1 && d <= 5) || d == 8;
+  if (!compiled || m < 16 || T < 2) return 0;
+  const int64_t fit = (64ll << 20) / ffbsi_step_bytes(d, n);
+  return fit < 1 ? 1 : fit < T - 1 ? fit : T - 1;
 }
 
 }  // namespace
@@ -498,27 +627,40 @@ int mocat_ffbsi_step(int model, int d, const float* params, const float* particl
   if (!params || !particles || !log_weight || !x_next || !key || !x_out || n <= 0 || n >= 0xFFFFFFFFll || m <= 0 ||
       m >= 0xFFFFFFFFll)
     return MOCAT_ERR_ARG;
-  if (model == 1) {
-    if (d != 1) return MOCAT_ERR_ARG;
-    return launch_ffbsi<SvTrans, 1>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-  }
-  if (model != 0) return MOCAT_ERR_ARG;
-  switch (d) {
-    case 1: return launch_ffbsi<LgTrans<1>, 1>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    case 2: return launch_ffbsi<LgTrans<2>, 2>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    case 3: return launch_ffbsi<LgTrans<3>, 3>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    case 4: return launch_ffbsi<LgTrans<4>, 4>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    case 5: return launch_ffbsi<LgTrans<5>, 5>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    case 8: return launch_ffbsi<LgTrans<8>, 8>(params, particles, log_weight, n, x_next, m, key, idx, x_out, stream);
-    default: {
-      if (d < 1 || d > kRtMaxDim) return MOCAT_ERR_ARG;
-      const int per = 256 / kWave;
-      hipLaunchKernelGGL(ffbsi_step_rt_kernel, dim3((unsigned)((m + per - 1) / per)), dim3(256), 0, stream, d, params,
-                         particles, log_weight, n, x_next, m, key, idx, x_out);
-      MOCAT_LAUNCH_CHECK();
-      return MOCAT_OK;
+  return ffbsi_step_dispatch(model, d, params, particles, log_weight, nullptr, nullptr, n, x_next, m, key, idx, x_out,
+                             stream);
+}
+
+int mocat_ffbsi_workspace_bytes(int model, int d, int64_t T, int64_t n, int64_t m, int64_t* bytes) {
+  if (d < 1 || T < 1 || n <= 0 || m <= 0 || !bytes) return MOCAT_ERR_ARG;
+  *bytes = ffbsi_block(model, d, T, n, m) * ffbsi_step_bytes(d, n);
+  return MOCAT_OK;
+}
+
+int mocat_ffbsi_run(int model, int d, const float* params, const float* particles, const float* log_weight, int64_t T,
+                    int64_t n, int64_t m, const uint32_t* keys, void* workspace, int64_t workspace_bytes, int32_t* idx,
+                    float* x_out, hipStream_t stream) {
+  if (!params || !particles || !log_weight || !keys || !idx || !x_out || T < 1 || n <= 0 || n >= 0xFFFFFFFFll || m <= 0 ||
+      m >= 0xFFFFFFFFll || d < 1)
+    return MOCAT_ERR_ARG;
+  const int64_t B = ffbsi_block(model, d, T, n, m);
+  if (B > 0 && (!workspace || workspace_bytes < B * ffbsi_step_bytes(d, n))) return MOCAT_ERR_SIZE;
+  float* p = static_cast<float*>(workspace);
+  float* lim = p + B * n * d;
+  int64_t lo = T - 1;  // the prepared block starts here
+  for (int64_t t = T - 2; t >= 0; --t) {
+    if (B > 0 && t < lo) {
+      lo = t - B + 1 > 0 ? t - B + 1 : 0;
+      const int rc = ffbsi_prep_dispatch(model, d, params, particles + lo * n * d, log_weight + lo * n,
+                                         (t - lo + 1) * n, p, lim, stream);
+      if (rc != MOCAT_OK) return rc;
     }
+    const int rc = ffbsi_step_dispatch(model, d, params, particles + t * n * d, log_weight + t * n,
+                                       B > 0 ? p + (t - lo) * n * d : nullptr, B > 0 ? lim + (t - lo) * n : nullptr, n,
+                                       x_out + (t + 1) * m * d, m, keys + 2 * t, idx + t * m, x_out + t * m * d, stream);
+    if (rc != MOCAT_OK) return rc;
   }
+  return MOCAT_OK;
 }
 
 }  // extern "C"

@@ -33,11 +33,13 @@ struct GumbelRow {
   uint32_t bi = kNoIndex;
   bool nan = false;
 
-  MOCAT_DEV void offer(bool act, uint32_t j, uint32_t bits, float logit) {
-    const bool c = act && !(PRUNE && gumbel_upper(bits) + logit < top);
+  // bound: at least logit(j).
+  template <class Logit>
+  MOCAT_DEV void offer(bool act, uint32_t j, uint32_t bits, float bound, Logit logit) {
+    const bool c = act && !(PRUNE && gumbel_upper(bits) + bound < top);
     if (PRUNE && __ballot(c) == 0ull) return;
     if (c) {
-      const float v = gumbel_exact(bits) + logit;
+      const float v = gumbel_exact(bits) + logit(j);
       nan = nan || isnan(v);
       if (bi == kNoIndex || v > best || (v == best && j < bi)) {
         best = v;
@@ -48,19 +50,17 @@ struct GumbelRow {
   }
 
   // the maximum over the wave, the lower index on ties (first maximum); kNoIndex without candidates
-  MOCAT_DEV uint32_t first_max() const {
-    float b = best;
-    uint32_t i = bi;
+  MOCAT_DEV uint32_t first_max() {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(b, o, kWave);
-      const uint32_t oi = (uint32_t)__shfl_xor((int)i, o, kWave);
-      if (oi != kNoIndex && (i == kNoIndex || ob > b || (ob == b && oi < i))) {
-        b = ob;
-        i = oi;
+      const float ob = __shfl_xor(best, o, kWave);
+      const uint32_t oi = (uint32_t)__shfl_xor((int)bi, o, kWave);
+      if (oi != kNoIndex && (bi == kNoIndex || ob > best || (ob == best && oi < bi))) {
+        best = ob;
+        bi = oi;
       }
     }
-    return i;
+    return bi;
   }
   MOCAT_DEV bool met_nan() const { return __any(nan) != 0; }
 };
@@ -72,7 +72,7 @@ MOCAT_DEV uint32_t gumbel_row(Key k, uint32_t S, uint32_t off, uint32_t n, int l
     for (uint64_t j0 = 0; j0 < n; j0 += kWave) {
       const bool act = j0 + (uint64_t)lane < n;
       const uint32_t j = (uint32_t)j0 + (uint32_t)lane, jc = act ? j : n - 1u;
-      row.offer(act, j, bits_at(k, S, off + jc), logit(jc));
+      row.offer(act, j, bits_at(k, S, off + jc), logit(jc), logit);
     }
   };
   GumbelRow<true> row;
@@ -81,6 +81,39 @@ MOCAT_DEV uint32_t gumbel_row(Key k, uint32_t S, uint32_t off, uint32_t n, int l
   GumbelRow<false> all;
   draw(all);
   return all.first_max();
+}
+
+// argmax_j gumbel(k, (n,))_j + logit(j) with logit(j) <= bound(j): elements j and j + ceil(n / 2) are the two
+// words of a threefry block. Wave `part` of `parts` takes every parts-th 64 blocks; `best` and the index
+// returned are its own part's.
+template <class Bound, class Logit>
+MOCAT_DEV uint32_t gumbel_argmax(Key k, uint32_t n, int lane, uint32_t part, uint32_t parts, Bound bound, Logit logit,
+                                 float* best = nullptr) {
+  const uint32_t h = (n + 1u) >> 1;
+  auto draw = [&](auto& row) {
+    for (uint64_t j0 = (uint64_t)part * kWave; j0 < h; j0 += (uint64_t)parts * kWave) {
+      const bool act = j0 + (uint64_t)lane < h;
+      const uint32_t j = act ? (uint32_t)j0 + (uint32_t)lane : 0u;
+      const bool act1 = act && j + h < n;
+      const uint32_t j1 = act1 ? j + h : 0u;
+      const float b0 = bound(j), b1 = bound(j1);
+      uint32_t w0, w1;
+      bits_pair(k, n, j, w0, w1);
+      row.offer(act, j, w0, b0, logit);
+      row.offer(act1, j1, w1, b1, logit);
+    }
+    row.first_max();
+  };
+  GumbelRow<true> row;
+  draw(row);
+  if (!row.met_nan()) {
+    if (best) *best = row.best;
+    return row.bi;
+  }
+  GumbelRow<false> all;
+  draw(all);
+  if (best) *best = all.best;
+  return all.bi;
 }
 
 // Rows m and m + rows / 2 of gumbel(k, (rows, n)) for an even number of rows: element m n + j and the same
@@ -96,8 +129,8 @@ MOCAT_DEV void gumbel_row_pair(Key k, uint32_t S, uint32_t off, uint32_t n, int 
       uint32_t w0 = off + jc, w1 = off + jc + h;
       threefry2x32(k.a, k.b, w0, w1);
       const float l = logit(jc);
-      a.offer(act, j, w0, l);
-      b.offer(act, j, w1, l);
+      a.offer(act, j, w0, l, logit);
+      b.offer(act, j, w1, l, logit);
     }
   };
   GumbelRow<true> a, b;

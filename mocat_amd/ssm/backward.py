@@ -1,7 +1,7 @@
 """Backward simulation for state-space models (mocat/src/ssm/backward.py): forward filtering then
 full backward resampling of whole trajectories on the GPU.
 
-Full backward resampling is one launch of the FFBSi kernel per step (one wave per trajectory,
+Full backward resampling is one launch of the FFBSi kernel per step (a wave or a workgroup per trajectory,
 Gumbel-max over the N filter particles with the same key tree as mocat: t_keys = split(key, T),
 then split(t_keys[t], M) per trajectory), N x M transition potentials per step. Rejection sampling
 (maximum_rejections > 0) runs mocat's accept/reject rounds on the GPU, two launches per round.
@@ -20,6 +20,9 @@ from .filtering import run_particle_filter_for_marginals
 
 _P = _lib.c_ptr
 _lib.register("mocat_ffbsi_step", [_lib.c_i32, _lib.c_i32, _P, _P, _P, _lib.c_i64, _P, _lib.c_i64, _P, _P, _P, _P])
+_lib.register("mocat_ffbsi_workspace_bytes", [_lib.c_i32, _lib.c_i32, _lib.c_i64, _lib.c_i64, _lib.c_i64, _P])
+_lib.register("mocat_ffbsi_run", [_lib.c_i32, _lib.c_i32, _P, _P, _P, _lib.c_i64, _lib.c_i64, _lib.c_i64, _P, _P,
+                                  _lib.c_i64, _P, _P, _P])
 _lib.register("mocat_resample_categorical", [_P, _lib.c_i64, _lib.c_i64, _P, _P, _P])
 _lib.register("mocat_gather_rows", [_P, _P, _lib.c_i64, _lib.c_i64, _P, _P])
 _lib.register("mocat_ffbsi_rejection_workspace_bytes", [_lib.c_i64, _P])
@@ -73,9 +76,11 @@ def backward_simulation(ssm_scenario, marginal_particles: cdict, random_key, n_s
                       _lib.ptr(anc[ind]), _lib.ptr(out[ind]), _lib.ptr(evals[ind + 1]), st)
         num_evals = evals.cpu().to(torch.float64)  # [0, steps t = 0 .. T-2] (backward.py:205)
     else:
-        for ind in range(T - 2, -1, -1):
-            _lib.call("mocat_ffbsi_step", model, d, _lib.ptr(params), _lib.ptr(vals[ind]), _lib.ptr(lw[ind]), n,
-                      _lib.ptr(out[ind + 1]), m, _lib.ptr(keys[ind]), _lib.ptr(anc[ind]), _lib.ptr(out[ind]), st)
+        nb = _lib.ctypes.c_int64(0)
+        _lib.call("mocat_ffbsi_workspace_bytes", model, d, T, n, m, _lib.ctypes.byref(nb))
+        ws = torch.empty(int(nb.value), dtype=torch.uint8, device="cuda")
+        _lib.call("mocat_ffbsi_run", model, d, _lib.ptr(params), _lib.ptr(vals), _lib.ptr(lw), T, n, m, _lib.ptr(keys),
+                  _lib.ptr(ws), int(ws.numel()), _lib.ptr(anc), _lib.ptr(out), st)
         num_evals = torch.cat([torch.zeros(1, dtype=torch.float64),
                                torch.full((T - 1,), float(n) * m, dtype=torch.float64)])
     res = cdict(**{k: v for k, v in marginal_particles.__dict__.items() if k != "log_weight"})
