@@ -36,6 +36,8 @@ _lib.register("mocat_pf_hook", [_lib.c_i32, _lib.c_i32, _lib.c_i32, _lib.c_i32, 
 _lib.register("mocat_resample", [_P, _lib.c_i64, _lib.c_i32, _lib.c_i32, _P, _P, _P, _P])
 _lib.register("mocat_pf_compiled_shape", [_lib.c_i32, _lib.c_i32, _lib.c_i32, _P])
 _lib.register("mocat_gather_rows", [_P, _P, _lib.c_i64, _lib.c_i64, _P, _P])
+_lib.register("mocat_kalman_filter", [_P, _lib.c_i32, _lib.c_i64, _lib.c_i32, _lib.c_i32, _P, _P, _P, _P, _P, _P])
+_lib.register("mocat_kalman_smoother", [_P, _lib.c_i32, _lib.c_i64, _lib.c_i32, _P, _P, _P, _P, _P, _P, _P, _P])
 _lib.register("mocat_enkf_hook", [_lib.c_i32, _lib.c_i32, _lib.c_i32, _P, _P, _P, _lib.c_i64, _P, _P, _P, _P])
 _lib.register("mocat_resample_noalloc", [_P, _lib.c_i64, _lib.c_i32, _lib.c_i32, _P, _P, _P])
 _lib.register("mocat_resample_categorical", [_P, _lib.c_i64, _lib.c_i64, _P, _P, _P])
@@ -848,11 +850,55 @@ def _kalman_mats(lgssm):
             f(lgssm.likelihood_covariance), f(lgssm.initial_mean), f(lgssm.initial_covariance), dev)
 
 
+KALMAN_MAX_DIM = 8  # the Kalman kernels' largest state or observation dimension
+
+
+def _padded(a, m_pad, diag=0.0):
+    """a in the upper left of an m_pad x m_pad FP64 matrix, diag on the diagonal below its rows."""
+    a = np.asarray(a, np.float64)
+    out = np.diag(np.where(np.arange(m_pad) < a.shape[0], 0.0, diag))
+    out[:a.shape[0], :a.shape[1]] = a
+    return out
+
+
+def _on_device(parts):
+    return torch.from_numpy(np.concatenate([p.reshape(-1) for p in parts])).to(mr.default_device())
+
+
+def _kalman_filter_kernel(lgssm, yn):
+    """The filter in one launch, or None when the dimensions have no kernel or an innovation covariance has no
+    Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
+    observations H = 0, R = 1, y = 0."""
+    T, dy = yn.shape
+    d = int(np.shape(lgssm.transition_matrix)[0])
+    k = max(d, dy)
+    if not T or k > KALMAN_MAX_DIM or np.shape(lgssm.likelihood_matrix) != (dy, d):
+        return None
+    model = _on_device([_padded(lgssm.transition_matrix, k), _padded(lgssm.transition_covariance, k, 1.0),
+                        _padded(lgssm.likelihood_matrix, k), _padded(lgssm.likelihood_covariance, k, 1.0),
+                        _padded(lgssm.initial_covariance, k, 1.0),
+                        np.pad(np.asarray(lgssm.initial_mean, np.float64).reshape(-1), (0, k - d)),
+                        np.pad(yn, ((0, 0), (0, k - dy)))])
+    out = torch.empty(T * (d + d * d + k + 1) + 2, dtype=torch.float64, device=model.device)
+    means, covs, ll, scratch, info = torch.split(out, [T * d, T * d * d, 1, T * (k + 1), 1])
+    _lib.call("mocat_kalman_filter", _lib.ptr(model), k, T, d, dy, _lib.ptr(means), _lib.ptr(covs), _lib.ptr(ll),
+              _lib.ptr(scratch), _lib.ptr(info), _lib.stream_handle())
+    if int(info.view(torch.int32)[0]):
+        return None
+    return KalmanOutput(means.reshape(T, d), covs.reshape(T, d, d), ll[0])
+
+
 def run_kalman_filter_for_marginals(lgssm, y, t=None):
     """Kalman filter means/covariances (mocat/src/ssm/linear_gaussian/kalman.py:16-57), returned as
     mocat's (means (T, d), covs (T, d, d)) tuple; `.log_likelihood` holds log p(y_0:T) (not in mocat).
     The t = 0 prior covariance is the initial covariance (mocat uses its square root, kalman.py:20,
-    the same for the identity). FP64 torch on the GPU."""
+    the same for the identity). FP64 on the GPU: one kernel up to dimension KALMAN_MAX_DIM, else (and where
+    an innovation covariance is not positive definite, which raises) torch operations step by step."""
+    yn = np.asarray(y.detach().cpu() if isinstance(y, torch.Tensor) else y, np.float64)
+    yn = yn.reshape(len(yn), -1)
+    out = _kalman_filter_kernel(lgssm, yn)
+    if out is not None:
+        return out
     A, Q, H, R, m, P, dev = _kalman_mats(lgssm)
     yy = torch.as_tensor(np.asarray(y.detach().cpu() if isinstance(y, torch.Tensor) else y), dtype=torch.float64,
                          device=dev).reshape(len(y), -1)
@@ -875,17 +921,38 @@ def run_kalman_filter_for_marginals(lgssm, y, t=None):
     return KalmanOutput(torch.stack(means), torch.stack(covs), ll)
 
 
+def _kalman_smoother_kernel(lgssm, f_mus, f_covs):
+    """The smoother in three launches, or None when the dimension has no kernel or a predicted covariance has
+    no Cholesky factor."""
+    T, d = f_mus.shape
+    if not T or d > KALMAN_MAX_DIM or f_covs.shape != (T, d, d) or np.shape(lgssm.transition_matrix) != (d, d):
+        return None
+    model = _on_device([_padded(lgssm.transition_matrix, d), _padded(lgssm.transition_covariance, d)])
+    out = torch.empty(T * (d + d * d) + (T - 1) * 3 * d * d + 1, dtype=torch.float64, device=model.device)
+    out[-1] = 0.0
+    means, covs, lags, scratch, info = torch.split(out, [T * d, T * d * d, (T - 1) * d * d, 2 * (T - 1) * d * d, 1])
+    _lib.call("mocat_kalman_smoother", _lib.ptr(model), d, T, d, _lib.ptr(f_mus), _lib.ptr(f_covs), _lib.ptr(means),
+              _lib.ptr(covs), _lib.ptr(lags), _lib.ptr(scratch), _lib.ptr(info), _lib.stream_handle())
+    if int(info.view(torch.int32)[0]):
+        return None
+    return means.reshape(T, d), covs.reshape(T, d, d), lags.reshape(T - 1, d, d)
+
+
 def run_kalman_smoother_for_marginals_and_lag_ones(lgssm, y, t=None, filter_output=None):
     """Rauch-Tung-Striebel backward pass (mocat/src/ssm/linear_gaussian/kalman.py:60-98) in FP64: back
     gain J = P_t A^T (A P_t A^T + Q)^-1, m_t = f_t + J (m_t+1 - A f_t), P_t = F_t + J (P_t+1 - A F_t A^T - Q) J^T,
     and mocat's lag-one term written as it is there, f_t . m_t+1 + J (P_t+1 + (m_t+1 - f_t+1) . m_t+1)
     (dot products of the mean vectors, as jnp's @ on 1-D arrays evaluates them). Returns
     (means (T, d), covs (T, d, d), lag_ones (T-1, d, d))."""
-    A, Q, _, _, _, _, dev = _kalman_mats(lgssm)
+    dev = mr.default_device()
     f_mus, f_covs = filter_output if filter_output is not None else run_kalman_filter_for_marginals(lgssm, y, t)
     f_mus = torch.as_tensor(f_mus, dtype=torch.float64, device=dev)
     f_covs = torch.as_tensor(f_covs, dtype=torch.float64, device=dev)
     T = f_mus.shape[0]
+    out = _kalman_smoother_kernel(lgssm, f_mus.contiguous(), f_covs.contiguous()) if f_mus.dim() == 2 else None
+    if out is not None:
+        return out
+    A, Q, _, _, _, _, dev = _kalman_mats(lgssm)
     mu, cov = f_mus[-1], f_covs[-1]
     mus, covs, lags = [mu], [cov], []
     for i in range(T - 2, -1, -1):
