@@ -388,6 +388,12 @@ int mocat_svgd_gmm_run(float* x, int64_t n, int64_t d, int K, const float* means
 int mocat_ksd_rows(const float* x, const float* grad_potential, const float* weights, int64_t n, int64_t d,
                    int kernel, float bandwidth, float c, float beta, int js_count, double* part,
                    hipStream_t stream);
+/* The discrepancy itself: *out = sqrt(sum_ij w_i w_j k_0(x_i, x_j)) / sum(w) (FP64; weights may be NULL: ones),
+ * over the pairs i <= j. workspace: mocat_ksd_workspace_bytes(n). */
+int mocat_ksd_workspace_bytes(int64_t n, int64_t* bytes);
+int mocat_ksd(const float* x, const float* grad_potential, const double* weights, int64_t n, int64_t d, int kernel,
+              float bandwidth, float c, float beta, void* workspace, int64_t workspace_bytes, double* out,
+              hipStream_t stream);
 /* ---- KSD over random minibatches (replaces mocat/src/metrics.py:101-104,126-128, ksd with
  * ensemble_batchsize = batch): inds[i][b] (int32, in [0, n)) are particle i's batch;
  * row_k[i] = sum_b weights[inds[i][b]] * k_0(x_i, x_inds[i][b]) and row_w[i] = sum_b

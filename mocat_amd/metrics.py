@@ -10,8 +10,8 @@ log_ess_log_weight / ess_log_weight follow mocat/src/metrics.py:69-78:
 2 * logsumexp(w) - logsumexp(2 w), reduced in FP64 by the reduction kernel of libmocat_amd.
 
 ksd follows mocat/src/metrics.py:88-130 for the Gaussian and IMQ kernels over the full ensemble: the
-weighted k_0 row sums come from the tiled pair kernel of libmocat_amd (FP32 coordinate sums, FP64
-row sums), the final weighting and square root are FP64.
+weighted k_0 sum comes from the tiled pair kernel of libmocat_amd (FP32 coordinate sums, the weights, the
+sum and the square root in FP64).
 """
 from __future__ import annotations
 
@@ -21,6 +21,9 @@ from . import _lib as _l
 
 _l.register("mocat_ksd_rows", [_l.c_ptr, _l.c_ptr, _l.c_ptr, _l.c_i64, _l.c_i64, _l.c_i32, _l.c_f32, _l.c_f32,
                                _l.c_f32, _l.c_i32, _l.c_ptr, _l.c_ptr])
+_l.register("mocat_ksd_workspace_bytes", [_l.c_i64, _l.c_ptr])
+_l.register("mocat_ksd", [_l.c_ptr, _l.c_ptr, _l.c_ptr, _l.c_i64, _l.c_i64, _l.c_i32, _l.c_f32, _l.c_f32, _l.c_f32, _l.c_ptr,
+                          _l.c_i64, _l.c_ptr, _l.c_ptr])
 _l.register("mocat_ksd_batch_rows", [_l.c_ptr, _l.c_ptr, _l.c_ptr, _l.c_i64, _l.c_i64, _l.c_i64, _l.c_ptr, _l.c_i32,
                                      _l.c_f32, _l.c_f32, _l.c_f32, _l.c_ptr, _l.c_ptr, _l.c_ptr])
 
@@ -113,17 +116,16 @@ def ksd(sample, kernel, grad_potential: torch.Tensor = None, log_weight: torch.T
     x = x.reshape(x.shape[0], -1).contiguous()
     g = torch.as_tensor(grad_potential, dtype=torch.float32, device="cuda").reshape(x.shape).contiguous()
     n, d = x.shape
-    if log_weight is not None:
-        w64 = torch.exp(torch.as_tensor(log_weight, device="cuda").to(torch.float64).reshape(n))
-        w = w64.to(torch.float32).contiguous()
-    else:
-        w64, w = torch.ones(n, dtype=torch.float64, device="cuda"), None
+    w64 = None if log_weight is None else \
+        torch.exp(torch.as_tensor(log_weight, device="cuda").to(torch.float64).reshape(n)).contiguous()
     if ensemble_batchsize is not None:
         # metrics.py:101-104: batch_i = random.choice(random_key, n, (n, ensemble_batchsize))[i]
         if random_key is None:
             raise TypeError("ensemble_batchsize needs random_key")
         from . import random as mrandom
         batch = int(ensemble_batchsize)
+        w = None if w64 is None else w64.to(torch.float32)
+        w64 = torch.ones(n, dtype=torch.float64, device="cuda") if w64 is None else w64
         inds = mrandom.choice(random_key, n, (n, batch)).contiguous()
         row_k = torch.empty(n, dtype=torch.float64, device="cuda")
         row_w = torch.empty(n, dtype=torch.float64, device="cuda")
@@ -131,11 +133,10 @@ def ksd(sample, kernel, grad_potential: torch.Tensor = None, log_weight: torch.T
                   _KSD_KERNELS[name], float(params["bandwidth"]), float(params.get("c", 1.0)),
                   float(params.get("beta", -0.5)), _lib.ptr(row_k), _lib.ptr(row_w), _lib.stream_handle())
         return float(torch.sqrt((w64 * row_k / (w64.sum() * row_w)).sum()).item())
-    tiles = -(-n // 64)
-    js = max(1, min(tiles, 64))
-    part = torch.empty((js, n), dtype=torch.float64, device="cuda")
-    _lib.call("mocat_ksd_rows", _lib.ptr(x), _lib.ptr(g), _lib.ptr(w), n, d, _KSD_KERNELS[name],
-              float(params["bandwidth"]), float(params.get("c", 1.0)), float(params.get("beta", -0.5)), js,
-              _lib.ptr(part), _lib.stream_handle())
-    s = w64.sum()
-    return float(torch.sqrt((part.sum(0) * w64).sum() / (s * s)).item())
+    nb = _lib.ctypes.c_int64(0)
+    _lib.call("mocat_ksd_workspace_bytes", n, _lib.ctypes.byref(nb))
+    ws = torch.empty(int(nb.value) // 8 + 1, dtype=torch.float64, device="cuda")
+    _lib.call("mocat_ksd", _lib.ptr(x), _lib.ptr(g), _lib.ptr(w64), n, d, _KSD_KERNELS[name], float(params["bandwidth"]),
+              float(params.get("c", 1.0)), float(params.get("beta", -0.5)), _lib.ptr(ws), int(nb.value),
+              _lib.ctypes.c_void_p(ws[-1:].data_ptr()), _lib.stream_handle())
+    return float(ws[-1].item())
