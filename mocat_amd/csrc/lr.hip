@@ -303,24 +303,37 @@ MOCAT_DEV void split_bf16(float v, __bf16& hi, __bf16& lo) {
 
 // ------------------------------------------------------------------------------------------
 // BF16 split-precision MFMA engine (every product hi*hi + hi*lo + lo*hi, FP32 accumulation).
-// Z = X Theta^T is accumulated with rows of X on the M side and the 32 chains on N, so each lane's
+// Z = X Theta^T is accumulated with rows of X on the M side and 32 chains on N, so each lane's
 // accumulator column is one chain; R = sigmoid(Z) - y is formed in registers and reused directly as
 // the A operand (chains x rows) of G = R X: the K slots of that operand are the rows the lane already
 // holds, and X's second packed layout lists its rows in the same order. With NW waves, wave w takes
 // the 32-row blocks rb = w + NW j; two waves per SIMD (NW = 8) let one wave's row functions on the
 // vector ALU overlap the other's MFMAs.
-template <int DP, int NT>
+//
+// A workgroup takes NCT tiles of 32 chains. What bounds one tile is the first-level cache: every wave streams its
+// blocks' operands through it at 64 B per clock, 32 KB per 32 rows at d > 64 (2050 clocks for four waves, their
+// MFMAs 1540) and 16 KB at d <= 64 (2050 clocks for eight waves, the MFMAs 1540); leaving out the transcendentals or
+// taking the operands from a hot line changes little there, and neither do two blocks at once per wave (slower) or
+// waves out of phase. Two tiles use each operand twice and are bound by the matrix cores: 309 TFLOP/s algorithmic at
+// d = 100 is 1190 TFLOP/s issued, where a large bf16 product reaches 1344. (One MFMA for the last columns' three
+// products, at d = 50 and 100 10 instead of 12 and 19 instead of 24 per block, would give another 6%, but sums them in
+// another order: chains of 200 leapfrog steps then end up to 3e-5 from where they ended before.)
+template <int DP, int NT, int NCT>
 struct Bf16Engine {
   using L = PackLayout<DP>;
   static constexpr int KB = L::KB, NB = L::NB, NW = NT / kWave;
   static_assert(NW % 4 == 0, "whole SIMDs");
   static_assert(L::kAScale == -kLog2E, "the rows expect the scaled A layout");
-  static constexpr bool kThetaRegs = DP <= 64;
+  static constexpr bool kThetaRegs = DP <= 64 && NCT == 1;
   static constexpr int GS = DP + 4;  // row stride of the partial gradients (spreads LDS banks)
   struct alignas(16) Smem {
     alignas(16) float gred[NW][CT * GS];
-    alignas(16) bf16x8 thl[2][KB][64];  // theta^T operand, hi and lo parts, per lane
-    float ured[NW][2][CT];
+    alignas(16) bf16x8 thl[NCT][2][KB][64];  // theta^T operands, hi and lo parts, per lane
+    float ured[NW][2][NCT * CT];
+  };
+  struct Acc {
+    floatx16 g[NCT][NB];  // the wave's partial gradients
+    float u[NCT];         // and potential terms
   };
   struct ABuf {
     bf16x8 h[KB], l[KB];
@@ -330,56 +343,28 @@ struct Bf16Engine {
     bf16x8 h[2][NB], l[2][NB];
   };
 
-  static MOCAT_DEV void eval(Smem& s, const float* X, const float* y, const void* packed, int n, int d,
-                             const float* theta, float* lik, float* glik, bool want_pot) {
-    // the potential terms are needed after the last leapfrog step only: two compiled passes, so that
-    // each block's row functions and MFMAs form one straight-line region the scheduler can interleave
-    if (want_pot)
-      pass<true>(s, packed, n, theta, lik, glik);
-    else
-      pass<false>(s, packed, n, theta, lik, glik);
-  }
-
-  template <bool WANT_POT>
-  static MOCAT_DEV void pass(Smem& s, const void* packed, int n, const float* theta, float* lik, float* glik) {
-    const int t = threadIdx.x;
-    for (int e = t; e < KB * 64; e += NT) {
-      const int kb = e / 64, ln = e % 64;
-      const float* src = theta + (ln & 31) * DP + kb * 16 + (ln >> 5) * 8;
-      bf16x8 h8, l8;
+  // Writes columns k .. k + 3 (k a multiple of 4) of chain c of tile ct into theta's operands.
+  static MOCAT_DEV void put_theta(Smem& s, int ct, int c, int k, const float* v) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 h4, l4;
 #pragma unroll
-      for (int s2 = 0; s2 < 8; ++s2) {
-        __bf16 h, l;
-        split_bf16(src[s2], h, l);
-        h8[s2] = h;
-        l8[s2] = l;
-      }
-      s.thl[0][kb][ln] = h8;
-      s.thl[1][kb][ln] = l8;
+    for (int q = 0; q < 4; ++q) {
+      __bf16 h, l;
+      split_bf16(v[q], h, l);
+      h4[q] = h;
+      l4[q] = l;
     }
-    __syncthreads();
-    partials<WANT_POT>(s, packed, n);
-    __syncthreads();
-    for (int e = t; e < CT * DP; e += NT) {
-      const int c = e / DP, k = e - c * DP;
-      float acc = s.gred[0][c * GS + k];
-#pragma unroll
-      for (int q = 1; q < NW; ++q) acc += s.gred[q][c * GS + k];
-      glik[e] = acc;
-    }
-    if (t < CT) {
-      float acc = 0.f;
-      for (int q = 0; q < NW; ++q) acc += s.ured[q][0][t] + s.ured[q][1][t];
-      lik[t] = acc;
-    }
-    __syncthreads();
+    const int ln = c + 32 * ((k / 8) & 1);  // operand (k / 16, lane ln), elements k % 8 ..
+    reinterpret_cast<bf16x4*>(&s.thl[ct][0][k / 16][ln])[(k / 4) & 1] = h4;
+    reinterpret_cast<bf16x4*>(&s.thl[ct][1][k / 16][ln])[(k / 4) & 1] = l4;
   }
 
   // The block loop of one gradient evaluation. Theta's operands are read from s.thl (written by the
-  // caller before a barrier); each wave leaves its partial gradient in s.gred[w] ([chain][GS]) and its
-  // potential partials in s.ured[w]. The caller synchronises before reading them.
+  // caller before a barrier); each wave returns its partial gradients and leaves its potential partials in
+  // s.ured[w]. Two compiled passes (the potential terms are needed after the last leapfrog step only), so that
+  // each block's row functions and MFMAs form one straight-line region the scheduler can interleave.
   template <bool WANT_POT>
-  static MOCAT_DEV void partials(Smem& s, const void* packed, int n) {
+  static MOCAT_DEV void partials(Smem& s, const void* packed, int n, Acc& acc) {
     const int t = threadIdx.x;
     const int lane = t & (kWave - 1), w = t / kWave, g = lane >> 5, col = lane & 31;
     const int nrb = (n + 31) / 32;
@@ -389,16 +374,18 @@ struct Bf16Engine {
     if constexpr (kThetaRegs) {
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-        th[kb] = s.thl[0][kb][lane];
-        tl[kb] = s.thl[1][kb][lane];
+        th[kb] = s.thl[0][0][kb][lane];
+        tl[kb] = s.thl[0][1][kb][lane];
       }
     }
-    floatx16 gacc[NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int ct = 0; ct < NCT; ++ct) {
+      acc.u[ct] = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) gacc[nb][r] = 0.f;
-    float upart = 0.f;
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc.g[ct][nb][r] = 0.f;
+    }
 
     auto blk = [&](int j) { return base + (int64_t)(w + j * NW) * L::BLOCK_BYTES; };
     auto load_a = [&](ABuf& a, int j) {
@@ -423,26 +410,29 @@ struct Bf16Engine {
           b.l[kb2][nb] = B[((1 * 2 + kb2) * NB + nb) * 64 + lane];
         }
     };
-    auto gemm1 = [&](const ABuf& a, floatx16& z) {
+    auto gemm1 = [&](const ABuf& a, floatx16 (&z)[NCT]) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) z[r] = 0.f;
+      for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[ct][r] = 0.f;
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
-        bf16x8 h8, l8;
-        if constexpr (kThetaRegs) {
-          h8 = th[kb];
-          l8 = tl[kb];
-        } else {
-          h8 = s.thl[0][kb][lane];
-          l8 = s.thl[1][kb][lane];
+        bf16x8 h8[NCT], l8[NCT];
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+          h8[ct] = kThetaRegs ? th[kThetaRegs ? kb : 0] : s.thl[ct][0][kb][lane];
+          l8[ct] = kThetaRegs ? tl[kThetaRegs ? kb : 0] : s.thl[ct][1][kb][lane];
         }
-        z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h[kb], h8, z, 0, 0, 0);
-        z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h[kb], l8, z, 0, 0, 0);
-        z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l[kb], h8, z, 0, 0, 0);
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) z[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h[kb], h8[ct], z[ct], 0, 0, 0);
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) z[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h[kb], l8[ct], z[ct], 0, 0, 0);
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) z[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l[kb], h8[ct], z[ct], 0, 0, 0);
       }
     };
-    // one block: rows of Z_j (zc) with labels and B operands bc, then G += R_j X_j
-    auto step = [&](int j, const floatx16& zc, const BBuf& bc) {
+    // one block: rows of Z_j with labels and B operands bc, then G += R_j X_j
+    auto step = [&](const floatx16 (&z)[NCT], const BBuf& bc) {
       float yv[16];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -451,50 +441,54 @@ struct Bf16Engine {
         yv[4 * q + 2] = bc.y[q].z;
         yv[4 * q + 3] = bc.y[q].w;
       }
-      float rv[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        if constexpr (WANT_POT) {
-          float cc;
-          rv[r] = lr_row_full_hw(zc[r], yv[r], cc);
-          upart += cc;  // padding rows are taken out after the loop
-        } else {
-          rv[r] = lr_row_grad_hw(zc[r], yv[r]);
+      for (int ct = 0; ct < NCT; ++ct) {
+        float rv[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          if constexpr (WANT_POT) {
+            float cc;
+            rv[r] = lr_row_full_hw(z[ct][r], yv[r], cc);
+            acc.u[ct] += cc;  // padding rows are taken out after the loop
+          } else {
+            rv[r] = lr_row_grad_hw(z[ct][r], yv[r]);
+          }
         }
-      }
-      typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-      u32x4 ph[2], pl[2];
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 ph[2], pl[2];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        uint32_t hw, lw;
-        split_pair(rv[2 * q], rv[2 * q + 1], hw, lw);
-        ph[q >> 2][q & 3] = hw;
-        pl[q >> 2][q & 3] = lw;
-      }
+        for (int q = 0; q < 8; ++q) {
+          uint32_t hw, lw;
+          split_pair(rv[2 * q], rv[2 * q + 1], hw, lw);
+          ph[q >> 2][q & 3] = hw;
+          pl[q >> 2][q & 3] = lw;
+        }
 #pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2) {
-        const bf16x8 rh = __builtin_bit_cast(bf16x8, ph[kb2]), rl = __builtin_bit_cast(bf16x8, pl[kb2]);
+        for (int kb2 = 0; kb2 < 2; ++kb2) {
+          const bf16x8 rh = __builtin_bit_cast(bf16x8, ph[kb2]), rl = __builtin_bit_cast(bf16x8, pl[kb2]);
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          gacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, bc.h[kb2][nb], gacc[nb], 0, 0, 0);
-          gacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, bc.l[kb2][nb], gacc[nb], 0, 0, 0);
-          gacc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rl, bc.h[kb2][nb], gacc[nb], 0, 0, 0);
+          for (int nb = 0; nb < NB; ++nb) {
+            floatx16& ga = acc.g[ct][nb];
+            ga = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, bc.h[kb2][nb], ga, 0, 0, 0);
+            ga = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rh, bc.l[kb2][nb], ga, 0, 0, 0);
+            ga = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rl, bc.h[kb2][nb], ga, 0, 0, 0);
+          }
         }
       }
     };
     for (int j = 0; j < nmine; ++j) {
       ABuf a;
       BBuf b;
-      floatx16 z;
+      floatx16 z[NCT];
       load_a(a, j);
-      // At d <= 64 (two waves per SIMD) a wave issuing its first GEMM and the next loads runs at raised
-      // priority, so that the other wave's row functions fill the vector ALU meanwhile (measured 3%
-      // faster per HMC iteration at the bench shape; at d > 64, one wave per SIMD, it does not apply)
-      if constexpr (DP == 64) __builtin_amdgcn_s_setprio(1);
+      // At two waves per SIMD a wave issuing its first GEMM and the next loads runs at raised priority, so that
+      // the other wave's row functions fill the vector ALU meanwhile (measured 3% faster per HMC iteration at
+      // the bench shape; at one wave per SIMD it does not apply)
+      if constexpr (NW == 8) __builtin_amdgcn_s_setprio(1);
       gemm1(a, z);
       load_b(b, j);
-      if constexpr (DP == 64) __builtin_amdgcn_s_setprio(0);
-      step(j, z, b);
+      if constexpr (NW == 8) __builtin_amdgcn_s_setprio(0);
+      step(z, b);
     }
     if constexpr (WANT_POT) {
       // padding rows of the last block (x = 0, y = 0.5: z = 0) each added the same term
@@ -505,15 +499,33 @@ struct Bf16Engine {
         int npad = 0;
 #pragma unroll
         for (int r = 0; r < 16; ++r) npad += (rbl * 32 + acc_row(r, lane) >= n);
-        upart -= (float)npad * cpad;
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) acc.u[ct] -= (float)npad * cpad;
       }
+#pragma unroll
+      for (int ct = 0; ct < NCT; ++ct) s.ured[w][g][ct * CT + col] = acc.u[ct];
     }
-    // every wave leaves its partials; readers sum them over the waves in order (deterministic)
-    s.ured[w][g][col] = upart;
+  }
+
+  // Leaves the wave's partial gradient of tile ct in s.gred[w] ([chain][GS]); readers (after a barrier) sum the
+  // waves' in order.
+  static MOCAT_DEV void put_partials(Smem& s, const Acc& acc, int ct) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, col = lane & 31;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s.gred[w][acc_row(r, lane) * GS + nb * 32 + col] = gacc[nb][r];
+      for (int r = 0; r < 16; ++r) s.gred[w][acc_row(r, lane) * GS + nb * 32 + col] = acc.g[ct][nb][r];
+  }
+  static MOCAT_DEV floatx4 gradient(const Smem& s, int c, int k) {
+    floatx4 v = *reinterpret_cast<const floatx4*>(&s.gred[0][c * GS + k]);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const floatx4*>(&s.gred[w][c * GS + k]);
+    return v;
+  }
+  static MOCAT_DEV float potential(const Smem& s, int c) {  // c: chain of the NCT tiles
+    float lk = 0.f;
+    for (int w = 0; w < NW; ++w) lk += s.ured[w][0][c] + s.ured[w][1][c];
+    return lk;
   }
 };
 
@@ -680,6 +692,67 @@ __global__ __launch_bounds__(NT) void lr_eval_kernel(LrArgs a, const float* __re
   if (t < CT && c0 + t < C) {
     if (prior_pot) prior_pot[c0 + t] = ts.prior[t];
     if (lik_pot) lik_pot[c0 + t] = ts.likv[t];
+  }
+}
+
+// The evaluation with the bf16x3 engine: thread t owns chain c = t % 32 of each of the NCT tiles and the columns
+// k0 = EPT (t / 32) .. of it, whose values stay in registers.
+template <int DP, int NT, int NCT>
+__global__ __launch_bounds__(NT) void lr_eval_bf16_kernel(LrArgs a, const float* __restrict__ theta, int64_t C,
+                                                          float* prior_pot, float* lik_pot, float* grad_prior,
+                                                          float* grad_lik) {
+  using E = Bf16Engine<DP, NT, NCT>;
+  constexpr int NG = NT / CT, EPT = DP / NG;
+  static_assert(NG * EPT == DP && EPT % 4 == 0, "thread ownership");
+  __shared__ typename E::Smem es;
+  const int t = threadIdx.x, c = t % CT, kg = t / CT, k0 = kg * EPT;
+  const int d = a.d;
+  const int64_t c0 = (int64_t)blockIdx.x * (NCT * CT);
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    const int64_t chain = c0 + ct * CT + c;
+    float th[EPT];
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) {
+      th[q] = (chain < C && k0 + q < d) ? theta[chain * d + k0 + q] : 0.f;
+      if (grad_prior && chain < C && k0 + q < d) grad_prior[chain * d + k0 + q] = a.prior_prec * th[q];
+    }
+#pragma unroll
+    for (int q = 0; q < EPT; q += 4) E::put_theta(es, ct, c, k0 + q, &th[q]);
+  }
+  __syncthreads();
+  typename E::Acc acc;
+  if (lik_pot)
+    E::template partials<true>(es, a.packed, a.n, acc);
+  else
+    E::template partials<false>(es, a.packed, a.n, acc);
+#pragma unroll
+  for (int ct = 0; ct < NCT; ++ct) {
+    if (ct) __syncthreads();  // the previous tile's partials have been read
+    E::put_partials(es, acc, ct);
+    __syncthreads();
+    const int64_t chain = c0 + ct * CT + c;
+#pragma unroll
+    for (int q = 0; q < EPT; q += 4) {
+      const floatx4 gv = E::gradient(es, c, k0 + q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (grad_lik && chain < C && k0 + q + e < d) grad_lik[chain * d + k0 + q + e] = gv[e];
+    }
+  }
+  if (lik_pot && t < NCT * CT && c0 + t < C) lik_pot[c0 + t] = E::potential(es, t);
+  if (prior_pot) {
+    const int lane = t & (kWave - 1);
+    for (int64_t chain = c0 + t / kWave; chain < C && chain < c0 + NCT * CT; chain += E::NW) {
+      float s2 = 0.f;
+      for (int q = lane; q < d; q += kWave) s2 += theta[chain * d + q] * theta[chain * d + q];
+      s2 = wave_sum(s2);
+      // prec == 0: improper flat prior, potential 0 (mocat's default uniform prior, core.py:183-189)
+      if (lane == 0)
+        prior_pot[chain] = a.prior_prec > 0.f
+                               ? fmaf(0.5f * (float)d, kLog2Pi - logf(a.prior_prec), 0.5f * a.prior_prec * s2)
+                               : 0.f;
+    }
   }
 }
 
@@ -884,42 +957,45 @@ __global__ __launch_bounds__(NT) void hmc_lr_kernel(HmcArgs h) {
 constexpr int kThreads = 512;
 
 // The same iteration as hmc_lr_kernel for the bf16x3 engine, with the tile state in
-// registers: thread t owns chain c = t % 32 and the EPT = DP / (NT / 32) columns k0 = EPT * (t / 32) ..
-// of position, momentum and gradient. A leapfrog step is then: update the owned elements and write
-// their bf16 hi/lo split into the engine's theta operand (barrier), the engine's block loop (barrier),
+// registers: thread t owns, in each of the NCT tiles, chain c = t % 32 and the EPT = DP / (NT / 32) columns
+// k0 = EPT * (t / 32) .. of position, momentum and gradient. A leapfrog step is then: update the owned elements
+// and write their bf16 hi/lo split into the engine's theta operand (barrier), the engine's block loop (barrier),
 // and the owned gradient elements summed from every wave's partials. The refreshed momenta, position
 // and gradient of the pre-proposal state stay in global memory until a proposal is accepted (as in
-// hmc_lr_kernel); per-chain scalars and keys live in LDS.
-template <int DP, int NT>
+// hmc_lr_kernel); per-chain scalars and keys live in LDS and in the first NCT * 32 threads.
+template <int DP, int NT, int NCT>
 __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
-  using E = Bf16Engine<DP, NT>;
+  using E = Bf16Engine<DP, NT, NCT>;
   constexpr int NG = NT / CT;  // column groups
   constexpr int EPT = DP / NG;
-  static_assert(NG * EPT == DP && EPT % 4 == 0, "thread ownership");
+  constexpr int NC = NCT * CT;  // chains of the workgroup
+  static_assert(NG * EPT == DP && EPT % 4 == 0 && NC <= NT, "thread ownership");
   __shared__ typename E::Smem es;
-  __shared__ float sq0[NG][CT], sq1[NG][CT], sqt[NG][CT];
-  __shared__ float step[CT], pot[CT], prior[CT], likv[CT], alpha[CT];
-  __shared__ uint32_t sub[CT][2];
-  __shared__ int accept[CT];
+  __shared__ float sq0[NG][NC], sq1[NG][NC], sqt[NG][NC];
+  __shared__ float step[NC], pot[NC], prior[NC], likv[NC], alpha[NC];
+  __shared__ uint32_t sub[NC][2];
+  __shared__ int accept[NC];
   const int t = threadIdx.x, c = t % CT, kg = t / CT, k0 = kg * EPT;
   const int d = h.lr.d;
-  const int64_t c0 = (int64_t)blockIdx.x * CT;
-  const int nvalid = (int)((h.C - c0) < CT ? (h.C - c0) : CT);
-  const bool cv = c < nvalid;
-  const int64_t row = (c0 + c) * (int64_t)d;
+  const int64_t c0 = (int64_t)blockIdx.x * NC;
+  const int nvalid = (int)((h.C - c0) < NC ? (h.C - c0) : NC);
   const float prec = h.lr.prior_prec, temp = h.lr.temperature;
+  auto valid = [&](int ct) { return ct * CT + c < nvalid; };
+  auto row = [&](int ct) { return (c0 + ct * CT + c) * (int64_t)d; };
 
-  float th[EPT], p[EPT], g[EPT];
+  float th[NCT][EPT], p[NCT][EPT], g[NCT][EPT];
 #pragma unroll
-  for (int q = 0; q < EPT; ++q) {
-    const int k = k0 + q;
-    const bool v = cv && k < d;
-    th[q] = v ? h.theta[row + k] : 0.f;
-    p[q] = v ? h.mom[row + k] : 0.f;
-    g[q] = v ? h.grad[row + k] : 0.f;
-  }
+  for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) {
+      const int k = k0 + q;
+      const bool v = valid(ct) && k < d;
+      th[ct][q] = v ? h.theta[row(ct) + k] : 0.f;
+      p[ct][q] = v ? h.mom[row(ct) + k] : 0.f;
+      g[ct][q] = v ? h.grad[row(ct) + k] : 0.f;
+    }
   Key key{0u, 0u};
-  if (t < CT) {
+  if (t < NC) {
     const bool v = t < nvalid;
     pot[t] = v ? h.pot[c0 + t] : 0.f;
     prior[t] = v ? h.prior[c0 + t] : 0.f;
@@ -934,7 +1010,7 @@ __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
     // ---- always: p <- -p ; (key, sub) = split(key) ; OU refresh (standard_mcmc.py:107-123); then the
     // proposal's keys = split(key, L+1), key = keys[0] (standard_mcmc.py:129-131)
     float pot0 = 0.f, prior0 = 0.f, lik0 = 0.f;
-    if (t < CT) {
+    if (t < NC) {
       const Key nk = split_at(key, 2, 0), sk = split_at(key, 2, 1);
       sub[t][0] = sk.a;
       sub[t][1] = sk.b;
@@ -944,72 +1020,67 @@ __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
       lik0 = likv[t];
     }
     __syncthreads();
-    const float hh = step[c];
-    {
-      const float decay = __expf(-h.friction * hh);
-      const float noise = sqrtf(1.f - __expf(-2.f * h.friction * hh));
-      const Key sk{sub[c][0], sub[c][1]};
+    float hh[NCT];
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
+      hh[ct] = step[ct * CT + c];
+      const float decay = __expf(-h.friction * hh[ct]);
+      const float noise = sqrtf(1.f - __expf(-2.f * h.friction * hh[ct]));
+      const Key sk{sub[ct * CT + c][0], sub[ct * CT + c][1]};
       float s2 = 0.f;
 #pragma unroll
       for (int q = 0; q < EPT; ++q) {
         const int k = k0 + q;
         if (k < d) {
-          p[q] = -p[q] * decay + noise * normal_from_bits(bits_at(sk, (uint32_t)d, (uint32_t)k));
-          if (cv) h.mom[row + k] = p[q];  // the refreshed momenta, kept for a rejection
+          p[ct][q] = -p[ct][q] * decay + noise * normal_from_bits(bits_at(sk, (uint32_t)d, (uint32_t)k));
+          if (valid(ct)) h.mom[row(ct) + k] = p[ct][q];  // the refreshed momenta, kept for a rejection
         }
-        s2 += p[q] * p[q];
+        s2 += p[ct][q] * p[ct][q];
       }
-      sq0[kg][c] = s2;
+      sq0[kg][ct * CT + c] = s2;
     }
     // ---- leapfrog (utils.py:117-146)
     for (int s = 0; s < h.leapfrog_steps; ++s) {
       const bool last = s == h.leapfrog_steps - 1;
-      float s2 = 0.f;
 #pragma unroll
-      for (int q = 0; q < EPT; ++q) {
-        const float ph = p[q] - (hh / 2.f) * g[q];
-        p[q] = ph;
-        th[q] = (k0 + q < d) ? th[q] + hh * ph : 0.f;
-        s2 += th[q] * th[q];
-      }
-      if (last) sqt[kg][c] = s2;
-      typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+      for (int ct = 0; ct < NCT; ++ct) {
+        float s2 = 0.f;
 #pragma unroll
-      for (int j = 0; j < EPT / 4; ++j) {
-        bf16x4 h4, l4;
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          __bf16 hb, lb;
-          split_bf16(th[4 * j + s4], hb, lb);
-          h4[s4] = hb;
-          l4[s4] = lb;
+        for (int q = 0; q < EPT; ++q) {
+          const float ph = p[ct][q] - (hh[ct] / 2.f) * g[ct][q];
+          p[ct][q] = ph;
+          th[ct][q] = (k0 + q < d) ? th[ct][q] + hh[ct] * ph : 0.f;
+          s2 += th[ct][q] * th[ct][q];
         }
-        // columns colb .. colb + 3 of chain c: operand (kb, lane c + 32 * half), elements colb % 8 ..
-        const int colb = k0 + 4 * j;
-        const int ln = c + 32 * ((colb / 8) & 1);
-        reinterpret_cast<bf16x4*>(&es.thl[0][colb / 16][ln])[(colb / 4) & 1] = h4;
-        reinterpret_cast<bf16x4*>(&es.thl[1][colb / 16][ln])[(colb / 4) & 1] = l4;
+        if (last) sqt[kg][ct * CT + c] = s2;
+#pragma unroll
+        for (int q = 0; q < EPT; q += 4) E::put_theta(es, ct, c, k0 + q, &th[ct][q]);
       }
       __syncthreads();
+      typename E::Acc acc;
       if (last)
-        E::template partials<true>(es, h.lr.packed, h.lr.n);
+        E::template partials<true>(es, h.lr.packed, h.lr.n, acc);
       else
-        E::template partials<false>(es, h.lr.packed, h.lr.n);
-      __syncthreads();
+        E::template partials<false>(es, h.lr.packed, h.lr.n, acc);
 #pragma unroll
-      for (int q = 0; q < EPT; q += 4) {
-        floatx4 acc = *reinterpret_cast<const floatx4*>(&es.gred[0][c * E::GS + k0 + q]);
+      for (int ct = 0; ct < NCT; ++ct) {
+        if (ct) __syncthreads();  // the previous tile's partials have been read
+        E::put_partials(es, acc, ct);
+        __syncthreads();
 #pragma unroll
-        for (int w = 1; w < E::NW; ++w) acc += *reinterpret_cast<const floatx4*>(&es.gred[w][c * E::GS + k0 + q]);
+        for (int q = 0; q < EPT; q += 4) {
+          const floatx4 gv = E::gradient(es, c, k0 + q);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          g[q + e] = prec * th[q + e] + temp * acc[e];
-          p[q + e] = p[q + e] - (hh / 2.f) * g[q + e];
+          for (int e = 0; e < 4; ++e) {
+            // explicit, so that every tile count contracts it alike
+            g[ct][q + e] = fmaf(temp, gv[e], prec * th[ct][q + e]);
+            p[ct][q + e] = p[ct][q + e] - (hh[ct] / 2.f) * g[ct][q + e];
+          }
         }
       }
-      if (last && t < CT) {
-        float lk = 0.f, st = 0.f;
-        for (int w = 0; w < E::NW; ++w) lk += es.ured[w][0][t] + es.ured[w][1][t];
+      if (last && t < NC) {
+        const float lk = E::potential(es, t);
+        float st = 0.f;
         for (int q = 0; q < NG; ++q) st += sqt[q][t];
         // prec == 0: improper flat prior, potential 0 (mocat's default uniform prior, core.py:183-189)
         const float pr = prec > 0.f ? 0.5f * prec * st + 0.5f * (float)d * (kLog2Pi - logf(prec)) : 0.f;
@@ -1017,16 +1088,18 @@ __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
         likv[t] = lk;
         pot[t] = pr + temp * lk;
       }
+      if (NCT > 1 && !last) __syncthreads();  // the last tile's partials have been read before the next step's
     }
-    {
+#pragma unroll
+    for (int ct = 0; ct < NCT; ++ct) {
       float s2 = 0.f;
 #pragma unroll
-      for (int q = 0; q < EPT; ++q) s2 += p[q] * p[q];
-      sq1[kg][c] = s2;
+      for (int q = 0; q < EPT; ++q) s2 += p[ct][q] * p[ct][q];
+      sq1[kg][ct * CT + c] = s2;
     }
     __syncthreads();
     // ---- correction (metropolis.py:48-70, 118-161)
-    if (t < CT) {
+    if (t < NC) {
       float k0s = 0.f, k1s = 0.f;
       for (int q = 0; q < NG; ++q) {
         k0s += sq0[q][t];
@@ -1058,25 +1131,29 @@ __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
     }
     __syncthreads();
     // accepted: momenta <- -p' and the proposal is stored; rejected: the pre-proposal state is read back
-    const bool acc = accept[c] != 0;
 #pragma unroll
-    for (int q = 0; q < EPT; ++q) {
-      const int k = k0 + q;
-      const bool v = cv && k < d;
-      if (acc) {
-        p[q] = -p[q];
-        if (v) {
-          h.theta[row + k] = th[q];
-          h.grad[row + k] = g[q];
+    for (int ct = 0; ct < NCT; ++ct) {
+      const bool acc = accept[ct * CT + c] != 0;
+#pragma unroll
+      for (int q = 0; q < EPT; ++q) {
+        const int k = k0 + q;
+        const bool v = valid(ct) && k < d;
+        if (acc) {
+          p[ct][q] = -p[ct][q];
+          if (v) {
+            h.theta[row(ct) + k] = th[ct][q];
+            h.grad[row(ct) + k] = g[ct][q];
+          }
+        } else {
+          p[ct][q] = v ? h.mom[row(ct) + k] : 0.f;
+          th[ct][q] = v ? h.theta[row(ct) + k] : 0.f;
+          g[ct][q] = v ? h.grad[row(ct) + k] : 0.f;
         }
-      } else {
-        p[q] = v ? h.mom[row + k] : 0.f;
-        th[q] = v ? h.theta[row + k] : 0.f;
-        g[q] = v ? h.grad[row + k] : 0.f;
-      }
-      if (v) {
-        if (h.tr_value) h.tr_value[((int64_t)it * h.C + c0 + c) * d + k] = th[q];
-        if (h.tr_mom) h.tr_mom[((int64_t)it * h.C + c0 + c) * d + k] = p[q];
+        if (v) {
+          const int64_t o = ((int64_t)it * h.C + c0 + ct * CT + c) * d + k;
+          if (h.tr_value) h.tr_value[o] = th[ct][q];
+          if (h.tr_mom) h.tr_mom[o] = p[ct][q];
+        }
       }
     }
     if (t < nvalid) {
@@ -1088,8 +1165,10 @@ __global__ __launch_bounds__(NT) void hmc_lr_bf16_kernel(HmcArgs h) {
   }
   // write back the final per-chain state (position and gradient are already in place)
 #pragma unroll
-  for (int q = 0; q < EPT; ++q)
-    if (cv && k0 + q < d) h.mom[row + k0 + q] = p[q];
+  for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+    for (int q = 0; q < EPT; ++q)
+      if (valid(ct) && k0 + q < d) h.mom[row(ct) + k0 + q] = p[ct][q];
   if (t < nvalid) {
     h.pot[c0 + t] = pot[t];
     h.prior[c0 + t] = prior[t];
@@ -1127,28 +1206,41 @@ int dispatch_hmc(const HmcArgs& h, hipStream_t st) {
 }
 
 // bf16x3: two waves per SIMD at d <= 64; at d <= 128 one wave per SIMD (the operand registers of a
-// 128-column block, and the LDS of eight waves' partial gradients, do not fit two waves)
+// 128-column block, and the LDS of eight waves' partial gradients, do not fit two waves). Two tiles of
+// chains per workgroup from kTwoTiles chains (a workgroup for each of 256 CUs): X 20000 x 100, 65536 positions,
+// potential and gradient 2107 -> 1697 us, one MALA move 2141 -> 1860; X 2000 x 50, 32768 positions 89 -> 70.
 constexpr int kBf16Threads64 = 512, kBf16Threads128 = 256;
+constexpr int64_t kTwoTiles = 256 * 2 * CT;
 
-int dispatch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, float* lp, float* gp, float* gl,
-                       hipStream_t st) {
-  const unsigned blocks = (unsigned)((C + CT - 1) / CT);
-  if (a.d <= 64)
-    hipLaunchKernelGGL((lr_eval_kernel<Bf16Engine<64, kBf16Threads64>, 64, kBf16Threads64>), dim3(blocks),
-                       dim3(kBf16Threads64), 0, st, a, theta, C, pp, lp, gp, gl);
+unsigned tiles(int64_t C, int nct) { return (unsigned)((C + nct * CT - 1) / (nct * CT)); }
+
+template <int DP>
+int launch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, float* lp, float* gp, float* gl,
+                     hipStream_t st) {
+  constexpr int NT = DP == 64 ? kBf16Threads64 : kBf16Threads128;
+  if (C < kTwoTiles)
+    hipLaunchKernelGGL((lr_eval_bf16_kernel<DP, NT, 1>), dim3(tiles(C, 1)), dim3(NT), 0, st, a, theta, C, pp, lp, gp, gl);
   else
-    hipLaunchKernelGGL((lr_eval_kernel<Bf16Engine<128, kBf16Threads128>, 128, kBf16Threads128>), dim3(blocks),
-                       dim3(kBf16Threads128), 0, st, a, theta, C, pp, lp, gp, gl);
+    hipLaunchKernelGGL((lr_eval_bf16_kernel<DP, NT, 2>), dim3(tiles(C, 2)), dim3(NT), 0, st, a, theta, C, pp, lp, gp, gl);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }
 
+int dispatch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, float* lp, float* gp, float* gl,
+                       hipStream_t st) {
+  return a.d <= 64 ? launch_eval_bf16<64>(a, theta, C, pp, lp, gp, gl, st)
+                   : launch_eval_bf16<128>(a, theta, C, pp, lp, gp, gl, st);
+}
+
 int dispatch_hmc_bf16(const HmcArgs& h, hipStream_t st) {
-  const unsigned blocks = (unsigned)((h.C + CT - 1) / CT);
-  if (h.lr.d <= 64)
-    hipLaunchKernelGGL((hmc_lr_bf16_kernel<64, kBf16Threads64>), dim3(blocks), dim3(kBf16Threads64), 0, st, h);
+  if (h.lr.d <= 64)  // two tiles' chain state does not fit two waves per SIMD (spilled: 576 against 518 us)
+    hipLaunchKernelGGL((hmc_lr_bf16_kernel<64, kBf16Threads64, 1>), dim3(tiles(h.C, 1)), dim3(kBf16Threads64), 0, st, h);
+  else if (h.C < kTwoTiles)
+    hipLaunchKernelGGL((hmc_lr_bf16_kernel<128, kBf16Threads128, 1>), dim3(tiles(h.C, 1)), dim3(kBf16Threads128), 0, st,
+                       h);
   else
-    hipLaunchKernelGGL((hmc_lr_bf16_kernel<128, kBf16Threads128>), dim3(blocks), dim3(kBf16Threads128), 0, st, h);
+    hipLaunchKernelGGL((hmc_lr_bf16_kernel<128, kBf16Threads128, 2>), dim3(tiles(h.C, 2)), dim3(kBf16Threads128), 0, st,
+                       h);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }
