@@ -88,14 +88,21 @@ def require_gpu(t: torch.Tensor | None = None):
         raise MocatKernelError("mocat_amd kernels take device tensors; got a host tensor")
 
 
+# The two helpers below run several times per entry-point call, and for the smallest calls they are a good part of the
+# time (a potential and gradient of 40 points: 21.6 us a call, 9 of them here): the current stream comes from torch's
+# raw handle (0.4 us instead of 2.9), and a device tensor is its own proof of a GPU (0.3 us instead of 0.9).
 def stream_handle() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+
+
+_NULL = ctypes.c_void_p(0)
 
 
 def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
     if t is None:
-        return ctypes.c_void_p(0)
-    require_gpu(t)
+        return _NULL
+    if not t.is_cuda:
+        require_gpu(t)
     if not t.is_contiguous():
         raise MocatKernelError("mocat_amd kernels take contiguous tensors")
     return ctypes.c_void_p(t.data_ptr())
