@@ -824,6 +824,112 @@ __global__ __launch_bounds__(256) void resample_search_kernel(const uint64_t* __
     idx[j] = ancestor_at(csum, n, W, k, method, u_sys, j);
 }
 
+// From kSplitMin weights the prefix sums are spread over chunks of RCH weights, a workgroup each (the two launches of
+// one workgroup and the search: 17 us at 4096 log-weights, 48 at 16384, 170 at 65536; these three: 15, 15, 16, and 37 us
+// at 2^20): the chunks' maxima (left in the output's first entries until the search overwrites them),
+// then each chunk's own inclusive sums, then the search, which adds the earlier chunks' totals. All
+// sums are exact integers, so they and the ancestors are those of one workgroup.
+constexpr int RT = 1024, RCH = 4 * RT;
+constexpr int64_t kSplitMin = 4096, kSplitChunks = 4096;  // chunk totals fit the search's LDS up to 2^24 weights
+
+__global__ __launch_bounds__(RT) void resample_max_kernel(const float* __restrict__ w, int64_t n, int from_log,
+                                                          float* __restrict__ cmax) {
+  __shared__ float red[RT / kWave];
+  float m = from_log ? -INFINITY : 0.f;
+  const int64_t i0 = (int64_t)blockIdx.x * RCH;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t i = i0 + k * RT + threadIdx.x;
+    if (i < n) m = fmaxf(m, w[i]);
+  }
+  m = block_max(m, red);
+  if (threadIdx.x == 0) cmax[blockIdx.x] = m;
+}
+
+__global__ __launch_bounds__(RT) void resample_chunk_kernel(const float* __restrict__ w, int64_t n, int from_log,
+                                                            const float* __restrict__ cmax, uint64_t* __restrict__ csum) {
+  __shared__ float red[RT / kWave];
+  __shared__ uint64_t wtot[RT / kWave];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+  float m = from_log ? -INFINITY : 0.f;
+  for (int64_t c = t; c < gridDim.x; c += RT) m = fmaxf(m, cmax[c]);
+  m = block_max(m, red);
+  auto weight = [&](float x) {  // as resample_csum_kernel
+    const float v = from_log ? __expf(x - m) : x;
+    return v > 0.f ? v : 0.f;
+  };
+  const int shift = quant_shift(weight(m), n);  // the hardware exponential is monotone
+  const int64_t i0 = (int64_t)blockIdx.x * RCH + 4 * t;
+  uint64_t q[4], own = 0ull;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    q[k] = i0 + k < n ? quantise(weight(w[i0 + k]), shift) : 0ull;
+    own += q[k];
+  }
+  const uint64_t incl = wave_inclusive_scan(own);
+  if (lane == kWave - 1) wtot[wv] = incl;
+  __syncthreads();
+  uint64_t run = incl - own;
+  for (int k = 0; k < wv; ++k) run += wtot[k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    run += q[k];
+    if (i0 + k < n) csum[i0 + k] = run;
+  }
+}
+
+__global__ __launch_bounds__(256) void resample_split_search_kernel(const uint64_t* __restrict__ csum, int64_t n,
+                                                                    const uint32_t* key, int method, int32_t* idx) {
+  extern __shared__ uint64_t ends[];  // inclusive sums at the chunks' ends
+  const int nchunk = (int)((n + RCH - 1) / RCH);
+  for (int c = threadIdx.x; c < nchunk; c += 256) {
+    const int64_t e = (int64_t)(c + 1) * RCH;
+    ends[c] = csum[(e < n ? e : n) - 1];
+  }
+  __syncthreads();
+  if (threadIdx.x < kWave) {  // one wave turns the totals into running sums
+    uint64_t base = 0ull;
+    for (int c0 = 0; c0 < nchunk; c0 += kWave) {
+      const int c = c0 + threadIdx.x;
+      const uint64_t v = wave_inclusive_scan(c < nchunk ? ends[c] : (uint64_t)0) + base;
+      if (c < nchunk) ends[c] = v;
+      base = __shfl(v, kWave - 1, kWave);
+    }
+  }
+  __syncthreads();
+  const Key k{key[0], key[1]};
+  const double W = (double)ends[nchunk - 1];
+  const double u_sys = method == 0 ? systematic_uniform(k) : 0.0;
+  for (int64_t j = blockIdx.x * (int64_t)256 + threadIdx.x; j < n; j += (int64_t)gridDim.x * 256) {
+    const double t = method == 0 ? ((double)j + u_sys) * (W / (double)n)
+                                 : (double)uniform_from_bits(bits_at(k, (uint32_t)n, (uint32_t)j), 0.f, 1.f) * W;
+    // first index whose sum exceeds t (the sums are integers below 2^52), n - 1 if none
+    int lo = 0, hi = nchunk;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if ((double)ends[mid] > t)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    int64_t a = n - 1;
+    if (lo < nchunk) {
+      const uint64_t off = lo ? ends[lo - 1] : 0ull;
+      const int64_t b = (int64_t)lo * RCH;
+      int64_t l = 0, h = (b + RCH < n ? RCH : n - b);
+      while (l < h) {
+        const int64_t mid = (l + h) >> 1;
+        if ((double)(off + csum[b + mid]) > t)
+          h = mid;
+        else
+          l = mid + 1;
+      }
+      a = b + l < n ? b + l : n - 1;
+    }
+    idx[j] = (int32_t)a;
+  }
+}
+
 // random.categorical(key, lw, shape=(n_out,)): one wave per unit of two outputs, the lanes over the n
 // Gumbel draws of each row of the (n_out, n) matrix.
 __global__ __launch_bounds__(256) void categorical_kernel(const float* __restrict__ lw, int64_t n, int64_t n_out,
@@ -2523,10 +2629,21 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters, bool small) {
 
 namespace {
 
-// The two launches of resampling from weights: exact prefix sums into ws (n uint64, every entry
+// The launches of resampling from weights: exact prefix sums into ws (n uint64, every entry
 // written before it is read), then the ancestor search.
 int launch_resample(const float* weights, int64_t n, int method, int from_log, const uint32_t* key, uint64_t* ws,
                     int32_t* idx, hipStream_t stream) {
+  const int64_t nchunk = (n + RCH - 1) / RCH;
+  if (n > kSplitMin && nchunk <= kSplitChunks) {
+    const dim3 grid((unsigned)nchunk);
+    float* cmax = reinterpret_cast<float*>(idx);
+    hipLaunchKernelGGL(resample_max_kernel, grid, dim3(RT), 0, stream, weights, n, from_log, cmax);
+    hipLaunchKernelGGL(resample_chunk_kernel, grid, dim3(RT), 0, stream, weights, n, from_log, (const float*)cmax, ws);
+    hipLaunchKernelGGL(resample_split_search_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)), dim3(256),
+                       (size_t)nchunk * sizeof(uint64_t), stream, (const uint64_t*)ws, n, key, method, idx);
+    MOCAT_LAUNCH_CHECK();
+    return MOCAT_OK;
+  }
   hipLaunchKernelGGL(resample_csum_kernel, dim3(1), dim3(NT), 0, stream, weights, n, from_log, ws);
   const int64_t blocks = (n + 255) / 256;
   hipLaunchKernelGGL(resample_search_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,

@@ -28,57 +28,9 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint32_t* __restrict_
 
 struct Smem {
   double m[NW], s1[NW], s2[NW];
-  double bc[8];
+  double bc[2];
+  int pass;
 };
-
-// (lse(w), lse(2w)) of w_i = lw_i - db * lik_i over the block, FP64, in two passes: the maximum m,
-// then sum exp(w_i - m) and its square (one exponential per element); partial sums are combined in a
-// fixed order (lanes by butterfly, waves in index order).
-__device__ void lse_pair(const float* __restrict__ lw, const float* __restrict__ lik, int64_t n, double db, Smem& s,
-                         double& lse, double& lse2) {
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  double mx = -INFINITY;
-  int has_nan = 0;
-  for (int64_t i = t; i < n; i += NT) {
-    const double v = (double)lw[i] - db * (double)lik[i];
-    if (isnan(v)) has_nan = 1;
-    else mx = fmax(mx, v);
-  }
-  const bool nan_seen = __syncthreads_or(has_nan) != 0;
-  mx = wave_max(mx);
-  if (lane == 0) s.m[w] = mx;
-  __syncthreads();
-  double m = s.m[0];
-  for (int i = 1; i < NW; ++i) m = fmax(m, s.m[i]);
-  if (nan_seen || m == -INFINITY) {
-    __syncthreads();  // every thread has read s.m before a later call rewrites it
-    lse = nan_seen ? NAN : -INFINITY;
-    lse2 = lse;
-    return;
-  }
-  double s1 = 0.0, s2 = 0.0;
-  for (int64_t i = t; i < n; i += NT) {
-    const double e = exp((double)lw[i] - db * (double)lik[i] - m);
-    s1 += e;
-    s2 += e * e;
-  }
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  __syncthreads();
-  if (lane == 0) {
-    s.s1[w] = s1;
-    s.s2[w] = s2;
-  }
-  __syncthreads();
-  double a1 = 0.0, a2 = 0.0;
-  for (int i = 0; i < NW; ++i) {
-    a1 += s.s1[i];
-    a2 += s.s2[i];
-  }
-  __syncthreads();  // every thread has read the partials before a later call rewrites them
-  lse = m + log(a1);
-  lse2 = 2.0 * m + log(a2);
-}
 
 struct TemperArgs {
   const float* lw;        // [n] current (resampled) log weights
@@ -101,82 +53,262 @@ struct TemperArgs {
   double* out;            // [8]: beta_new, ess_new, lse_new, lse_prev, log_stepsize_new, alpha_mean, iters, f_min
 };
 
-__global__ __launch_bounds__(NT) void temper_kernel(TemperArgs a) {
+// The particles of one workgroup: i = (k * G + g) * NT + t for workgroup g of G. The first kRegs per
+// thread are read once and kept in registers over all evaluations, any others are read again each time.
+constexpr int kRegs = 4;
+struct Share {
+  int64_t n, stride, first;  // stride = G * NT
+  const float *lw, *lik;
+  float rl[kRegs], rk[kRegs];
+  template <class F>
+  MOCAT_DEV void each(F f) const {
+#pragma unroll
+    for (int k = 0; k < kRegs; ++k) {
+      const int64_t i = first + k * stride;
+      if (i < n) f(i, rl[k], rk[k]);
+    }
+    for (int64_t i = first + kRegs * stride; i < n; i += stride) f(i, lw[i], lik[i]);
+  }
+};
+MOCAT_DEV Share share_of(const float* lw, const float* lik, int64_t n) {
+  Share s;
+  s.n = n;
+  s.stride = (int64_t)gridDim.x * NT;
+  s.first = (int64_t)blockIdx.x * NT + threadIdx.x;
+  s.lw = lw;
+  s.lik = lik;
+#pragma unroll
+  for (int k = 0; k < kRegs; ++k) {
+    const int64_t i = s.first + k * s.stride;
+    s.rl[k] = i < n ? lw[i] : 0.f;
+    s.rk[k] = i < n ? lik[i] : 0.f;
+  }
+  return s;
+}
+
+// Workgroups of a split evaluation, and what they exchange: two sets of slots used in turn, so that a
+// workgroup that is one exchange ahead never overwrites what another still reads, and the barrier's
+// arrival count and abort flag. A workgroup that polls max_polls times without seeing every arrival sets
+// the flag and leaves, as does every workgroup that sees it; temper_kernel<false> then does the work.
+constexpr int kMaxSplit = 32;
+static_assert(kMaxSplit <= kWave, "one wave combines the workgroups' slots");
+struct TemperWs {
+  double slot[2][kMaxSplit][4];
+  uint32_t bar[2];
+};
+struct Exchange {
+  TemperWs* ws;
+  uint32_t max_polls, count;
+
+  // Publishes this workgroup's values (thread 0's), waits for all: true when every workgroup arrived.
+  MOCAT_DEV bool run(const double* v, int nv, bool wait, Smem& s) {
+    const int par = count & 1;
+    ++count;
+    if (threadIdx.x == 0) {
+      for (int k = 0; k < nv; ++k) ws->slot[par][blockIdx.x][k] = v[k];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __hip_atomic_fetch_add(&ws->bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int ok = 1;
+      const uint32_t target = count * gridDim.x;
+      for (uint32_t polls = 0; wait; ++polls) {
+        if (__hip_atomic_load(&ws->bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+          ok = 0;
+          break;
+        }
+        if (polls >= max_polls) {
+          __hip_atomic_store(&ws->bar[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ok = 0;
+          break;
+        }
+        if (__hip_atomic_load(&ws->bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      s.pass = ok;
+    }
+    __syncthreads();
+    const bool ok = s.pass != 0;
+    __syncthreads();
+    return ok;
+  }
+  MOCAT_DEV const double* slots(int g) const { return ws->slot[(count - 1) & 1][g]; }
+};
+
+// (lse(w), lse(2w)) of w_i = lw_i - db * lik_i, FP64: the workgroup's maximum m and the sums of
+// exp(w_i - m) and its square (one exponential per element), partial sums combined in a fixed order (lanes by
+// butterfly, waves in index order, workgroups by butterfly after scaling to the common maximum), so that every
+// workgroup finds the same values and takes the same decisions. false: the exchange was given up.
+template <bool SPLIT>
+MOCAT_DEV bool lse_pair(const Share& sh, double db, Exchange& ex, Smem& s, double& lse, double& lse2) {
+  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
+  double mx = -INFINITY;
+  int has_nan = 0;
+  sh.each([&](int64_t, float l, float k) {
+    const double v = (double)l - db * (double)k;
+    if (isnan(v)) has_nan = 1;
+    else mx = fmax(mx, v);
+  });
+  const bool nan_seen = __syncthreads_or(has_nan) != 0;
+  mx = wave_max(mx);
+  if (lane == 0) s.m[w] = mx;
+  __syncthreads();
+  double m = s.m[0];
+  for (int i = 1; i < NW; ++i) m = fmax(m, s.m[i]);
+  double s1 = 0.0, s2 = 0.0;
+  if (!nan_seen && m != -INFINITY)
+    sh.each([&](int64_t, float l, float k) {
+      const double e = exp((double)l - db * (double)k - m);
+      s1 += e;
+      s2 += e * e;
+    });
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  if (lane == 0) {
+    s.s1[w] = s1;
+    s.s2[w] = s2;
+  }
+  __syncthreads();
+  double a1 = 0.0, a2 = 0.0;
+  for (int i = 0; i < NW; ++i) {
+    a1 += s.s1[i];
+    a2 += s.s2[i];
+  }
+  __syncthreads();  // every thread has read the partials before a later call rewrites them
+  bool bad = nan_seen;
+  if constexpr (SPLIT) {
+    const double v[4] = {m, a1, a2, nan_seen ? 1.0 : 0.0};
+    if (!ex.run(v, 4, true, s)) return false;
+    if (w == 0) {
+      const bool in = lane < (int)gridDim.x;
+      const double* o = ex.slots(in ? lane : 0);
+      const double mg = in ? o[0] : -INFINITY, ng = in ? o[3] : 0.0;
+      const double mm = wave_max(mg);
+      const double sc = in && mm != -INFINITY ? exp(mg - mm) : 0.0;
+      const double t1 = wave_sum(in ? o[1] * sc : 0.0), t2 = wave_sum(in ? o[2] * (sc * sc) : 0.0);
+      const double nn = wave_max(ng);
+      if (lane == 0) {
+        s.m[0] = mm;
+        s.s1[0] = t1;
+        s.s2[0] = t2;
+        s.bc[0] = nn;
+      }
+    }
+    __syncthreads();
+    m = s.m[0];
+    a1 = s.s1[0];
+    a2 = s.s2[0];
+    bad = s.bc[0] != 0.0;
+    __syncthreads();
+  }
+  if (bad || m == -INFINITY) {
+    lse = lse2 = bad ? NAN : -INFINITY;
+  } else {
+    lse = m + log(a1);
+    lse2 = 2.0 * m + log(a2);
+  }
+  return true;
+}
+
+// One evaluation is an FP64 exponential per particle and takes 10 us in one workgroup at 16384 particles, 132 us for
+// the whole search. SPLIT: a workgroup per 1024 particles (at most kMaxSplit), one exchange per evaluation;
+// the evaluations at b_t and at the chosen bound are those of the search.
+// Without SPLIT one workgroup; with a workspace only if the split search gave up.
+template <bool SPLIT>
+__global__ __launch_bounds__(NT) void temper_kernel(TemperArgs a, TemperWs* ws, uint32_t max_polls) {
   __shared__ Smem s;
+  if constexpr (!SPLIT)
+    if (ws && ws->bar[1] == 0u) return;
   const int t = threadIdx.x;
-  double lse, lse2;
+  const Share sh = share_of(a.lw, a.lik, a.n);
+  Exchange ex{ws, max_polls, 0u};
   const double logthr = log(a.ess * a.retain);
-  auto f = [&](double b) {
-    lse_pair(a.lw, a.lik, a.n, b - a.beta, s, lse, lse2);
-    return (2.0 * lse - lse2) - logthr;
-  };
-  double bnew, fmin_abs = 0.0;
+  double bnew, fmin_abs = 0.0, lse_prev, lse_new, lse2_new;
   int iters = 0;
   if (a.adaptive) {
-    double b0 = a.beta, b1 = a.max_temperature;
-    double e0 = f(b0), e1 = f(b1);
+    double b0 = a.beta, b1 = a.max_temperature, l0, m0, l1, m1;
+    if (!lse_pair<SPLIT>(sh, 0.0, ex, s, l0, m0)) return;
+    if (!lse_pair<SPLIT>(sh, b1 - a.beta, ex, s, l1, m1)) return;
+    double e0 = (2.0 * l0 - m0) - logthr, e1 = (2.0 * l1 - m1) - logthr;
+    lse_prev = l0;
     const bool increasing = e1 > e0;
     while (true) {
       const bool done = fmin(fabs(e0), fabs(e1)) < a.tol || iters >= a.max_iter || (e0 < 0 && e1 < 0) ||
                         (e0 > 0 && e1 > 0) || isnan(e0) || isnan(e1);
       if (done) break;
       const double np = b0 - e0 * (b1 - b0) / (e1 - e0);
-      const double ne = f(np);
+      double l, m;
+      if (!lse_pair<SPLIT>(sh, np - a.beta, ex, s, l, m)) return;
+      const double ne = (2.0 * l - m) - logthr;
       const bool replace_upper = increasing ? ne > 0 : ne < 0;
       if (replace_upper) {
         b1 = np;
         e1 = ne;
+        l1 = l;
+        m1 = m;
       } else {
         b0 = np;
         e0 = ne;
+        l0 = l;
+        m0 = m;
       }
       ++iters;
     }
     // bounds[argmin |evals|] (first on ties)
-    bnew = fabs(e1) < fabs(e0) ? b1 : b0;
+    const bool upper = fabs(e1) < fabs(e0);
+    bnew = upper ? b1 : b0;
+    lse_new = upper ? l1 : l0;
+    lse2_new = upper ? m1 : m0;
     fmin_abs = fmin(fabs(e0), fabs(e1));
   } else {
     bnew = a.next_beta;
+    double lse_prev2;
+    if (!lse_pair<SPLIT>(sh, 0.0, ex, s, lse_prev, lse_prev2)) return;
+    if (!lse_pair<SPLIT>(sh, bnew - a.beta, ex, s, lse_new, lse2_new)) return;
   }
   const double db = bnew - a.beta;
-  // previous lse (of lw) and the new weights
-  double lse_prev, lse_prev2;
-  lse_pair(a.lw, a.lik, a.n, 0.0, s, lse_prev, lse_prev2);
-  double lse_new, lse_new2;
-  lse_pair(a.lw, a.lik, a.n, db, s, lse_new, lse_new2);
   // weighted mean acceptance with weights exp(lw_new - max) (normalised)
   double amean = 0.0;
   if (a.alpha && a.k_alpha > 0) {
     double num = 0.0, den = 0.0;
-    for (int64_t i = t; i < a.n; i += NT) {
-      const double wi = exp((double)a.lw[i] - db * (double)a.lik[i] - lse_new);
+    sh.each([&](int64_t i, float l, float k) {
+      const double wi = exp((double)l - db * (double)k - lse_new);
       double am = 0.0;
-      for (int k = 0; k < a.k_alpha; ++k) am += (double)a.alpha[(int64_t)k * a.n + i];
+      for (int j = 0; j < a.k_alpha; ++j) am += (double)a.alpha[(int64_t)j * a.n + i];
       am /= (double)a.k_alpha;
       num += wi * am;
       den += wi;
-    }
-    __shared__ double rnum[NW], rden[NW];
+    });
     num = wave_sum(num);
     den = wave_sum(den);
     if ((t & (kWave - 1)) == 0) {
-      rnum[t / kWave] = num;
-      rden[t / kWave] = den;
+      s.s1[t / kWave] = num;
+      s.s2[t / kWave] = den;
     }
     __syncthreads();
     double N = 0.0, D = 0.0;
     for (int i = 0; i < NW; ++i) {
-      N += rnum[i];
-      D += rden[i];
+      N += s.s1[i];
+      D += s.s2[i];
+    }
+    __syncthreads();
+    if constexpr (SPLIT) {
+      const double v[2] = {N, D};
+      if (!ex.run(v, 2, blockIdx.x == 0, s)) return;
+      if (blockIdx.x == 0) {
+        N = D = 0.0;
+        for (int g = 0; g < (int)gridDim.x; ++g) {
+          N += ex.slots(g)[0];
+          D += ex.slots(g)[1];
+        }
+      }
     }
     amean = N / D;
   }
-  // written last so that lw_out may alias lw
-  __syncthreads();
-  for (int64_t i = t; i < a.n; i += NT) a.lw_out[i] = (float)((double)a.lw[i] - db * (double)a.lik[i]);
-  if (t == 0) {
+  // written last so that lw_out may alias lw: each thread its own particles
+  sh.each([&](int64_t i, float l, float k) { a.lw_out[i] = (float)((double)l - db * (double)k); });
+  if (t == 0 && blockIdx.x == 0) {
     a.out[0] = bnew;
-    a.out[1] = exp(2.0 * lse_new - lse_new2);
+    a.out[1] = exp(2.0 * lse_new - lse2_new);
     a.out[2] = lse_new;
     a.out[3] = lse_prev;
     a.out[4] = a.rm_stepsize != 0.0 ? a.log_stepsize + a.rm_stepsize * (amean - a.target) : a.log_stepsize;
@@ -184,6 +316,24 @@ __global__ __launch_bounds__(NT) void temper_kernel(TemperArgs a) {
     a.out[6] = (double)iters;
     a.out[7] = fmin_abs;
   }
+}
+
+__global__ void temper_clear_kernel(TemperWs* ws) { ws->bar[threadIdx.x] = 0u; }
+
+// One workgroup / split, the whole step with 4 search iterations: 42 / 61 us at 4096 particles, 60 / 62 at 8192, 92 / 65 at
+// 16384, 274 / 76 at 65536, 6690 / 199 at 2^20 (an exchange costs about as much as 8 particles per thread).
+constexpr int64_t kSplitMin = 12288;
+
+void launch_temper(const TemperArgs& a, TemperWs* ws, uint32_t max_polls, hipStream_t stream) {
+  if (a.n < kSplitMin) {
+    hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, (TemperWs*)nullptr, 0u);
+    return;
+  }
+  const int64_t want = (a.n + NT - 1) / NT;
+  const dim3 grid((unsigned)(want < kMaxSplit ? want : kMaxSplit));
+  hipLaunchKernelGGL(temper_clear_kernel, dim3(1), dim3(2), 0, stream, ws);
+  hipLaunchKernelGGL((temper_kernel<true>), grid, dim3(NT), 0, stream, a, ws, max_polls);
+  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, ws, 0u);
 }
 
 }  // namespace
@@ -209,7 +359,29 @@ int mocat_smc_temper(const float* log_weight, const float* lik, int64_t n, doubl
   if (!log_weight || !lik || !log_weight_out || !out || n <= 0 || max_iter < 0 || k_alpha < 0) return MOCAT_ERR_ARG;
   TemperArgs a{log_weight, lik, n, beta, ess, retain, max_temperature, tol, max_iter, adaptive, next_beta,
                alpha, k_alpha, log_stepsize, rm_stepsize, target, log_weight_out, out};
-  hipLaunchKernelGGL(temper_kernel, dim3(1), dim3(NT), 0, stream, a);
+  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, (TemperWs*)nullptr, 0u);
+  MOCAT_LAUNCH_CHECK();
+  return MOCAT_OK;
+}
+
+int mocat_smc_temper_workspace_bytes(int64_t* bytes) {
+  if (!bytes) return MOCAT_ERR_ARG;
+  *bytes = (int64_t)sizeof(TemperWs);
+  return MOCAT_OK;
+}
+
+int mocat_smc_temper_split(const float* log_weight, const float* lik, int64_t n, double beta, double ess, double retain,
+                           double max_temperature, double tol, int max_iter, int adaptive, double next_beta,
+                           const float* alpha, int k_alpha, double log_stepsize, double rm_stepsize, double target,
+                           float* log_weight_out, double* out, void* workspace, int64_t workspace_bytes, int max_polls,
+                           hipStream_t stream) {
+  if (!log_weight || !lik || !log_weight_out || !out || n <= 0 || max_iter < 0 || k_alpha < 0 || max_polls < 0 ||
+      log_weight == log_weight_out || (uintptr_t)workspace % 8)
+    return MOCAT_ERR_ARG;
+  if (!workspace || workspace_bytes < (int64_t)sizeof(TemperWs)) return MOCAT_ERR_SIZE;
+  TemperArgs a{log_weight, lik, n, beta, ess, retain, max_temperature, tol, max_iter, adaptive, next_beta,
+               alpha, k_alpha, log_stepsize, rm_stepsize, target, log_weight_out, out};
+  launch_temper(a, (TemperWs*)workspace, (uint32_t)max_polls, stream);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }

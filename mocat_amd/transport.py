@@ -34,6 +34,9 @@ _lib.register("mocat_gather_rows", [_P, _P, _lib.c_i64, _lib.c_i64, _P, _P])
 _lib.register("mocat_smc_temper", [_P, _P, _lib.c_i64, _lib.c_f64, _lib.c_f64, _lib.c_f64, _lib.c_f64, _lib.c_f64,
                                    _lib.c_i32, _lib.c_i32, _lib.c_f64, _P, _lib.c_i32, _lib.c_f64, _lib.c_f64,
                                    _lib.c_f64, _P, _P, _P])
+_lib.register("mocat_smc_temper_workspace_bytes", [_P])
+_lib.register("mocat_smc_temper_split", _lib.SIGNATURES["mocat_smc_temper"][:-1] + [_P, _lib.c_i64, _lib.c_i32, _P])
+TEMPER_POLLS = 1 << 22  # polls of one wait between the workgroups of the temperature search
 
 
 def gather_rows(t: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
@@ -112,10 +115,14 @@ class MetropolisedSMCSampler(TemperedSMCSampler):
         k_alpha = 0 if alpha_trace is None else int(alpha_trace.shape[0])
         rm = float(p.rm_stepsize) if (self.rm and alpha_trace is not None) else 0.0
         target = float(self.mcmc_sampler.tuning.target or 0.0)
-        _lib.call("mocat_smc_temper", _lib.ptr(lw), _lib.ptr(lik), int(lw.shape[0]), float(beta), float(ess),
+        nbytes = _lib.c_i64(0)
+        _lib.call("mocat_smc_temper_workspace_bytes", _lib.ctypes.byref(nbytes))
+        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=lw.device)
+        _lib.call("mocat_smc_temper_split", _lib.ptr(lw), _lib.ptr(lik), int(lw.shape[0]), float(beta), float(ess),
                   float(p.ess_threshold_retain), float(self.max_temperature), float(p.bisection_tol),
                   int(p.max_bisection_iter), int(adaptive), nb, _lib.ptr(alpha_trace), k_alpha, float(log_h), rm,
-                  target, _lib.ptr(lw_out), _lib.ptr(out), _lib.stream_handle())
+                  target, _lib.ptr(lw_out), _lib.ptr(out), _lib.ptr(ws), nbytes.value, TEMPER_POLLS,
+                  _lib.stream_handle())
         return lw_out, out.cpu().numpy()
 
     def _resample(self, state, lw, key):
