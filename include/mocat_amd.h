@@ -328,6 +328,30 @@ int mocat_smc_temper_split(const float* log_weight, const float* lik, int64_t n,
                            const float* alpha, int k_alpha, double log_stepsize, double rm_stepsize, double target,
                            float* log_weight_out, double* out, void* workspace, int64_t workspace_bytes, int max_polls,
                            hipStream_t stream);
+/* The part of one temperature before the evaluation (mocat/src/transport/smc.py:73-99): keys = split(key, n + 2),
+ * move_keys[i] = split(keys[i], 3)[0] ([n][2]), next_key = keys[n + 1]. method 0 systematic, 1 multinomial,
+ * 2 categorical: with keys[n], value_out and momenta_out = the resampled rows of value and momenta ([n][d])
+ * and log_weight_out = 0; no output may be its input. method -1: the keys alone (the others may be NULL).
+ * workspace: mocat_smc_resample_workspace_bytes bytes, 8-byte aligned. */
+int mocat_smc_resample_workspace_bytes(int64_t n, int64_t* bytes);
+int mocat_smc_resample(const uint32_t* key, int64_t n, int64_t d, int method, const float* log_weight,
+                       const float* value, const float* momenta, float* value_out, float* momenta_out,
+                       float* log_weight_out, uint32_t* move_keys, uint32_t* next_key, void* workspace,
+                       int64_t workspace_bytes, hipStream_t stream);
+/* The part after it: potential = prior_pot + beta lik_pot and grad = grad_prior + beta grad_lik (written),
+ * `steps` Metropolis-corrected iterations of mocat_hmc_lr_iterate at temperature beta with the one
+ * stepsize (written to stepsizes [n]), the step of mocat_smc_temper_split with the moves' acceptance
+ * probabilities (alpha_trace [steps][n]) and potential at the temperature found. out[9]: the eight
+ * values of mocat_smc_temper, then, as a uint64_t, how many entries of value are NaN. workspace and max_polls
+ * as mocat_smc_temper_split. */
+int mocat_smc_move(const float* X, const float* y, const void* packed, int64_t rows, int64_t d, int precision,
+                   float prior_prec, int64_t n, const float* grad_prior, const float* grad_lik, float* value,
+                   float* momenta, float* grad, float* potential, float* prior_pot, float* lik_pot, float* stepsizes,
+                   float* alpha, uint32_t* keys, int steps, int leapfrog_steps, float friction, float* alpha_trace,
+                   const float* log_weight, double beta, double stepsize, double log_stepsize, double ess,
+                   double retain, double max_temperature, double tol, int max_iter, int adaptive, double next_beta,
+                   double rm_stepsize, double target, float* log_weight_out, double* out, void* workspace,
+                   int64_t workspace_bytes, int max_polls, hipStream_t stream);
 
 /* ------------------------------------------------------------------------------------- SVGD
  * One SVGD.update with the Gaussian kernel and adagrad(step, momentum)

@@ -3,11 +3,11 @@
 Tempered SMC (MetropolisedSMCSampler / RMMetropolisedSMCSampler, mocat/src/transport/smc.py:228-428)
 per temperature iteration, as mocat orders it (smc.py:73-99, 193-225):
   keys = split(key, n + 2); key = keys[-1]
-  resample with keys[-2] if ESS <= ess_threshold_resample * n   (gather of every particle field)
+  resample with keys[-2] if ESS <= ess_threshold_resample * n   (gather of values and momenta)
   move every particle at the current temperature: Underdamped.startup (re-evaluates potential and
       gradient, key split(keys[i], 3)[0]) then mcmc_steps Metropolis-corrected updates
       (fused iteration kernel; MALA when leapfrog_steps = 1)
-  next temperature by regula falsi on the ESS (FP64, one workgroup), reweight, ESS, log-normaliser,
+  next temperature by regula falsi on the ESS (FP64), reweight, ESS, log-normaliser,
       Robbins-Monro stepsize update from the weighted mean acceptance (RM variant)
 The iteration stops when the temperature reaches max_temperature.
 
@@ -36,6 +36,12 @@ _lib.register("mocat_smc_temper", [_P, _P, _lib.c_i64, _lib.c_f64, _lib.c_f64, _
                                    _lib.c_f64, _P, _P, _P])
 _lib.register("mocat_smc_temper_workspace_bytes", [_P])
 _lib.register("mocat_smc_temper_split", _lib.SIGNATURES["mocat_smc_temper"][:-1] + [_P, _lib.c_i64, _lib.c_i32, _P])
+_lib.register("mocat_smc_resample_workspace_bytes", [_lib.c_i64, _P])
+_lib.register("mocat_smc_resample", [_P, _lib.c_i64, _lib.c_i64, _lib.c_i32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
+                                     _lib.c_i64, _P])
+_lib.register("mocat_smc_move", [_P, _P, _P, _lib.c_i64, _lib.c_i64, _lib.c_i32, _lib.c_f32, _lib.c_i64] + [_P] * 11
+              + [_lib.c_i32, _lib.c_i32, _lib.c_f32, _P, _P] + [_lib.c_f64] * 7 + [_lib.c_i32, _lib.c_i32]
+              + [_lib.c_f64] * 3 + [_P, _P, _P, _lib.c_i64, _lib.c_i32, _P])
 TEMPER_POLLS = 1 << 22  # polls of one wait between the workgroups of the temperature search
 
 
@@ -106,37 +112,66 @@ class MetropolisedSMCSampler(TemperedSMCSampler):
         self.parameters.max_bisection_iter = int(max_bisection_iter)
 
     # -- device helpers -------------------------------------------------------------------------
+    def _temper_args(self, beta, ess, it):
+        """Arguments of the temperature step from ess on, and the workspace it exchanges partial sums in."""
+        p = self.parameters
+        adaptive = self.temperature_schedule is None
+        nb = 0.0 if adaptive else float(self.temperature_schedule[min(it, len(self.temperature_schedule) - 1)])
+        nbytes = _lib.c_i64(0)
+        _lib.call("mocat_smc_temper_workspace_bytes", _lib.ctypes.byref(nbytes))
+        return (float(ess), float(p.ess_threshold_retain), float(self.max_temperature), float(p.bisection_tol),
+                int(p.max_bisection_iter), int(adaptive), nb), nbytes.value
+
     def _temper(self, lw, lik, beta, ess, it, log_h, alpha_trace=None):
         p = self.parameters
         out = torch.empty(8, dtype=torch.float64, device=lw.device)
         lw_out = torch.empty_like(lw)
-        adaptive = self.temperature_schedule is None
-        nb = 0.0 if adaptive else float(self.temperature_schedule[min(it, len(self.temperature_schedule) - 1)])
         k_alpha = 0 if alpha_trace is None else int(alpha_trace.shape[0])
         rm = float(p.rm_stepsize) if (self.rm and alpha_trace is not None) else 0.0
         target = float(self.mcmc_sampler.tuning.target or 0.0)
-        nbytes = _lib.c_i64(0)
-        _lib.call("mocat_smc_temper_workspace_bytes", _lib.ctypes.byref(nbytes))
-        ws = torch.empty(nbytes.value, dtype=torch.uint8, device=lw.device)
-        _lib.call("mocat_smc_temper_split", _lib.ptr(lw), _lib.ptr(lik), int(lw.shape[0]), float(beta), float(ess),
-                  float(p.ess_threshold_retain), float(self.max_temperature), float(p.bisection_tol),
-                  int(p.max_bisection_iter), int(adaptive), nb, _lib.ptr(alpha_trace), k_alpha, float(log_h), rm,
-                  target, _lib.ptr(lw_out), _lib.ptr(out), _lib.ptr(ws), nbytes.value, TEMPER_POLLS,
-                  _lib.stream_handle())
+        args, nbytes = self._temper_args(beta, ess, it)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=lw.device)
+        _lib.call("mocat_smc_temper_split", _lib.ptr(lw), _lib.ptr(lik), int(lw.shape[0]), float(beta), *args,
+                  _lib.ptr(alpha_trace), k_alpha, float(log_h), rm, target, _lib.ptr(lw_out), _lib.ptr(out),
+                  _lib.ptr(ws), nbytes, TEMPER_POLLS, _lib.stream_handle())
         return lw_out, out.cpu().numpy()
 
-    def _resample(self, state, lw, key):
-        n = lw.shape[0]
-        if self.resampling == "categorical":
-            from .ssm.filtering import categorical
-            idx = categorical(key, lw, n)
+    def _resample(self, state, lw, key, resample, ws):
+        """The keys of one temperature and, if asked, the resampled particles: the evaluation that follows
+        replaces every field but value and momenta. Returns (log weights, move keys, next key)."""
+        n, d = state.value.shape
+        method = {"categorical": 2, "systematic": 0, "multinomial": 1}[self.resampling] if resample else -1
+        pkeys = torch.empty((n, 2), dtype=key.dtype, device=lw.device)
+        nkey = torch.empty(2, dtype=key.dtype, device=lw.device)
+        value, momenta = state.value, state.momenta
+        if resample:
+            if value.element_size() != 4:
+                raise TypeError("resampling handles 4-byte element types")
+            value, momenta = value.contiguous(), momenta.contiguous()
+            state.value, state.momenta, lw_in = torch.empty_like(value), torch.empty_like(momenta), lw
+            lw = torch.empty_like(lw)
+            ptrs = [_lib.ptr(t) for t in (lw_in, value, momenta, state.value, state.momenta, lw)]
         else:
-            from .ssm.filtering import resample_indices
-            idx = resample_indices(lw, key, self.resampling, log_weights=True)
-        for k in ("value", "grad_potential", "momenta", "potential", "prior_potential", "likelihood_potential",
-                  "alpha"):
-            setattr(state, k, gather_rows(getattr(state, k), idx))
-        return state, idx
+            ptrs = [None] * 6
+        _lib.call("mocat_smc_resample", _lib.ptr(key), n, d, method, *ptrs, _lib.ptr(pkeys), _lib.ptr(nkey),
+                  _lib.ptr(ws), int(ws.numel()), _lib.stream_handle())
+        return lw, pkeys, nkey
+
+    def _fused_moves(self, scenario, state, h, pkeys, beta, steps, alpha_trace, grads, stepsize, lw, ess, it, ws):
+        """forward_proposal's corrected Underdamped updates at `beta` and adapt, in one call. Returns the new log
+        weights and the step's results with the count of NaN values."""
+        p, n = self.parameters, int(lw.shape[0])
+        out = torch.empty(9, dtype=torch.float64, device=lw.device)
+        lw_out = torch.empty_like(lw)
+        args, nbytes = self._temper_args(beta, ess, it)
+        _lib.call("mocat_smc_move", *scenario.kernel_args(), n, _lib.ptr(grads[0]), _lib.ptr(grads[1]),
+                  _lib.ptr(state.value), _lib.ptr(state.momenta), _lib.ptr(state.grad_potential),
+                  _lib.ptr(state.potential), _lib.ptr(state.prior_potential), _lib.ptr(state.likelihood_potential),
+                  _lib.ptr(stepsize), _lib.ptr(state.alpha), _lib.ptr(pkeys), steps, int(p.leapfrog_steps),
+                  float(p.friction), _lib.ptr(alpha_trace), _lib.ptr(lw), float(beta), h, math.log(h), *args,
+                  float(p.rm_stepsize) if self.rm else 0.0, float(self.mcmc_sampler.tuning.target or 0.0),
+                  _lib.ptr(lw_out), _lib.ptr(out), _lib.ptr(ws), nbytes, TEMPER_POLLS, _lib.stream_handle())
+        return lw_out, out
 
     def _user_moves(self, scenario, state, stepsize, keys, beta, steps, alpha_trace):
         """forward_proposal's corrected Underdamped updates at temperature beta for a scenario without a
@@ -199,6 +234,10 @@ class MetropolisedSMCSampler(TemperedSMCSampler):
                                 "bisection_iters")}
         stacks = {k: [] for k in stack}
 
+        def snapshot():
+            for k in stack:
+                stacks[k].append((lw if k == "log_weight" else getattr(state, k)).clone())
+
         def record(alpha_mean, iters):
             hist["temperature"].append(beta)
             hist["ess"].append(ess)
@@ -206,58 +245,59 @@ class MetropolisedSMCSampler(TemperedSMCSampler):
             hist["stepsize"].append(h)
             hist["alpha_mean"].append(alpha_mean)
             hist["bisection_iters"].append(iters)
-            for k in stack:
-                stacks[k].append((lw if k == "log_weight" else getattr(state, k)).clone())
 
+        snapshot()
         record(1.0, 0)
         it = 0
-        if fused:
-            X, y, packed, nrows, d, prec, pprec = scenario.kernel_args()
         steps = int(p.mcmc_steps)
-        alpha_trace = torch.empty((steps, n), dtype=torch.float32, device=pp.device)
+        dev = pp.device
+        alpha_trace = torch.empty((steps, n), dtype=torch.float32, device=dev)
+        nbytes = _lib.c_i64(0)
+        _lib.call("mocat_smc_resample_workspace_bytes", n, _lib.ctypes.byref(nbytes))
+        ws = torch.empty(max(nbytes.value, self._temper_args(beta, ess, 0)[1]), dtype=torch.uint8, device=dev)
         while beta < self.max_temperature and it < self.max_iter:
             it += 1
-            keys_all = mr.split(key, n + 2)
-            key = keys_all[-1].contiguous()
-            if ess <= p.ess_threshold_resample * n:
-                state, _ = self._resample(state, lw, keys_all[-2].contiguous())
-                lw = torch.zeros(n, dtype=torch.float32, device=lw.device)
+            resample = ess <= p.ess_threshold_resample * n
+            lw, pkeys, key = self._resample(state, lw, key, resample, ws)
+            if resample:
                 ess = float(n)
             # forward_proposal: Underdamped.startup then mcmc_steps corrected updates at `beta`
-            pkeys = mr.split(keys_all[:n].contiguous(), 3)[:, 0].contiguous()
             pp, lp, gp, gl = evaluate(scenario, state.value, beta)
-            state.potential = pp + beta * lp
-            state.grad_potential = (gp + beta * gl).contiguous()
             state.prior_potential, state.likelihood_potential = pp, lp
-            stepsize = torch.full((n,), h, dtype=torch.float32, device=lw.device)
-            if not fused:
-                self._user_moves(scenario, state, stepsize, pkeys, beta, steps, alpha_trace)
-            else:
-                _lib.call("mocat_hmc_lr_iterate", X, y, packed, nrows, d, prec, pprec, float(beta), n,
-                          _lib.ptr(state.value), _lib.ptr(state.momenta), _lib.ptr(state.grad_potential),
-                          _lib.ptr(state.potential), _lib.ptr(state.prior_potential),
-                          _lib.ptr(state.likelihood_potential), _lib.ptr(stepsize), _lib.ptr(state.alpha),
-                          _lib.ptr(pkeys), 0, steps, int(p.leapfrog_steps), float(p.friction), 1, 0.0, 1.0, 2 / 3,
-                          math.inf, _P(0), _P(0), _lib.ptr(alpha_trace), _P(0), _P(0), _lib.stream_handle())
+            stepsize = torch.empty(n, dtype=torch.float32, device=dev)
             # adapt: next temperature, reweight, ESS, log-normaliser, RM stepsize
-            lw, out = self._temper(lw, state.likelihood_potential, beta, ess, it, math.log(h), alpha_trace)
-            beta_new = float(out[0])
+            if fused:
+                lw, out = self._fused_moves(scenario, state, h, pkeys, beta, steps, alpha_trace, (gp, gl), stepsize, lw,
+                                            ess, it, ws)
+            else:
+                state.potential = pp + beta * lp
+                state.grad_potential = (gp + beta * gl).contiguous()
+                self._user_moves(scenario, state, stepsize.fill_(h), pkeys, beta, steps, alpha_trace)
+                lw, out = self._temper(lw, state.likelihood_potential, beta, ess, it, math.log(h), alpha_trace)
+                state.potential = state.prior_potential + float(out[0]) * state.likelihood_potential
+            if steps > 0 and (not fused or "alpha" in stack):
+                state.alpha = alpha_trace.mean(0)
+            snapshot()
+            if fused:
+                out = out.cpu().numpy()
+                nan = np.float32(out.view(np.int64)[8]) / np.float32(state.value.numel()) > np.float32(0.1)
+            else:
+                nan = bool(torch.isnan(state.value).float().mean() > 0.1)
             lnc += float(out[2]) - float(out[3])
             ess = float(out[1])
             if self.rm:
                 h = math.exp(float(out[4]))
-            beta = beta_new
-            state.potential = state.prior_potential + beta * state.likelihood_potential
-            state.alpha = alpha_trace.mean(0) if steps > 0 else state.alpha
+            beta = float(out[0])
             record(float(out[5]), int(out[6]))
-            if bool(torch.isnan(state.value).float().mean() > 0.1):
+            if nan:
                 break
+        if fused and it > 0 and steps > 0:
+            state.alpha = alpha_trace.mean(0)
         torch.cuda.synchronize()
         elapsed = time.perf_counter() - t0
         chain = cdict()
         for k in stack:
             chain.__dict__[k] = torch.stack(stacks[k])
-        dev = lw.device
         for k, v in hist.items():
             chain.__dict__[k] = torch.tensor(v, dtype=torch.float64, device=dev)
         chain.final_state = state
