@@ -318,7 +318,7 @@ int mocat_smc_temper(const float* log_weight, const float* lik, int64_t n, doubl
                      double max_temperature, double tol, int max_iter, int adaptive, double next_beta,
                      const float* alpha, int k_alpha, double log_stepsize, double rm_stepsize, double target,
                      float* log_weight_out, double* out, hipStream_t stream);
-/* The same step with the particles shared by several workgroups from 12288 on. log_weight_out must not
+/* The same step with the particles shared by several workgroups from 4096 on. log_weight_out must not
  * be log_weight; workspace: mocat_smc_temper_workspace_bytes bytes, 8-byte aligned, contents arbitrary. The
  * workgroups wait for each other at most max_polls polls per evaluation (usually 1 << 22); if one gives
  * up, one workgroup does the step alone in the same call. */

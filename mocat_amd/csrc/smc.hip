@@ -18,9 +18,6 @@ using namespace mocat;
 
 namespace {
 
-constexpr int NT = 1024;
-constexpr int NW = NT / kWave;
-
 __global__ __launch_bounds__(256) void gather_kernel(const uint32_t* __restrict__ src, const int32_t* __restrict__ idx,
                                                      int64_t n_out, int64_t width, uint32_t* __restrict__ dst) {
   const int64_t total = n_out * width;
@@ -29,12 +26,6 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint32_t* __restrict_
     dst[e] = src[(int64_t)idx[j] * width + k];
   }
 }
-
-struct Smem {
-  double m[NW], s1[NW], s2[NW];
-  double bc[2];
-  int pass;
-};
 
 struct TemperArgs {
   const float* lw;        // [n] current (resampled) log weights
@@ -60,260 +51,347 @@ struct TemperArgs {
 // The particles of one workgroup: i = (k * G + g) * NT + t for workgroup g of G. The first kRegs per
 // thread are read once and kept in registers over all evaluations, any others are read again each time.
 constexpr int kRegs = 4;
+template <int NT, bool ALPHA>
 struct Share {
   int64_t n, stride, first;  // stride = G * NT
-  const float *lw, *lik;
+  const float *lw, *lik, *alpha;
+  int k_alpha;
   float rl[kRegs], rk[kRegs];
+  double ra[ALPHA ? kRegs : 1];  // mean acceptance probability of the moves
+  MOCAT_DEV Share(const TemperArgs& a)
+      : n(a.n), stride((int64_t)gridDim.x * NT), first((int64_t)blockIdx.x * NT + threadIdx.x), lw(a.lw), lik(a.lik),
+        alpha(a.alpha), k_alpha(a.alpha ? a.k_alpha : 0) {
+#pragma unroll
+    for (int k = 0; k < kRegs; ++k) {
+      const int64_t i = first + k * stride;
+      rl[k] = i < n ? lw[i] : 0.f;
+      rk[k] = i < n ? lik[i] : 0.f;
+      if constexpr (ALPHA) ra[k] = i < n ? mean_alpha(i) : 0.0;
+    }
+  }
+  MOCAT_DEV double mean_alpha(int64_t i) const {
+    double am = 0.0;
+    for (int j = 0; j < k_alpha; ++j) am += (double)alpha[(int64_t)j * n + i];
+    return k_alpha > 0 ? am / (double)k_alpha : 0.0;
+  }
   template <class F>
-  MOCAT_DEV void each(F f) const {
+  MOCAT_DEV void each(F f) const {  // f(i, log weight, likelihood potential)
 #pragma unroll
     for (int k = 0; k < kRegs; ++k) {
       const int64_t i = first + k * stride;
       if (i < n) f(i, rl[k], rk[k]);
     }
+#pragma unroll 4
     for (int64_t i = first + kRegs * stride; i < n; i += stride) f(i, lw[i], lik[i]);
   }
-};
-MOCAT_DEV Share share_of(const float* lw, const float* lik, int64_t n) {
-  Share s;
-  s.n = n;
-  s.stride = (int64_t)gridDim.x * NT;
-  s.first = (int64_t)blockIdx.x * NT + threadIdx.x;
-  s.lw = lw;
-  s.lik = lik;
+  // s += (e, e^2, with ALPHA e * mean acceptance), e = exp(lw - db * lik - ref)
+  MOCAT_DEV void sums(double db, double ref, double s[3]) const {
+    auto add = [&](float l, float k, double am) {
+      const double e = exp((double)l - db * (double)k - ref);
+      s[0] += e;
+      s[1] += e * e;
+      if constexpr (ALPHA) s[2] += e * am;
+    };
 #pragma unroll
-  for (int k = 0; k < kRegs; ++k) {
-    const int64_t i = s.first + k * s.stride;
-    s.rl[k] = i < n ? lw[i] : 0.f;
-    s.rk[k] = i < n ? lik[i] : 0.f;
+    for (int k = 0; k < kRegs; ++k)
+      if (first + k * stride < n) add(rl[k], rk[k], ALPHA ? ra[k] : 0.0);
+#pragma unroll 4
+    for (int64_t i = first + kRegs * stride; i < n; i += stride) add(lw[i], lik[i], ALPHA ? mean_alpha(i) : 0.0);
   }
-  return s;
-}
+};
 
 // Workgroups of a split evaluation, and what they exchange: two sets of slots used in turn, so that a
 // workgroup that is one exchange ahead never overwrites what another still reads, and the barrier's
 // arrival count and abort flag. A workgroup that polls max_polls times without seeing every arrival sets
 // the flag and leaves, as does every workgroup that sees it; temper_kernel<false> then does the work.
-constexpr int kMaxSplit = 32;
-static_assert(kMaxSplit <= kWave, "one wave combines the workgroups' slots");
+// Slots are written and read by agent-scope atomics, which pass the caches: no cache is written back or
+// dropped for them.
+constexpr int kSlots = 10;
+constexpr int kMaxSplit = 128;
 struct TemperWs {
-  double slot[2][kMaxSplit][4];
+  double slot[2][kMaxSplit][kSlots];
   uint32_t bar[2];
 };
 struct Exchange {
   TemperWs* ws;
   uint32_t max_polls, count;
 
-  // Publishes this workgroup's values (thread 0's), waits for all: true when every workgroup arrived.
-  MOCAT_DEV bool run(const double* v, int nv, bool wait, Smem& s) {
+  // Wave 0: publishes this workgroup's values (the same in every lane), waits for all of them.
+  template <int NV>
+  MOCAT_DEV bool run(const double (&v)[NV]) {
+    static_assert(NV <= kSlots, "a slot holds the values");
     const int par = count & 1;
     ++count;
+    int ok = 1;
     if (threadIdx.x == 0) {
-      for (int k = 0; k < nv; ++k) ws->slot[par][blockIdx.x][k] = v[k];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        __hip_atomic_store(&ws->slot[par][blockIdx.x][k], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the values have arrived before the count does
       __hip_atomic_fetch_add(&ws->bar[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      int ok = 1;
       const uint32_t target = count * gridDim.x;
-      for (uint32_t polls = 0; wait; ++polls) {
-        if (__hip_atomic_load(&ws->bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-          ok = 0;
-          break;
-        }
+      for (uint32_t polls = 0;; ++polls) {
         if (polls >= max_polls) {
           __hip_atomic_store(&ws->bar[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           ok = 0;
           break;
         }
         if (__hip_atomic_load(&ws->bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
-        __builtin_amdgcn_s_sleep(1);
+        if ((polls & 63u) == 63u && __hip_atomic_load(&ws->bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+          ok = 0;
+          break;
+        }
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      s.pass = ok;
+      asm volatile("" ::: "memory");
     }
-    __syncthreads();
-    const bool ok = s.pass != 0;
-    __syncthreads();
-    return ok;
+    return __shfl(ok, 0, kWave) != 0;
   }
-  MOCAT_DEV const double* slots(int g) const { return ws->slot[(count - 1) & 1][g]; }
+  MOCAT_DEV double get(int g, int k) const {
+    return __hip_atomic_load(&ws->slot[(count - 1) & 1][g][k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 };
 
-// (lse(w), lse(2w)) of w_i = lw_i - db * lik_i, FP64: the workgroup's maximum m and the sums of
-// exp(w_i - m) and its square (one exponential per element), partial sums combined in a fixed order (lanes by
-// butterfly, waves in index order, workgroups by butterfly after scaling to the common maximum), so that every
-// workgroup finds the same values and takes the same decisions. false: the exchange was given up.
+struct Eval {
+  double lse, lse2, am;  // lse(w), lse(2w), weighted mean acceptance
+};
+
 template <bool SPLIT>
-MOCAT_DEV bool lse_pair(const Share& sh, double db, Exchange& ex, Smem& s, double& lse, double& lse2) {
-  const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
-  double mx = -INFINITY;
-  int has_nan = 0;
-  sh.each([&](int64_t, float l, float k) {
-    const double v = (double)l - db * (double)k;
-    if (isnan(v)) has_nan = 1;
-    else mx = fmax(mx, v);
-  });
-  const bool nan_seen = __syncthreads_or(has_nan) != 0;
-  mx = wave_max(mx);
-  if (lane == 0) s.m[w] = mx;
-  __syncthreads();
-  double m = s.m[0];
-  for (int i = 1; i < NW; ++i) m = fmax(m, s.m[i]);
-  double s1 = 0.0, s2 = 0.0;
-  if (!nan_seen && m != -INFINITY)
+struct Temper {
+  static constexpr int NT = SPLIT ? 256 : 512, NW = NT / kWave;
+  using Particles = Share<NT, SPLIT>;
+  struct Smem {
+    double red[6][NW];
+    double mx[2][NW];
+    double bc[8];
+    int nan[2][NW];
+    int ok;
+  };
+
+  // w_i = lw_i - db * lik_i at db = 0 and db = db1 together, FP64: the maxima, then sums of exp(w_i - max).
+  // Partial sums are combined in a fixed order (lanes by butterfly, waves in index order, workgroups by lane and
+  // butterfly after scaling to the common maximum), so that every workgroup finds the same values and takes the
+  // same decisions. false: the exchange was given up.
+  static MOCAT_DEV bool ends(const Particles& sh, double db1, Exchange& ex, Smem& s, Eval& e0, Eval& e1) {
+    const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
+    const double db[2] = {0.0, db1};
+    double mx[2] = {-INFINITY, -INFINITY};
+    int bad[2] = {0, 0};
     sh.each([&](int64_t, float l, float k) {
-      const double e = exp((double)l - db * (double)k - m);
-      s1 += e;
-      s2 += e * e;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const double v = (double)l - db[q] * (double)k;
+        if (isnan(v)) bad[q] = 1;
+        else mx[q] = fmax(mx[q], v);
+      }
     });
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  if (lane == 0) {
-    s.s1[w] = s1;
-    s.s2[w] = s2;
-  }
-  __syncthreads();
-  double a1 = 0.0, a2 = 0.0;
-  for (int i = 0; i < NW; ++i) {
-    a1 += s.s1[i];
-    a2 += s.s2[i];
-  }
-  __syncthreads();  // every thread has read the partials before a later call rewrites them
-  bool bad = nan_seen;
-  if constexpr (SPLIT) {
-    const double v[4] = {m, a1, a2, nan_seen ? 1.0 : 0.0};
-    if (!ex.run(v, 4, true, s)) return false;
-    if (w == 0) {
-      const bool in = lane < (int)gridDim.x;
-      const double* o = ex.slots(in ? lane : 0);
-      const double mg = in ? o[0] : -INFINITY, ng = in ? o[3] : 0.0;
-      const double mm = wave_max(mg);
-      const double sc = in && mm != -INFINITY ? exp(mg - mm) : 0.0;
-      const double t1 = wave_sum(in ? o[1] * sc : 0.0), t2 = wave_sum(in ? o[2] * (sc * sc) : 0.0);
-      const double nn = wave_max(ng);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      mx[q] = wave_max(mx[q]);
+      const int any = __any(bad[q]);
       if (lane == 0) {
-        s.m[0] = mm;
-        s.s1[0] = t1;
-        s.s2[0] = t2;
-        s.bc[0] = nn;
+        s.mx[q][w] = mx[q];
+        s.nan[q][w] = any;
       }
     }
     __syncthreads();
-    m = s.m[0];
-    a1 = s.s1[0];
-    a2 = s.s2[0];
-    bad = s.bc[0] != 0.0;
+    double p[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      mx[q] = s.mx[q][0];
+      bad[q] = s.nan[q][0];
+      for (int i = 1; i < NW; ++i) {
+        mx[q] = fmax(mx[q], s.mx[q][i]);
+        bad[q] |= s.nan[q][i];
+      }
+      if (!bad[q] && mx[q] != -INFINITY) sh.sums(db[q], mx[q], p + 3 * q);
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      p[k] = wave_sum(p[k]);
+      if (lane == 0) s.red[k][w] = p[k];
+    }
     __syncthreads();
+    if (w == 0) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        p[k] = s.red[k][0];
+        for (int i = 1; i < NW; ++i) p[k] += s.red[k][i];
+      }
+      bool ok = true;
+      if constexpr (SPLIT) {
+        const double v[kSlots] = {mx[0], mx[1], bad[0] ? 1.0 : 0.0, bad[1] ? 1.0 : 0.0, p[0], p[1], p[2], p[3], p[4], p[5]};
+        ok = ex.run(v);
+        if (ok) {
+          const int G = (int)gridDim.x;
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            double m = -INFINITY, nn = 0.0;
+            for (int g = lane; g < G; g += kWave) {
+              m = fmax(m, ex.get(g, q));
+              nn = fmax(nn, ex.get(g, 2 + q));
+            }
+            mx[q] = wave_max(m);
+            bad[q] = wave_max(nn) != 0.0;
+            double a[3] = {0.0, 0.0, 0.0};
+            if (mx[q] != -INFINITY)
+              for (int g = lane; g < G; g += kWave) {
+                const double sc = exp(ex.get(g, q) - mx[q]);
+                a[0] += ex.get(g, 4 + 3 * q) * sc;
+                a[1] += ex.get(g, 5 + 3 * q) * (sc * sc);
+                a[2] += ex.get(g, 6 + 3 * q) * sc;
+              }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) p[3 * q + k] = wave_sum(a[k]);
+          }
+        }
+      }
+      if (lane == 0) {
+        s.ok = ok;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const double out = bad[q] ? NAN : -INFINITY;
+          const bool none = bad[q] || mx[q] == -INFINITY;
+          s.bc[3 * q] = none ? out : mx[q] + log(p[3 * q]);
+          s.bc[3 * q + 1] = none ? out : 2.0 * mx[q] + log(p[3 * q + 1]);
+          s.bc[3 * q + 2] = none ? NAN : p[3 * q + 2] / p[3 * q];
+        }
+      }
+    }
+    __syncthreads();
+    e0 = {s.bc[0], s.bc[1], s.bc[2]};
+    e1 = {s.bc[3], s.bc[4], s.bc[5]};
+    return s.ok != 0;
   }
-  if (bad || m == -INFINITY) {
-    lse = lse2 = bad ? NAN : -INFINITY;
-  } else {
-    lse = m + log(a1);
-    lse2 = 2.0 * m + log(a2);
-  }
-  return true;
-}
 
-// One evaluation is an FP64 exponential per particle and takes 10 us in one workgroup at 16384 particles, 132 us for
-// the whole search. SPLIT: a workgroup per 1024 particles (at most kMaxSplit), one exchange per evaluation;
-// the evaluations at b_t and at the chosen bound are those of the search.
-// Without SPLIT one workgroup; with a workspace only if the split search gave up.
+  // The same at one db, with the sums relative to `ref` in place of the maximum; bc: the three sums.
+  static MOCAT_DEV bool inner(const Particles& sh, double db, double ref, Exchange& ex, Smem& s, Eval& e) {
+    const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
+    double p[3] = {0.0, 0.0, 0.0};
+    sh.sums(db, ref, p);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      p[k] = wave_sum(p[k]);
+      if (lane == 0) s.red[k][w] = p[k];
+    }
+    __syncthreads();
+    if (w == 0) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        p[k] = s.red[k][0];
+        for (int i = 1; i < NW; ++i) p[k] += s.red[k][i];
+      }
+      bool ok = true;
+      if constexpr (SPLIT) {
+        ok = ex.run(p);
+        if (ok) {
+          double a[3] = {0.0, 0.0, 0.0};
+          for (int g = lane; g < (int)gridDim.x; g += kWave)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) a[k] += ex.get(g, k);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) p[k] = wave_sum(a[k]);
+        }
+      }
+      if (lane == 0) {
+        s.ok = ok;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s.bc[k] = p[k];
+      }
+    }
+    __syncthreads();
+    const double s1 = s.bc[0], s2 = s.bc[1];
+    e.lse = ref + log(s1);
+    e.lse2 = 2.0 * ref + log(s2);
+    e.am = s.bc[2] / s1;
+    return s.ok != 0;
+  }
+};
+
+// Sums below this may have lost terms to underflow: the evaluation is repeated relative to the maximum.
+constexpr double kTiny = -640.0;  // log; the smallest normal number is exp(-708)
+
+// One evaluation is an FP64 exponential per particle, and what surrounds it is latency: reductions, two barriers,
+// the exchange. So the bracket's ends are evaluated together; inside the bracket the sums are taken
+// relative to the chord through the ends' log-sum-exps (log-sum-exp is convex in the temperature, so no exponential
+// exceeds 1) instead of to a maximum found first; and the result's values are those of the evaluation that was
+// chosen.
+// SPLIT: a workgroup of 256 per 256 particles (at most kMaxSplit), one exchange per evaluation, which carries the
+// weighted acceptance along. Without SPLIT one workgroup of 512, which sums the acceptance at the end; with
+// a workspace only if the split search gave up.
 template <bool SPLIT>
-__global__ __launch_bounds__(NT) void temper_kernel(TemperArgs a, TemperWs* ws, uint32_t max_polls) {
-  __shared__ Smem s;
+__global__ __launch_bounds__(Temper<SPLIT>::NT) void temper_kernel(TemperArgs a, TemperWs* ws, uint32_t max_polls) {
+  using T = Temper<SPLIT>;
+  __shared__ typename T::Smem s;
   if constexpr (!SPLIT)
     if (ws && ws->bar[1] == 0u) return;
-  const int t = threadIdx.x;
-  const Share sh = share_of(a.lw, a.lik, a.n);
+  const typename T::Particles sh(a);
   Exchange ex{ws, max_polls, 0u};
   const double logthr = log(a.ess * a.retain);
-  double bnew, fmin_abs = 0.0, lse_prev, lse_new, lse2_new;
+  auto f = [&](const Eval& e) { return (2.0 * e.lse - e.lse2) - logthr; };
+  double bnew = a.next_beta, fmin_abs = 0.0;
   int iters = 0;
+  Eval lo, hi;
+  if (!T::ends(sh, (a.adaptive ? a.max_temperature : a.next_beta) - a.beta, ex, s, lo, hi)) return;
+  const double lse_prev = lo.lse;
+  Eval at = hi;
   if (a.adaptive) {
-    double b0 = a.beta, b1 = a.max_temperature, l0, m0, l1, m1;
-    if (!lse_pair<SPLIT>(sh, 0.0, ex, s, l0, m0)) return;
-    if (!lse_pair<SPLIT>(sh, b1 - a.beta, ex, s, l1, m1)) return;
-    double e0 = (2.0 * l0 - m0) - logthr, e1 = (2.0 * l1 - m1) - logthr;
-    lse_prev = l0;
-    const bool increasing = e1 > e0;
+    double b0 = a.beta, b1 = a.max_temperature;
+    double f0 = f(lo), f1 = f(hi);
+    const bool increasing = f1 > f0;
     while (true) {
-      const bool done = fmin(fabs(e0), fabs(e1)) < a.tol || iters >= a.max_iter || (e0 < 0 && e1 < 0) ||
-                        (e0 > 0 && e1 > 0) || isnan(e0) || isnan(e1);
+      const bool done = fmin(fabs(f0), fabs(f1)) < a.tol || iters >= a.max_iter || (f0 < 0 && f1 < 0) ||
+                        (f0 > 0 && f1 > 0) || isnan(f0) || isnan(f1);
       if (done) break;
-      const double np = b0 - e0 * (b1 - b0) / (e1 - e0);
-      double l, m;
-      if (!lse_pair<SPLIT>(sh, np - a.beta, ex, s, l, m)) return;
-      const double ne = (2.0 * l - m) - logthr;
+      const double np = b0 - f0 * (b1 - b0) / (f1 - f0);
+      const double ref = lo.lse + (hi.lse - lo.lse) * ((np - b0) / (b1 - b0));
+      Eval e;
+      if (!T::inner(sh, np - a.beta, ref, ex, s, e)) return;
+      if (!(e.lse2 - 2.0 * ref > kTiny)) {
+        Eval unused;
+        if (!T::ends(sh, np - a.beta, ex, s, unused, e)) return;
+      }
+      const double ne = f(e);
       const bool replace_upper = increasing ? ne > 0 : ne < 0;
       if (replace_upper) {
         b1 = np;
-        e1 = ne;
-        l1 = l;
-        m1 = m;
+        f1 = ne;
+        hi = e;
       } else {
         b0 = np;
-        e0 = ne;
-        l0 = l;
-        m0 = m;
+        f0 = ne;
+        lo = e;
       }
       ++iters;
     }
     // bounds[argmin |evals|] (first on ties)
-    const bool upper = fabs(e1) < fabs(e0);
+    const bool upper = fabs(f1) < fabs(f0);
     bnew = upper ? b1 : b0;
-    lse_new = upper ? l1 : l0;
-    lse2_new = upper ? m1 : m0;
-    fmin_abs = fmin(fabs(e0), fabs(e1));
-  } else {
-    bnew = a.next_beta;
-    double lse_prev2;
-    if (!lse_pair<SPLIT>(sh, 0.0, ex, s, lse_prev, lse_prev2)) return;
-    if (!lse_pair<SPLIT>(sh, bnew - a.beta, ex, s, lse_new, lse2_new)) return;
+    at = upper ? hi : lo;
+    fmin_abs = fmin(fabs(f0), fabs(f1));
   }
   const double db = bnew - a.beta;
   // weighted mean acceptance with weights exp(lw_new - max) (normalised)
   double amean = 0.0;
   if (a.alpha && a.k_alpha > 0) {
-    double num = 0.0, den = 0.0;
-    sh.each([&](int64_t i, float l, float k) {
-      const double wi = exp((double)l - db * (double)k - lse_new);
-      double am = 0.0;
-      for (int j = 0; j < a.k_alpha; ++j) am += (double)a.alpha[(int64_t)j * a.n + i];
-      am /= (double)a.k_alpha;
-      num += wi * am;
-      den += wi;
-    });
-    num = wave_sum(num);
-    den = wave_sum(den);
-    if ((t & (kWave - 1)) == 0) {
-      s.s1[t / kWave] = num;
-      s.s2[t / kWave] = den;
+    amean = at.am;
+    if constexpr (!SPLIT) {
+      double num = 0.0, den = 0.0;
+      sh.each([&](int64_t i, float l, float k) {
+        const double wi = exp((double)l - db * (double)k - at.lse);
+        num += wi * sh.mean_alpha(i);
+        den += wi;
+      });
+      num = block_sum(num, s.red[0]);
+      den = block_sum(den, s.red[1]);
+      amean = num / den;
     }
-    __syncthreads();
-    double N = 0.0, D = 0.0;
-    for (int i = 0; i < NW; ++i) {
-      N += s.s1[i];
-      D += s.s2[i];
-    }
-    __syncthreads();
-    if constexpr (SPLIT) {
-      const double v[2] = {N, D};
-      if (!ex.run(v, 2, blockIdx.x == 0, s)) return;
-      if (blockIdx.x == 0) {
-        N = D = 0.0;
-        for (int g = 0; g < (int)gridDim.x; ++g) {
-          N += ex.slots(g)[0];
-          D += ex.slots(g)[1];
-        }
-      }
-    }
-    amean = N / D;
   }
   // written last so that lw_out may alias lw: each thread its own particles
   sh.each([&](int64_t i, float l, float k) { a.lw_out[i] = (float)((double)l - db * (double)k); });
-  if (t == 0 && blockIdx.x == 0) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
     a.out[0] = bnew;
-    a.out[1] = exp(2.0 * lse_new - lse2_new);
-    a.out[2] = lse_new;
+    a.out[1] = exp(2.0 * at.lse - at.lse2);
+    a.out[2] = at.lse;
     a.out[3] = lse_prev;
     a.out[4] = a.rm_stepsize != 0.0 ? a.log_stepsize + a.rm_stepsize * (amean - a.target) : a.log_stepsize;
     a.out[5] = amean;
@@ -324,21 +402,21 @@ __global__ __launch_bounds__(NT) void temper_kernel(TemperArgs a, TemperWs* ws, 
 
 __global__ void temper_clear_kernel(TemperWs* ws) { ws->bar[threadIdx.x] = 0u; }
 
-// One workgroup / split, the whole step with 4 search iterations: 42 / 61 us at 4096 particles, 60 / 62 at 8192, 92 / 65 at
-// 16384, 274 / 76 at 65536, 6690 / 199 at 2^20 (an exchange costs about as much as 8 particles per thread).
-constexpr int64_t kSplitMin = 12288;
+// One workgroup / split, the whole step with 4 search iterations: 25 / 29 us at 2048 particles, 33 / 31 at 4096, 47 / 33 at
+// 8192, 74 / 34 at 16384, 233 / 44 at 65536. One workgroup of 1024 spilled registers and took 51 us at 4096.
+constexpr int64_t kSplitMin = 4096;
 
 // cleared: an earlier kernel on the stream has set ws->bar to zero.
 void launch_temper(const TemperArgs& a, TemperWs* ws, uint32_t max_polls, bool cleared, hipStream_t stream) {
   if (a.n < kSplitMin) {
-    hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, (TemperWs*)nullptr, 0u);
+    hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(Temper<false>::NT), 0, stream, a, (TemperWs*)nullptr, 0u);
     return;
   }
-  const int64_t want = (a.n + NT - 1) / NT;
+  const int64_t want = (a.n + Temper<true>::NT - 1) / Temper<true>::NT;
   const dim3 grid((unsigned)(want < kMaxSplit ? want : kMaxSplit));
   if (!cleared) hipLaunchKernelGGL(temper_clear_kernel, dim3(1), dim3(2), 0, stream, ws);
-  hipLaunchKernelGGL((temper_kernel<true>), grid, dim3(NT), 0, stream, a, ws, max_polls);
-  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, ws, 0u);
+  hipLaunchKernelGGL((temper_kernel<true>), grid, dim3(Temper<true>::NT), 0, stream, a, ws, max_polls);
+  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(Temper<false>::NT), 0, stream, a, ws, 0u);
 }
 
 unsigned blocks_for(int64_t total) {
@@ -441,7 +519,7 @@ int mocat_smc_temper(const float* log_weight, const float* lik, int64_t n, doubl
   if (!log_weight || !lik || !log_weight_out || !out || n <= 0 || max_iter < 0 || k_alpha < 0) return MOCAT_ERR_ARG;
   TemperArgs a{log_weight, lik, n, beta, ess, retain, max_temperature, tol, max_iter, adaptive, next_beta,
                alpha, k_alpha, log_stepsize, rm_stepsize, target, log_weight_out, out};
-  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(NT), 0, stream, a, (TemperWs*)nullptr, 0u);
+  hipLaunchKernelGGL((temper_kernel<false>), dim3(1), dim3(Temper<false>::NT), 0, stream, a, (TemperWs*)nullptr, 0u);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }

@@ -32,7 +32,7 @@ def _temper(lw, lik, beta, retain, alpha, polls, schedule=None):
 
 
 # around the split, a last workgroup of one particle, more workgroups' worth than the limit, more than the registers hold
-@pytest.mark.parametrize("n", [1, 12287, 12288, 12289, 32 * 1024 + 1, 4 * 32 * 1024 + 777])
+@pytest.mark.parametrize("n", [1, 513, 4095, 4096, 4097, 12289, 32 * 1024 + 1, 4 * 32 * 1024 + 777])
 @pytest.mark.parametrize("polls", [1 << 22, 0])  # 0: every workgroup gives up at its first wait
 @pytest.mark.parametrize("retain,schedule", [(0.5, None), (0.2, None), (0.5, 0.3)])
 def test_temper_split(n, polls, retain, schedule):
@@ -71,6 +71,26 @@ def test_temper_split_non_finite(bad, want):
     new, out = _temper(lw, np.zeros(n, np.float32), 0.1, 0.5, np.ones((1, n), np.float32), 1 << 22, 0.3)
     assert np.isnan(out[2]) if want == "nan" else out[2] == -np.inf
     np.testing.assert_array_equal(new, lw)
+
+
+@pytest.mark.parametrize("n", [4, 700, 16384])
+@pytest.mark.parametrize("scale", [1.0, 3000.0])  # the larger one underflows against the chord inside the bracket
+def test_temper_wide_bracket(n, scale):
+    rng = np.random.default_rng(n)
+    lik = (scale * rng.gamma(2.0, size=n)).astype(np.float32)
+    lik[0] = 0.0
+    new, out = _temper(np.zeros(n, np.float32), lik, 0.0, 0.6, np.ones((1, n), np.float32), 1 << 22)
+    b = out[0]
+    v = -b * lik.astype(np.float64)
+    f = 2 * _lse(v) - _lse(2 * v) - math.log(0.6 * n)
+    end = -lik.astype(np.float64)
+    if 2 * _lse(end) - _lse(2 * end) > math.log(0.6 * n):  # no root: the ESS at 1 is still above the target
+        f0 = math.log(1 / 0.6)
+        assert b == (1.0 if abs(f) < f0 else 0.0)
+    else:
+        assert 0.0 < b < 1.0 and abs(f) < 1e-5 + 1e-10
+    np.testing.assert_allclose(out[1], math.exp(2 * _lse(v) - _lse(2 * v)), rtol=1e-9)
+    np.testing.assert_allclose(out[5], 1.0, rtol=1e-12)
 
 
 @pytest.mark.parametrize("n", [4096, 4097, 8192, 8193, 3 * 4096 + 1, 65 * 4096 + 5])
