@@ -954,6 +954,224 @@ __global__ __launch_bounds__(NT) void hmc_lr_kernel(HmcArgs h) {
   }
 }
 
+// The iteration for a diagonal Gaussian: LPC lanes per chain, lane q of them with the columns GK q .. GK q + GK - 1 of
+// position, momentum and gradient in registers, so that an iteration has neither LDS state nor global traffic (a tile of
+// 32 chains in LDS as hmc_lr_kernel keeps took about 25 barriers per iteration: 70 us for 5 moves of 16384 chains
+// at d = 20, here 30 us; 219 and 97 us at d = 100). What is left is the vector ALU: threefry and the normals, which the lanes of a chain share
+// by blocks of two words and pass on through LDS. Sums over columns keep hmc_lr_kernel's order: the likelihood
+// one column after the other, the squared norms by the butterfly of a wave that holds column k in lane k.
+constexpr int GK = 8;
+
+// The product alone, never contracted into the sum that takes it.
+MOCAT_DEV float product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+template <int LPC>
+MOCAT_DEV float gauss_sqnorm(const float (&v)[GK], int q) {
+  float a[GK];
+#pragma unroll
+  for (int j = 0; j < GK; ++j) {
+    if constexpr (LPC == 16) {  // columns k and k + 64 are one lane's
+      const float o = __shfl_xor(v[j], 8, kWave);
+      const float lo = (q & 8) ? o : v[j], hi = (q & 8) ? v[j] : o;
+      a[j] = fmaf(hi, hi, product(lo, lo));
+    } else {
+      a[j] = product(v[j], v[j]);
+    }
+  }
+#pragma unroll
+  for (int o = (LPC == 16 ? 8 : LPC) / 2; o > 0; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < GK; ++j) a[j] += __shfl_xor(a[j], o, kWave);
+#pragma unroll
+  for (int o = GK / 2; o > 0; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < o; ++j) a[j] += a[j + o];
+  return a[0];
+}
+
+// Orders a wave's own LDS writes and reads: a chain's lanes are of one wave.
+MOCAT_DEV void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Words 0 and 1 of `S` words of key k, each lane of a pair computing one of their two threefry blocks.
+template <int LPC>
+MOCAT_DEV Key pair_words(Key k, uint32_t S, int q) {
+  if constexpr (LPC == 1) {
+    return Key{bits_at(k, S, 0), bits_at(k, S, 1)};
+  } else {
+    const uint32_t w = bits_at(k, S, (uint32_t)(q & 1)), o = __shfl_xor(w, 1, kWave);
+    return (q & 1) ? Key{o, w} : Key{w, o};
+  }
+}
+
+// split(k, 2): four words from two blocks.
+template <int LPC>
+MOCAT_DEV void pair_split(Key k, int q, Key& first, Key& second) {
+  if constexpr (LPC == 1) {
+    first = split_at(k, 2, 0);
+    second = split_at(k, 2, 1);
+  } else {
+    uint32_t a, b;
+    bits_pair(k, 4u, (uint32_t)(q & 1), a, b);
+    const uint32_t oa = __shfl_xor(a, 1, kWave), ob = __shfl_xor(b, 1, kWave);
+    first = (q & 1) ? Key{oa, a} : Key{a, oa};
+    second = (q & 1) ? Key{ob, b} : Key{b, ob};
+  }
+}
+
+template <int LPC>
+__global__ __launch_bounds__(256) void hmc_gauss_kernel(HmcArgs h) {
+  constexpr int NC = 256 / LPC;
+  __shared__ float normals[NC][GK * LPC + 1];
+  const int t = threadIdx.x, q = t % LPC, c = t / LPC, k0 = q * GK, first = (t & (kWave - 1)) - q;
+  const int d = h.lr.d;
+  const int64_t chain = (int64_t)blockIdx.x * NC + c;
+  const bool live = chain < h.C;
+  const float prec = h.lr.prior_prec, temp = h.lr.temperature;
+  float th[GK], p[GK], g[GK], mu[GK], lam[GK];
+#pragma unroll
+  for (int j = 0; j < GK; ++j) {
+    const bool v = k0 + j < d;
+    mu[j] = v ? h.lr.X[k0 + j] : 0.f;
+    lam[j] = v ? h.lr.y[k0 + j] : 0.f;
+    th[j] = v && live ? h.theta[chain * d + k0 + j] : 0.f;
+    p[j] = v && live ? h.mom[chain * d + k0 + j] : 0.f;
+    g[j] = v && live ? h.grad[chain * d + k0 + j] : 0.f;
+  }
+  float pot = live ? h.pot[chain] : 0.f, prior = live ? h.prior[chain] : 0.f, lik = live ? h.lik[chain] : 0.f;
+  float step = live ? h.step[chain] : 1.f, alpha = live ? h.alpha[chain] : 0.f;
+  Key key = live ? Key{h.keys[2 * chain], h.keys[2 * chain + 1]} : Key{0u, 0u};
+  const uint32_t hd = (uint32_t)(d + 1) >> 1, L1 = (uint32_t)h.leapfrog_steps + 1u;
+  for (int it = 0; it < h.n_iter; ++it) {
+    const int64_t iter = h.iter0 + it + 1;
+    // ---- always: p <- -p ; (key, sub) = split(key) ; OU refresh (standard_mcmc.py:107-123); then the
+    // proposal's keys = split(key, L+1), key = keys[0] (standard_mcmc.py:129-131)
+    Key nk, sk;
+    pair_split<LPC>(key, q, nk, sk);
+    key = pair_words<LPC>(nk, 2u * L1, q);
+    float u = 0.f;
+    if (h.correction > 0) {  // the acceptance's uniform (metropolis.py:60-61)
+      Key uk;
+      pair_split<LPC>(key, q, nk, uk);
+      key = nk;
+      u = uniform_from_bits(bits_at(uk, 1, 0), 0.f, 1.f);
+    }
+#pragma unroll
+    for (int j = 0; j < GK / 2; ++j) {
+      const uint32_t i = (uint32_t)(j * LPC + q);
+      if (j * LPC >= (int)hd) break;
+      uint32_t w0, w1;
+      bits_pair(sk, (uint32_t)d, i, w0, w1);
+      const float z0 = normal_from_bits(w0), z1 = normal_from_bits(w1);
+      if (i < hd) normals[c][i] = z0;
+      if (i + hd < (uint32_t)d) normals[c][i + hd] = z1;
+    }
+    wave_sync();
+    const float decay = __expf(-h.friction * step);
+    const float noise = sqrtf(1.f - __expf(-2.f * h.friction * step));
+    float p0[GK], th0[GK], g0[GK];  // the pre-proposal state, for a rejection
+#pragma unroll
+    for (int j = 0; j < GK; ++j) {
+      if (k0 + j < d) p[j] = fmaf(noise, normals[c][k0 + j], -(p[j] * decay));
+      p0[j] = p[j];
+      th0[j] = th[j];
+      g0[j] = g[j];
+    }
+    wave_sync();  // the normals have been read
+    const float kin0 = fmaf(0.5f, gauss_sqnorm<LPC>(p, q), 0.5f * (float)d * kLog2Pi);
+    // ---- leapfrog (utils.py:117-146)
+    float pot1 = pot, prior1 = prior, lik1 = lik;
+    for (int s = 0; s < h.leapfrog_steps; ++s) {
+      float cost[GK];
+#pragma unroll
+      for (int j = 0; j < GK; ++j) {
+        p[j] = fmaf(-(step / 2.f), g[j], p[j]);
+        th[j] = k0 + j < d ? fmaf(step, p[j], th[j]) : 0.f;
+        const float df = th[j] - mu[j];
+        cost[j] = product(product(product(0.5f, lam[j]), df), df);
+        g[j] = fmaf(prec, th[j], temp * product(lam[j], df));
+        p[j] = fmaf(-(step / 2.f), g[j], p[j]);
+      }
+      if (s == h.leapfrog_steps - 1) {
+        lik1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < LPC; ++r) {
+          float acc = lik1;
+#pragma unroll
+          for (int j = 0; j < GK; ++j) acc += cost[j];  // columns from d on: 0
+          lik1 = LPC == 1 ? acc : __shfl(acc, first + r, kWave);
+        }
+        // prec == 0: improper flat prior, potential 0 (mocat's default uniform prior, core.py:183-189)
+        prior1 = prec > 0.f ? fmaf(0.5f * prec, gauss_sqnorm<LPC>(th, q), 0.5f * (float)d * (kLog2Pi - logf(prec))) : 0.f;
+        pot1 = fmaf(temp, lik1, prior1);
+      }
+    }
+    // ---- correction (metropolis.py:48-70, 118-161)
+    const float kin1 = fmaf(0.5f, gauss_sqnorm<LPC>(p, q), 0.5f * (float)d * kLog2Pi);  // |-p|^2 == |p|^2
+    float a = 1.f;
+    bool acc = true;
+    if (h.correction > 0) {
+      a = fminf(1.f, __expf(-pot1 + pot - kin1 + kin0));
+      a = isnan(a) ? 0.f : a;
+      acc = u < a;
+    }
+    alpha = a;
+    if (acc) {
+      pot = pot1;
+      prior = prior1;
+      lik = lik1;
+    }
+    if (h.correction == 2 && (double)iter <= h.adapt_cut_off) {
+      const float rm = h.rm_scale * powf((float)iter, -h.rm_neg_exponent);
+      step = expf(logf(step) + rm * (a - h.target));
+    }
+    // accepted: momenta <- -p'; rejected: the pre-proposal state
+#pragma unroll
+    for (int j = 0; j < GK; ++j) {
+      p[j] = acc ? -p[j] : p0[j];
+      th[j] = acc ? th[j] : th0[j];
+      g[j] = acc ? g[j] : g0[j];
+    }
+    if (live) {
+      const int64_t o = (int64_t)it * h.C + chain;
+      if (h.tr_value || h.tr_mom)
+#pragma unroll
+        for (int j = 0; j < GK; ++j)
+          if (k0 + j < d) {
+            if (h.tr_value) h.tr_value[o * d + k0 + j] = th[j];
+            if (h.tr_mom) h.tr_mom[o * d + k0 + j] = p[j];
+          }
+      if (q == 0) {
+        if (h.tr_pot) h.tr_pot[o] = pot;
+        if (h.tr_alpha) h.tr_alpha[o] = alpha;
+        if (h.tr_step) h.tr_step[o] = step;
+      }
+    }
+  }
+  if (!live) return;
+#pragma unroll
+  for (int j = 0; j < GK; ++j)
+    if (k0 + j < d) {
+      h.theta[chain * d + k0 + j] = th[j];
+      h.mom[chain * d + k0 + j] = p[j];
+      h.grad[chain * d + k0 + j] = g[j];
+    }
+  if (q == 0) {
+    h.pot[chain] = pot;
+    h.prior[chain] = prior;
+    h.lik[chain] = lik;
+    h.step[chain] = step;
+    h.alpha[chain] = alpha;
+    h.keys[2 * chain] = key.a;
+    h.keys[2 * chain + 1] = key.b;
+  }
+}
+
 constexpr int kThreads = 512;
 
 // The same iteration as hmc_lr_kernel for the bf16x3 engine, with the tile state in
@@ -1205,6 +1423,27 @@ int dispatch_hmc(const HmcArgs& h, hipStream_t st) {
   return MOCAT_OK;
 }
 
+template <int LPC>
+void launch_gauss(const HmcArgs& h, hipStream_t st) {
+  const int64_t per = 256 / LPC;
+  hipLaunchKernelGGL((hmc_gauss_kernel<LPC>), dim3((unsigned)((h.C + per - 1) / per)), dim3(256), 0, st, h);
+}
+
+int dispatch_hmc_gauss(const HmcArgs& h, hipStream_t st) {
+  if (h.lr.d <= GK)
+    launch_gauss<1>(h, st);
+  else if (h.lr.d <= 2 * GK)
+    launch_gauss<2>(h, st);
+  else if (h.lr.d <= 4 * GK)
+    launch_gauss<4>(h, st);
+  else if (h.lr.d <= 8 * GK)
+    launch_gauss<8>(h, st);
+  else
+    launch_gauss<16>(h, st);
+  MOCAT_LAUNCH_CHECK();
+  return MOCAT_OK;
+}
+
 // bf16x3: two waves per SIMD at d <= 64; at d <= 128 one wave per SIMD (the operand registers of a
 // 128-column block, and the LDS of eight waves' partial gradients, do not fit two waves). Two tiles of
 // chains per workgroup from kTwoTiles chains (a workgroup for each of 256 CUs): X 20000 x 100, 65536 positions,
@@ -1315,7 +1554,7 @@ int mocat_hmc_lr_iterate(const float* X, const float* y, const void* packed, int
             C, theta, momenta, grad, potential, prior_pot, lik_pot, stepsize, alpha, keys, iter0, n_iter,
             leapfrog_steps, friction, correction, target, rm_scale, rm_neg_exponent, adapt_cut_off,
             trace_value, trace_potential, trace_alpha, trace_stepsize, trace_momenta};
-  if (precision == 2) return dispatch_hmc<GaussEngine>(h, stream);
+  if (precision == 2) return dispatch_hmc_gauss(h, stream);
   if (precision == 3) return dispatch_hmc<Fp64Engine>(h, stream);
   return precision == 0 ? dispatch_hmc<Fp32Engine>(h, stream) : dispatch_hmc_bf16(h, stream);
 }
