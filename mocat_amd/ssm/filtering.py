@@ -423,21 +423,25 @@ def _large_flags(ns, Ts, large_n, resampling=None):
     one workgroup / chunked, with the call's 0.5 ms on the host):
     * 128 with categorical resampling, whose n^2 draws per step need the whole GPU (64 particles: 0.90 /
       0.93 ms, 128: 1.66 / 0.97, 1024: 29.6 / 1.29);
-    * without filters of 4096 or more, 1024 (one filter of 512 particles 0.68 / 0.67 ms, of 1024 0.96 /
-      0.68, of 4095 2.85 / 0.81; 64 of 4095 3.24 / 1.78), unless those of 1024 to 4095 particles fill the
-      GPU with a workgroup each (256 of 4095: 4.93 / 5.21), then 4096;
-    * beside filters of 4096 or more, whose launches they join: 1024, or every filter when those below 1024
-      add fewer chunks than are there (a second stream for a few small filters may share a hardware queue
-      with the first, and the two then run one after the other)."""
+    * without filters of 4096 or more, one path for all, as a second stream for some of the filters may share a
+      hardware queue with the first and the two then run one after the other: the launches per step from a
+      largest filter of 512 particles on, unless there are so many filters that a workgroup for each fills
+      the GPU: from 128 of them on below 1024 particles, from 256 on above (100 steps of stochastic volatility,
+      one workgroup / launches: one filter of 377 particles 1.07 / 1.10 ms, of 614 1.32 / 1.11; 64 of at most 990 1.85 /
+      1.52, 256 3.2 / 3.6; 128 of 200 to 2975 over 200 steps 6.6 / 3.5, 300 of 207 to 4087 6.0 / 5.7, 500 7.9 / 8.9);
+    * beside filters of 4096 or more, whose launches they join: every filter when those below 1024 are no more
+      than 128 or than the chunks that are there (102 filters with one of 30000: 4.1 / 3.6), else those
+      from 1024 on (251 with one of 5000: 4.7 / 5.3)."""
     if large_n is None:
         ns = [int(n) for n in ns]
         chunks = sum(-(-n // 1024) for n in ns if n >= 4096)
         if resampling == "categorical":
             large_n = 128
         elif chunks:
-            large_n = 1 if sum(n < 1024 for n in ns) <= chunks else 1024
+            large_n = 1 if sum(n < 1024 for n in ns) <= max(chunks, 128) else 1024
         else:
-            large_n = 1024 if sum(n for n in ns if n >= 1024) <= 2 ** 19 else 4096
+            most = max(ns, default=0)
+            large_n = 1 if most >= 512 and len(ns) < (128 if most < 1024 else 256) else 4096
     return [int(n) >= int(large_n) for n in ns]
 
 
