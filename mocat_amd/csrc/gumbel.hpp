@@ -117,31 +117,37 @@ MOCAT_DEV uint32_t gumbel_argmax(Key k, uint32_t n, int lane, uint32_t part, uin
 }
 
 // Rows m and m + rows / 2 of gumbel(k, (rows, n)) for an even number of rows: element m n + j and the same
-// element of the other row are the two words of one threefry block.
+// element of the other row are the two words of one threefry block. Wave `part` of `parts` takes every
+// parts-th 64 columns.
+template <bool PRUNE, class Logit>
+MOCAT_DEV void gumbel_pair_draw(Key k, uint32_t S, uint32_t off, uint32_t n, int lane, uint32_t part, uint32_t parts,
+                                Logit logit, GumbelRow<PRUNE>& a, GumbelRow<PRUNE>& b) {
+  const uint32_t h = S >> 1;
+  for (uint64_t j0 = (uint64_t)part * kWave; j0 < n; j0 += (uint64_t)parts * kWave) {
+    const bool act = j0 + (uint64_t)lane < n;
+    const uint32_t j = (uint32_t)j0 + (uint32_t)lane, jc = act ? j : n - 1u;
+    uint32_t w0 = off + jc, w1 = off + jc + h;
+    threefry2x32(k.a, k.b, w0, w1);
+    const float l = logit(jc);
+    a.offer(act, j, w0, l, logit);
+    b.offer(act, j, w1, l, logit);
+  }
+  a.first_max();
+  b.first_max();
+}
+
 template <class Logit>
 MOCAT_DEV void gumbel_row_pair(Key k, uint32_t S, uint32_t off, uint32_t n, int lane, Logit logit, uint32_t& first,
                                uint32_t& second) {
-  const uint32_t h = S >> 1;
-  auto draw = [&](auto& a, auto& b) {
-    for (uint64_t j0 = 0; j0 < n; j0 += kWave) {
-      const bool act = j0 + (uint64_t)lane < n;
-      const uint32_t j = (uint32_t)j0 + (uint32_t)lane, jc = act ? j : n - 1u;
-      uint32_t w0 = off + jc, w1 = off + jc + h;
-      threefry2x32(k.a, k.b, w0, w1);
-      const float l = logit(jc);
-      a.offer(act, j, w0, l, logit);
-      b.offer(act, j, w1, l, logit);
-    }
-  };
   GumbelRow<true> a, b;
-  draw(a, b);
-  first = a.first_max();
-  second = b.first_max();
+  gumbel_pair_draw(k, S, off, n, lane, 0u, 1u, logit, a, b);
+  first = a.bi;
+  second = b.bi;
   if (!a.met_nan() && !b.met_nan()) return;
   GumbelRow<false> fa, fb;
-  draw(fa, fb);
-  first = fa.first_max();
-  second = fb.first_max();
+  gumbel_pair_draw(k, S, off, n, lane, 0u, 1u, logit, fa, fb);
+  first = fa.bi;
+  second = fb.bi;
 }
 
 // Rows of random.categorical(key, lw, (rows,)) by one wave: unit u of the ceil(rows / 2) that cover them
@@ -162,6 +168,68 @@ MOCAT_DEV void categorical_unit(const float* __restrict__ lw, uint32_t n, uint32
   for (uint32_t r = 2u * u; r < 2u * u + 2u && r < rows; ++r) {
     const uint32_t a = gumbel_row(key, S, r * n, n, lane, logit);
     if (lane == 0) idx[r] = (int32_t)a;
+  }
+}
+
+// The same unit by the P waves of a workgroup of P waves: each takes every P-th 64 columns of both rows, and the parts'
+// first maxima are compared in order. A row that met a NaN is drawn again by one wave. Every thread of the
+// workgroup calls it. For calls with too few rows for a wave each (dispatch: categorical_parts).
+template <int P>
+struct CategoricalParts {
+  float best[2][P];
+  uint32_t bi[2][P];
+  int nan[P];
+};
+template <int P>
+MOCAT_DEV void categorical_unit_parts(const float* __restrict__ lw, uint32_t n, uint32_t rows, Key key, uint32_t u,
+                                      CategoricalParts<P>& s, int32_t* __restrict__ idx) {
+  const uint32_t S = n * rows, lane = threadIdx.x & (kWave - 1), part = threadIdx.x / kWave;
+  auto logit = [&](uint32_t j) { return lw[j]; };
+  const bool pair = (rows & 1u) == 0u;
+  GumbelRow<true> a, b;
+  if (pair) {
+    gumbel_pair_draw(key, S, u * n, n, (int)lane, part, P, logit, a, b);
+  } else {
+    auto draw = [&](GumbelRow<true>& row, uint32_t off) {
+      for (uint64_t j0 = (uint64_t)part * kWave; j0 < n; j0 += (uint64_t)P * kWave) {
+        const bool act = j0 + (uint64_t)lane < n;
+        const uint32_t j = (uint32_t)j0 + lane, jc = act ? j : n - 1u;
+        row.offer(act, j, bits_at(key, S, off + jc), logit(jc), logit);
+      }
+      row.first_max();
+    };
+    draw(a, 2u * u * n);
+    if (2u * u + 1u < rows) draw(b, (2u * u + 1u) * n);
+  }
+  const bool nan = a.met_nan() || b.met_nan();
+  if (lane == 0) {
+    s.best[0][part] = a.best;
+    s.bi[0][part] = a.bi;
+    s.best[1][part] = b.best;
+    s.bi[1][part] = b.bi;
+    s.nan[part] = nan;
+  }
+  __syncthreads();
+  if (part != 0) return;
+  bool any = false;
+  for (int q = 0; q < P; ++q) any |= s.nan[q] != 0;
+  if (any) {
+    categorical_unit(lw, n, rows, key, u, (int)lane, idx);
+    return;
+  }
+  if (lane < 2) {
+    const uint32_t row = pair ? u + lane * (rows / 2) : 2u * u + lane;
+    float best = -INFINITY;
+    uint32_t bi = kNoIndex;
+    for (int q = 0; q < P; ++q) {
+      const float ob = s.best[lane][q];
+      const uint32_t oi = s.bi[lane][q];
+      if (oi != kNoIndex && (bi == kNoIndex || ob > best || (ob == best && oi < bi))) {
+        best = ob;
+        bi = oi;
+      }
+    }
+    if (row < rows) idx[row] = (int32_t)bi;
   }
 }
 

@@ -2048,20 +2048,46 @@ MOCAT_DEV LseAcc lf_small_combine(const LfArgs& a, const LfDesc& F, int64_t t, d
   return LseAcc{bad ? NAN : M, s1, s2};
 }
 
-// Categorical resampling: the rows of chunk c's kSmallCatBlocks blocks, one unit of two rows per wave; the
-// decision comes from the same combined accumulators as the step kernel's.
-constexpr int kSmallCatBlocks = SCH / 2 / LW;
-__global__ __launch_bounds__(LT) void lf_small_cat_kernel(LfArgs a, int64_t t) {
+// Categorical resampling: the rows of chunk c, in units of two rows; a wave per unit, or (P > 1) a workgroup of P
+// waves. The decision comes from the same combined accumulators as the step kernel's.
+template <int P>
+__global__ __launch_bounds__(P == 1 ? LT : P * kWave) void lf_small_cat_kernel(LfArgs a, int64_t t) {
   const LfDesc& F = a.cdesc[blockIdx.x];
   if (t >= F.T) return;
-  const int64_t u = (blockIdx.x - F.chunk0) * (SCH / 2) + blockIdx.y * LW + threadIdx.x / kWave;
+  constexpr int NU = P == 1 ? LW : 1;  // units of a workgroup
+  const int64_t u = (blockIdx.x - F.chunk0) * (SCH / 2) + blockIdx.y * NU + (P == 1 ? threadIdx.x / kWave : 0);
   if (u >= (F.n + 1) / 2) return;
   double g[3];
   const LseAcc r = lf_small_combine<false>(a, F, t, g);
   if (!lf_stats(r, F.n, a.ess_threshold).res) return;
   const StepKey& sk = a.skeys[F.key_slot + t];
-  categorical_unit(lf_lw_prev(a, t) + F.state_offset, (uint32_t)F.n, (uint32_t)F.n, Key{sk.k[0], sk.k[1]}, (uint32_t)u,
-                   threadIdx.x & (kWave - 1), a.anc + F.chunk0 * SCH);
+  const float* lw = lf_lw_prev(a, t) + F.state_offset;
+  const Key key{sk.k[0], sk.k[1]};
+  int32_t* anc = a.anc + F.chunk0 * SCH;
+  if constexpr (P == 1) {
+    categorical_unit(lw, (uint32_t)F.n, (uint32_t)F.n, key, (uint32_t)u, threadIdx.x & (kWave - 1), anc);
+  } else {
+    __shared__ CategoricalParts<P> parts;
+    categorical_unit_parts<P>(lw, (uint32_t)F.n, (uint32_t)F.n, key, (uint32_t)u, parts, anc);
+  }
+}
+
+template <int P>
+void launch_small_cat_p(const LfArgs& a, unsigned chunks, int64_t t, hipStream_t q) {
+  hipLaunchKernelGGL((lf_small_cat_kernel<P>), dim3(chunks, P == 1 ? SCH / 2 / LW : SCH / 2), dim3(P == 1 ? LT : P * kWave),
+                     0, q, a, t);
+}
+// Waves per unit: a filter of 1024 particles has 512 units for 1024 SIMDs, and splitting the rows over 4 waves takes 4 of its
+// 23 us per step; from 16 chunks on there are waves enough and the split only adds exact draws. 50 steps with 1 / 2 / 4 / 8
+// waves: one filter of 1024 1.39 / 1.28 / 1.19 / 1.20 ms, of 3001 3.11 / 2.72 / 2.39 / 2.60, of 4096 2.44 / 2.32 / 2.43 / 2.80;
+// 4 of 512 1.28 / 1.22 / 1.25 / 1.39, 16 of 512 1.59 / 1.73 / 2.05 / 2.67.
+void launch_small_cat(const LfArgs& a, unsigned chunks, int64_t t, hipStream_t q) {
+  if (chunks <= 6)
+    launch_small_cat_p<4>(a, chunks, t, q);
+  else if (chunks <= 16)
+    launch_small_cat_p<2>(a, chunks, t, q);
+  else
+    launch_small_cat_p<1>(a, chunks, t, q);
 }
 
 template <class Model, int D, int DY, bool GRAD>
@@ -2510,7 +2536,7 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
       hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD, 1>), chunks, blk, 0, q, a);
       for (int64_t t = 1; t <= max_T; ++t) {
         if (a.resampling == 2 && t < max_T)
-          hipLaunchKernelGGL(lf_small_cat_kernel, dim3(grid(t).x, kSmallCatBlocks), blk, 0, q, a, t);
+          launch_small_cat(a, grid(t).x, t, q);
         hipLaunchKernelGGL((lf_small_kernel<Model, D, DY, GRAD>), grid(t - 1), blk, 0, q, a, t);
       }
       hipLaunchKernelGGL((lf_finish_kernel<D, 1>), chunks, blk, 0, q, a);
