@@ -475,8 +475,7 @@ MOCAT_DEV uint64_t block_exclusive_scan(uint64_t v, BlockScratch& s, uint64_t& t
 MOCAT_DEV int quant_shift(float wmax, int64_t n) {
   int e;
   frexpf(wmax, &e);  // wmax = f * 2^e, f in [0.5, 1)
-  int bits_n = 0;
-  while ((1ll << bits_n) <= n) ++bits_n;
+  const int bits_n = n > 0 ? 64 - __clzll(n) : 0;
   const int qb = 52 - bits_n;
   return qb - e;
 }
@@ -942,17 +941,17 @@ __global__ __launch_bounds__(256) void categorical_kernel(const float* __restric
 
 // ---------------------------------------------------------------- large filters: grid-wide launches per step
 // One workgroup per filter leaves a large filter running long after the others have finished. Filters
-// flagged kPfLarge instead advance one time step per sequence of three launches over 1024-particle
+// flagged kPfLarge instead advance one time step per sequence of two launches over 1024-particle
 // chunks (all flagged filters batched in every launch):
 //   lf_prep    per chunk: combine the chunk accumulators of step t-1 in chunk order (every chunk of
 //              the filter alike; its first chunk writes the log-likelihood, ESS and filter state),
-//              the resampling decision and weight shift for step t, and the chunk's sum of quantised
-//              weights (resampling steps only);
-//   lf_csum    per chunk: the chunk's threefry blocks of the step's split(key, n) (every step), then
-//              offset = sum of the earlier chunks' totals, plus an inclusive block scan;
+//              the resampling decision and weight shift for step t, the chunk's threefry blocks of the
+//              step's split(key, n) (every step), and on resampling steps the inclusive sums of the
+//              chunk's quantised weights and their total;
+//   lf_offsets (filters beyond kOffsets chunks only) the inclusive sums of the totals;
 //   lf_cat     categorical resampling only: the Gumbel-max rows, one wave per two of them;
-//   lf_step    per chunk: ancestor (binary search in the exact prefix sums, or lf_cat's), then
-//              propagate, weight, outputs and the chunk accumulators of step t+1.
+//   lf_step    per chunk: ancestor (binary search in the exact prefix sums, a chunk's own sums plus
+//              the totals before it; or lf_cat's), then propagate, weight, outputs and the chunk accumulators of step t+1.
 // The weights are shifted by float(lse) and quantised with the shift of the largest weight exactly as
 // in pf_kernel, so for the same log-weights and key the ancestors are the same.
 //
@@ -966,6 +965,7 @@ constexpr int CH = LT * PPT;     // particles per chunk (one workgroup)
 constexpr int SCH = LT;          // particles per chunk of the one-launch step: one per thread
 constexpr int kSmallMax = 4096;  // largest filter of the one-launch step
 constexpr int SG = 256;          // prefix-sum search granularity (chunk ends staged in LDS)
+constexpr int kOffsets = 1024;     // chunk totals summed in LDS by each step workgroup (8 KB)
 constexpr int kSearchWin = 2048;   // prefix sums of a block's ancestor chunks staged in LDS (16 KB)
 constexpr int kChunkEnds = 4096;   // SG-block end sums staged in LDS (filters up to 2^20 particles);
                                    // dynamic LDS sized by the launch's largest filter (at most 32 KB)
@@ -1025,21 +1025,24 @@ struct LfArgs {
   double* part_s1;   // [n_chunks]
   double* part_s2;   // [n_chunks]
   double* part_g;    // [n_chunks][3] tangent sums (GRAD)
-  uint64_t* ctot;    // [n_chunks] quantised weight totals
+  uint64_t* ctot;    // [n_chunks] quantised weight totals of the chunks (csum and cends: sums within a chunk)
   LfState* st;       // [n_large]
-  uint64_t* cends;   // [n_chunks * CH / SG] prefix sums at the SG-block ends, per filter from chunk0 * CH / SG
-  int64_t* bounds;   // [n_chunks] systematic: ancestor of each chunk's first target
+  uint64_t* cends;   // [n_chunks * CH / SG] sums at the SG-block ends, per filter from chunk0 * CH / SG
+  uint64_t* coff;    // [n_chunks] filters of more than kOffsets chunks: inclusive sums of ctot
   StepKey* skeys;    // [key_slot + t] per filter
   uint32_t* bar;     // persistent kernel: [0] barrier arrivals, [1] abort flag (zeroed by the init launch)
   int32_t* anc;      // [n_chunks * CH] categorical: the step's ancestors, per filter from chunk0 * CH
   uint32_t* pkeys;   // [n_chunks * CH * 2] the step's split(step key, n), flat, per filter from chunk0 * CH * 2;
                      // null for the optimal proposal (its noise is not drawn from per-particle keys)
+  int big;           // some filter has more than kOffsets chunks and is resampled from prefix sums
 };
 
 struct LfScratch {
   float fm[LW];
   double d1[LW], d2[LW], g[LW][3];
   uint64_t u[LW];
+  float shift_m;  // lf_prep: the weight shift, the quantisation shift and the resampling decision
+  int shift_q, res;
 };
 
 // chunk-level reductions in a fixed order (wave butterflies, then waves in order)
@@ -1394,18 +1397,56 @@ MOCAT_DEV void lf_prep_chunk(const LfArgs& a, int64_t t, int64_t c, LfScratch& s
   const LfDesc F = a.cdesc[c];
   if (t - 1 >= F.T) return;
   const int64_t n = F.n, nchunk = (n + CH - 1) / CH;
-  // the chunk's weights for its quantised total are loaded first: they do not depend on the combine
-  const bool want_tot = t < F.T && a.resampling != 2;
+  const int64_t local = c - F.chunk0, i0 = local * CH + (int64_t)threadIdx.x * PPT;  // PPT consecutive particles
+  // the chunk's weights for its quantised sums are loaded first: they do not depend on the combine
+  const bool want_sums = t < F.T && a.resampling != 2;
   const float* lwp = lf_lw_prev(a, t) + F.state_offset;
   float lwv[PPT];
 #pragma unroll
-  for (int pk = 0; pk < PPT; ++pk) {
-    const int64_t i = (c - F.chunk0) * CH + pk * LT + threadIdx.x;
-    lwv[pk] = (want_tot && i < n) ? lwp[i] : 0.f;
+  for (int pk = 0; pk < PPT; ++pk) lwv[pk] = (want_sums && i0 + pk < n) ? lwp[i0 + pk] : 0.f;
+  if (a.pkeys && t < F.T) {
+    // split(step key, n) for the step kernel, one threefry block per key: block j of split's counter
+    // pairs (j, n + j) yields words j and n + j of the flat key array (key i = words 2i, 2i + 1), so
+    // the chunk's blocks j in [local * CH, (local + 1) * CH) fill words in both halves
+    const StepKey& skv = a.skeys[F.key_slot + t];
+    const uint32_t un = (uint32_t)n, ka = skv.k[0], kb = skv.k[1];
+    uint32_t* PK = a.pkeys + F.chunk0 * (2 * CH);
+#pragma unroll
+    for (int pk = 0; pk < PPT; ++pk) {
+      const int64_t j = local * CH + pk * LT + threadIdx.x;
+      if (j < n) {
+        uint32_t x0 = (uint32_t)j, x1 = (uint32_t)j + un;
+        threefry2x32(ka, kb, x0, x1);
+        PK[j] = x0;
+        PK[j + n] = x1;
+      }
+    }
   }
   double gsum[3] = {0.0, 0.0, 0.0};  // tangent sums relative to the filter's maximum (GRAD)
+  // One wave finds the statistics for the workgroup (FP64 logarithms and exponentials: 17.7 us per step with every wave
+  // doing so in a ragged batch of 256 filters, 16.7 with one); neighbouring chunks take different waves, that is SIMDs.
+  const bool stats = threadIdx.x / kWave == (unsigned)(c & (LW - 1));
   LseAcc r;
-  {
+  if (nchunk <= kWave) {
+    if (stats) {
+      // one partial per lane
+      const int k = threadIdx.x & (kWave - 1);
+      const bool have = k < nchunk;
+      const int64_t cc = F.chunk0 + (have ? k : 0);
+      const float pm = have ? a.part_m[cc] : -INFINITY;
+      double s1 = have ? a.part_s1[cc] : 0.0, s2 = have ? a.part_s2[cc] : 0.0;
+      if constexpr (GRAD)
+        for (int q = 0; q < 3; ++q) gsum[q] = have ? a.part_g[cc * 3 + q] : 0.0;
+      const bool anybad = __any(isnan(pm)) != 0;
+      const float M = wave_max(isnan(pm) ? -INFINITY : pm);
+      const double f = pm > -INFINITY ? exp((double)pm - (double)M) : 0.0;  // NaN and -inf partials add nothing
+      s1 = wave_sum(f > 0.0 ? s1 * f : 0.0);
+      s2 = wave_sum(f > 0.0 ? s2 * f * f : 0.0);
+      if constexpr (GRAD)
+        for (int q = 0; q < 3; ++q) gsum[q] = wave_sum(f > 0.0 ? gsum[q] * f : 0.0);
+      r = LseAcc{anybad ? NAN : M, s1, s2};
+    }
+  } else {
     // two passes over the chunk partials: their maximum, then the rescaled sums (one exponential each;
     // the tangent sums of a chunk are relative to its maximum, like its weight sums). Filters of at
     // most LT chunks (one partial per thread) load each partial once, in the first pass.
@@ -1494,20 +1535,38 @@ MOCAT_DEV void lf_prep_chunk(const LfArgs& a, int64_t t, int64_t c, LfScratch& s
     }
     r = LseAcc{anybad ? NAN : M, r1, r2};
   }
-  const LfStats v = lf_stats(r, n, a.ess_threshold);
-  if (c == F.chunk0 && threadIdx.x == 0) lf_update_state<GRAD>(a, F, t - 1, v, r, gsum);
-  const bool res = v.res != 0;
-  const float m = v.m;
-  const int shift = v.shift;
-  if (t >= F.T || !res || a.resampling == 2) return;
-  uint64_t q = 0;
+  if (stats) {
+    const LfStats v = lf_stats(r, n, a.ess_threshold);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+      s.shift_m = v.m;
+      s.shift_q = v.shift;
+      s.res = v.res;
+      if (c == F.chunk0) lf_update_state<GRAD>(a, F, t - 1, v, r, gsum);
+    }
+  }
+  if (!want_sums) return;
+  __syncthreads();
+  if (s.res == 0) return;
+  const float m = s.shift_m;
+  const int shift = s.shift_q;
+  // the chunk's own inclusive sums, their values at the SG-block ends, and its total
+  uint64_t q[PPT], own = 0;
 #pragma unroll
   for (int pk = 0; pk < PPT; ++pk) {
-    const int64_t i = (c - F.chunk0) * CH + pk * LT + threadIdx.x;
-    if (i < n) q += quantise(__expf(lwv[pk] - m), shift);
+    q[pk] = i0 + pk < n ? quantise(__expf(lwv[pk] - m), shift) : 0ull;
+    own += q[pk];
   }
-  const uint64_t tot = lf_block_sum(q, s);
-  if (threadIdx.x == 0) a.ctot[c] = tot;
+  uint64_t run = lf_block_inclusive_scan(own, s) - own;
+#pragma unroll
+  for (int pk = 0; pk < PPT; ++pk) {
+    run += q[pk];
+    const int64_t i = i0 + pk;
+    if (i < n) {
+      a.csum[F.state_offset + i] = run;
+      if ((i + 1) % SG == 0 || i == n - 1) a.cends[F.chunk0 * (CH / SG) + i / SG] = run;
+    }
+  }
+  if (threadIdx.x == LT - 1) a.ctot[c] = run;
 }
 
 template <bool GRAD>
@@ -1516,107 +1575,25 @@ __global__ __launch_bounds__(LT) void lf_prep_kernel(LfArgs a, int64_t t) {
   lf_prep_chunk<GRAD>(a, t, blockIdx.x, s);
 }
 
-// cs: CH entries of LDS (this chunk's prefix sums, for the systematic boundary searches)
-MOCAT_DEV void lf_csum_chunk(const LfArgs& a, int64_t t, int64_t c, LfScratch& s, uint64_t* cs) {
-  const LfDesc F = a.cdesc[c];
-  const int fi = F.slot;
-  if (t >= F.T) return;
-  const int64_t local = c - F.chunk0;
+// Filters of more than kOffsets chunks: the inclusive sums of the chunk totals, which lf_step_chunk forms in LDS for
+// smaller ones. One workgroup per filter.
+MOCAT_DEV void lf_offsets_filter(const LfArgs& a, int64_t t, int64_t f, LfScratch& s) {
+  const LfDesc F = a.desc[f];
   const int64_t nchunk = (F.n + CH - 1) / CH;
-  // loads that do not depend on each other are issued first: the filter state, the chunk's weights and
-  // (one per thread, for filters of at most LT chunks) the chunk totals; the weights and totals are
-  // used on resampling steps only
-  const LfState st = a.st[fi];
-  const bool sums = a.resampling != 2;
-  const int64_t i0 = local * CH + (int64_t)threadIdx.x * PPT;  // thread tid owns PPT consecutive particles
-  const float* lw = lf_lw_prev(a, t) + F.state_offset;
-  float lwv[PPT];
-#pragma unroll
-  for (int pk = 0; pk < PPT; ++pk) lwv[pk] = (sums && i0 + pk < F.n) ? lw[i0 + pk] : 0.f;
-  const bool one = nchunk <= LT;
-  const uint64_t tot1 = (sums && one && threadIdx.x < nchunk) ? a.ctot[F.chunk0 + threadIdx.x] : 0ull;
-  if (a.pkeys) {
-    // split(step key, n) for the step kernel, one threefry block per key: block j of split's counter
-    // pairs (j, n + j) yields words j and n + j of the flat key array (key i = words 2i, 2i + 1), so
-    // the chunk's blocks j in [local * CH, (local + 1) * CH) fill words in both halves
-    const StepKey skv = a.skeys[F.key_slot + t];
-    const uint32_t un = (uint32_t)F.n;
-    uint32_t* PK = a.pkeys + F.chunk0 * (2 * CH);
-#pragma unroll
-    for (int pk = 0; pk < PPT; ++pk) {
-      const int64_t j = local * CH + pk * LT + threadIdx.x;
-      if (j < F.n) {
-        uint32_t x0 = (uint32_t)j, x1 = (uint32_t)j + un;
-        threefry2x32(skv.k[0], skv.k[1], x0, x1);
-        PK[j] = x0;
-        PK[j + F.n] = x1;
-      }
-    }
-  }
-  if (!st.res || !sums) return;
-  uint64_t off = 0, wsum = 0;
-  if (one) {
-    wsum = tot1;
-    off = threadIdx.x < local ? tot1 : 0ull;
-  } else {
-    for (int64_t k = threadIdx.x; k < nchunk; k += LT) {
-      const uint64_t v = a.ctot[F.chunk0 + k];
-      wsum += v;
-      if (k < local) off += v;
-    }
-  }
-  off = lf_block_sum(off, s);
-  wsum = lf_block_sum(wsum, s);
-  const float su = a.skeys[F.key_slot + t].su;  // the step's systematic uniform (init launch)
-  uint64_t q[PPT], own = 0;
-#pragma unroll
-  for (int pk = 0; pk < PPT; ++pk) {
-    q[pk] = i0 + pk < F.n ? quantise(__expf(lwv[pk] - st.m), st.shift) : 0ull;
-    own += q[pk];
-  }
-  uint64_t run = off + lf_block_inclusive_scan(own, s) - own;
-#pragma unroll
-  for (int pk = 0; pk < PPT; ++pk) {
-    run += q[pk];
-    const int64_t i = i0 + pk;
-    cs[threadIdx.x * PPT + pk] = run;
-    if (i < F.n) {
-      a.csum[F.state_offset + i] = run;
-      // the SG-block end sums, contiguous per filter, for the step kernel's first search level
-      if ((i + 1) % SG == 0 || i == F.n - 1) a.cends[F.chunk0 * (CH / SG) + i / SG] = run;
-    }
-  }
-  if (a.resampling != 0) return;
-  // Systematic targets floor((j + u) W / n) rise with j, so chunk b's ancestors lie between the
-  // ancestors of its first target and of the next chunk's first target. The chunk whose sums hold a
-  // boundary target (earlier sums <= target < its last sum; the last chunk also takes targets at or
-  // beyond the total, clamped to n - 1 as in the search) finds its ancestor in LDS and records it.
-  __syncthreads();
-  const int64_t count = (F.n - local * CH) < CH ? (F.n - local * CH) : CH;
-  const uint64_t chunk_hi = cs[count - 1];
-  const bool last = local == nchunk - 1;
-  const double sstep = (double)wsum / (double)F.n;
-  for (int64_t b = threadIdx.x; b < nchunk; b += LT) {
-    const uint64_t tg = target_floor(((double)(b * CH) + (double)su) * sstep);
-    if (tg < off || (!last && tg >= chunk_hi)) continue;
-    int64_t lo = 0, len = count;
-    while (len > 0) {
-      const int64_t h = len >> 1;
-      if (cs[lo + h] <= tg) {
-        lo += h + 1;
-        len -= h + 1;
-      } else {
-        len = h;
-      }
-    }
-    a.bounds[F.chunk0 + b] = local * CH + (lo < count ? lo : count - 1);
+  if (t >= F.T || nchunk <= kOffsets || a.resampling == 2 || !a.st[F.slot].res) return;
+  uint64_t base = 0;
+  for (int64_t k0 = 0; k0 < nchunk; k0 += LT) {
+    const int64_t k = k0 + threadIdx.x;
+    const uint64_t incl = lf_block_inclusive_scan(k < nchunk ? a.ctot[F.chunk0 + k] : 0ull, s);
+    if (k < nchunk) a.coff[F.chunk0 + k] = base + incl;
+    __syncthreads();
+    for (int w = 0; w < LW; ++w) base += s.u[w];  // the waves' totals
   }
 }
 
-__global__ __launch_bounds__(LT) void lf_csum_kernel(LfArgs a, int64_t t) {
+__global__ __launch_bounds__(LT) void lf_offsets_kernel(LfArgs a, int64_t t) {
   __shared__ LfScratch s;
-  __shared__ uint64_t cs[CH];
-  lf_csum_chunk(a, t, blockIdx.x, s, cs);
+  lf_offsets_filter(a, t, blockIdx.x, s);
 }
 
 // Categorical resampling of step t: the Gumbel-max rows of chunk c, block `sub` of its kCatBlocks taking
@@ -1691,7 +1668,6 @@ MOCAT_DEV void upper_bound_lockstep(Get v, const int64_t* b, const int64_t* m, c
   for (int q = 0; q < P; ++q) out[q] = lo[q];
 }
 
-// win: kSearchWin entries of LDS; cend: cend_slots entries (staged by the multinomial search only)
 // For P targets that do not decrease with p (a thread's consecutive systematic targets): out[p] = the
 // first k in [b, e) with v(k) > tg[p] (v non-decreasing), or e; inactive targets (the chunk's tail, all
 // after the active ones) return the previous result. The first target takes a binary search; each
@@ -1724,9 +1700,10 @@ MOCAT_DEV void upper_bound_rising(Get v, int64_t b, int64_t e, const uint64_t* t
   }
 }
 
+// win: kSearchWin entries of LDS, off: kOffsets, cend: cend_slots (staged by the multinomial search only)
 template <class Model, int D, int DY, bool GRAD>
 MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t c, LfScratch& s, Model& model,
-                             uint64_t* win, uint64_t* cend) {
+                             uint64_t* win, uint64_t* cend, uint64_t* off) {
   const LfDesc F = a.cdesc[c];
   const int fi = F.slot;
   if (t >= F.T) return;
@@ -1756,30 +1733,34 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
   // thread searches for its PPT particles in lockstep (independent LDS or global reads overlap).
   // (res and the method are per filter: the branches are uniform over the workgroup.)
   const uint64_t* C = a.csum + F.state_offset;
-  const int64_t nsg = (n + SG - 1) / SG;
-  // systematic: the chunk's ancestor window comes from the prefix-sum pass (bounds); multinomial
-  // targets are unordered and take the two-level search over the staged block-end sums
-  const bool window = res && a.resampling == 0;
-  const bool two_level = res && a.resampling == 1 && nsg <= cend_slots;
-  bool staged = false;
-  int64_t lo = 0, whi = n - 1;
-  if (window) {
-    const int64_t cl = c - F.chunk0, nchunk = (n + CH - 1) / CH;
-    const int64_t b0 = a.bounds[c], b1 = cl + 1 < nchunk ? a.bounds[c + 1] : n - 1;
-    lo = b0 < 0 ? 0 : (b0 > n - 1 ? n - 1 : b0);
-    whi = b1 < lo ? lo : (b1 > n - 1 ? n - 1 : b1);
-  }
-  const double W = (res && a.resampling != 2) ? (double)C[n - 1] : 0.0;
-  const double sstep = W / (double)n;
-  // the chunk-end sums go first: their loads are in flight while thread 0 derives the step key
+  const int64_t nsg = (n + SG - 1) / SG, nchunk = (n + CH - 1) / CH;
+  const bool sums = res && a.resampling != 2;
+  const bool window = sums && a.resampling == 0;
+  const bool two_level = sums && a.resampling == 1 && nsg <= cend_slots;
   const uint64_t* CE = a.cends + F.chunk0 * (CH / SG);
-  if (two_level) stage_lds<8>(cend, nsg, [&](int64_t k) { return CE[k]; });
+  // the sums of C and CE are within a chunk: the totals of the chunks before it are added on reading. Every
+  // workgroup sums the totals itself (a launch for it, with the sums made global there, took 14 of 66 us per step at 2^20).
+  // Up to kWave of them are scanned by each wave in registers.
+  const bool in_wave = nchunk <= kWave, in_lds = nchunk <= kOffsets;
+  const int lane = tid & (kWave - 1);
+  const uint64_t* G = a.coff + F.chunk0;
+  uint64_t tot[kOffsets / LT], incl = 0;
+  const int64_t per = (nchunk + LT - 1) / LT;  // consecutive totals of a thread
+  if (sums && in_wave) {
+    incl = lane < nchunk ? a.ctot[F.chunk0 + lane] : 0ull;
+  } else if (sums && in_lds) {
+#pragma unroll
+    for (int u = 0; u < kOffsets / LT; ++u) {
+      const int64_t k = tid * per + u;
+      tot[u] = u < per && k < nchunk ? a.ctot[F.chunk0 + k] : 0ull;
+    }
+  }
   // the step key, the optimal proposal's first split key and the systematic uniform (init launch)
   const StepKey skv = a.skeys[F.key_slot + t];
   const uint32_t sk[4] = {skv.k[0], skv.k[1], skv.k[2], skv.k[3]};
   const float su = skv.su;
   load_shared_params(model, a.params + F.param_offset);
-  // the particles' split keys (lf_csum) are loaded before the ancestor search, which they do not need
+  // the particles' split keys (lf_prep) are loaded before the ancestor search, which they do not need
   const uint32_t* PK = a.pkeys + F.chunk0 * (2 * CH);
   uint2 kwp[PPT];
 #pragma unroll
@@ -1787,13 +1768,74 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
     const int64_t i = pidx(pk);
     kwp[pk] = (!Model::kOptimal && i < n) ? *reinterpret_cast<const uint2*>(PK + 2 * i) : make_uint2(0u, 0u);
   }
+  if (sums && in_wave) {
+    incl = wave_inclusive_scan(incl);
+    if (tid < nchunk) off[tid] = incl;
+  } else if (sums && in_lds) {
+    uint64_t own = 0;
+#pragma unroll
+    for (int u = 0; u < kOffsets / LT; ++u) own += tot[u];
+    uint64_t run = lf_block_inclusive_scan(own, s) - own;
+#pragma unroll
+    for (int u = 0; u < kOffsets / LT; ++u) {
+      const int64_t k = tid * per + u;
+      run += tot[u];
+      if (u < per && k < nchunk) off[k] = run;
+    }
+  }
   __syncthreads();
+  auto through = [&](int64_t k) -> uint64_t { return in_lds ? off[k] : G[k]; };  // the sum through chunk k
+  auto before = [&](int64_t k) -> uint64_t { return k > 0 ? through(k - 1) : 0ull; };
+  auto sum_at = [&](int64_t i) -> uint64_t { return C[i] + before(i / CH); };
+  const double W = sums ? (double)through(nchunk - 1) : 0.0;
+  const double sstep = W / (double)n;
   const Key ik{sk[0], sk[1]};
   auto cend_at = [&](int64_t k) { return cend[k]; };
-  if (window && whi - lo + 1 <= kSearchWin) {
-    stage_lds<8>(win, whi - lo + 1, [&](int64_t k) { return C[lo + k]; });
+  bool staged = false;
+  int64_t lo = 0, whi = n - 1;
+  if (two_level) {
+    stage_lds<8>(cend, nsg, [&](int64_t k) { return CE[k] + before(k / (CH / SG)); });
     __syncthreads();
-    staged = true;
+  }
+  if (window) {
+    // systematic targets floor((j + u) W / n) rise with j: this chunk's ancestors lie between those of its first and last
+    // target, whose chunks and SG-blocks bound the window (the last block takes targets at or beyond the total)
+    const int64_t jl = base + CH < n ? base + CH - 1 : n - 1;
+    const uint64_t tga = target_floor(((double)base + (double)su) * sstep);
+    const uint64_t tgb = target_floor(((double)jl + (double)su) * sstep);
+    // the first chunk whose sum exceeds the target: as many as do not
+    const uint64_t tw[2] = {tga, tgb};
+    int64_t kc[2] = {0, 0};
+    if (in_lds) {
+      for (int64_t k0 = 0; k0 < nchunk; k0 += kWave) {
+        const bool in = k0 + lane < nchunk;
+        const uint64_t v = in_wave ? incl : (in ? off[k0 + lane] : 0ull);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) kc[q] += __popcll(__ballot(in && v <= tw[q]));
+      }
+    } else {
+      const int64_t zero[2] = {0, 0}, all[2] = {nchunk, nchunk};
+      const bool both[2] = {true, true};
+      upper_bound_lockstep<2>(through, zero, all, tw, both, kc);
+    }
+    int64_t blk[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int64_t k = kc[q] < nchunk ? kc[q] : nchunk - 1, b0 = k * (CH / SG);
+      const int64_t nb = nsg - b0 < CH / SG ? nsg - b0 : CH / SG;
+      const uint64_t rel = tw[q] - before(k);
+      int64_t b = 0;
+#pragma unroll
+      for (int j = 0; j < CH / SG - 1; ++j) b += (j + 1 < nb && CE[b0 + j] <= rel) ? 1 : 0;
+      blk[q] = b0 + b;
+    }
+    lo = blk[0] * SG;
+    whi = ((blk[1] + 1) * SG < n ? (blk[1] + 1) * SG : n) - 1;
+    if (whi - lo + 1 <= kSearchWin) {
+      stage_lds<8>(win, whi - lo + 1, [&](int64_t k) { return sum_at(lo + k); });
+      staged = true;
+    }
+    __syncthreads();
   }
 
   // ancestors of the thread's PPT particles
@@ -1824,7 +1866,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
         if (staged)
           upper_bound_rising<PPT>([&](int64_t k) { return win[k - lo]; }, lo, whi + 1, tg, live, p);
         else
-          upper_bound_rising<PPT>([&](int64_t k) { return C[k]; }, lo, whi + 1, tg, live, p);
+          upper_bound_rising<PPT>(sum_at, lo, whi + 1, tg, live, p);
       } else {
         int64_t b[PPT], m[PPT];
 #pragma unroll
@@ -1835,7 +1877,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
         if (staged)
           upper_bound_lockstep<PPT>([&](int64_t k) { return win[k - lo]; }, b, m, tg, live, p);
         else
-          upper_bound_lockstep<PPT>([&](int64_t k) { return C[k]; }, b, m, tg, live, p);
+          upper_bound_lockstep<PPT>(sum_at, b, m, tg, live, p);
       }
 #pragma unroll
       for (int pk = 0; pk < PPT; ++pk)
@@ -1861,7 +1903,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
       if (staged)
         upper_bound_lockstep<PPT>([&](int64_t k) { return win[k - lo]; }, b, m, tg, in, p);
       else
-        upper_bound_lockstep<PPT>([&](int64_t k) { return C[k]; }, b, m, tg, in, p);
+        upper_bound_lockstep<PPT>(sum_at, b, m, tg, in, p);
 #pragma unroll
       for (int pk = 0; pk < PPT; ++pk)
         if (live[pk]) srcs[pk] = in[pk] ? p[pk] : n - 1;
@@ -1872,7 +1914,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
         zero[pk] = 0;
         all[pk] = n;
       }
-      upper_bound_lockstep<PPT>([&](int64_t k) { return C[k]; }, zero, all, tg, live, p);
+      upper_bound_lockstep<PPT>(sum_at, zero, all, tg, live, p);
 #pragma unroll
       for (int pk = 0; pk < PPT; ++pk)
         if (live[pk]) srcs[pk] = p[pk] < n ? p[pk] : n - 1;
@@ -1897,7 +1939,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
       shared_eps<D>(Key{sk[2], sk[3]}, (uint32_t)(n * D), (uint32_t)i, eps[pk]);
       continue;
     }
-    const Key ki{kwp[pk].x, kwp[pk].y};  // split(step key, n)[i] (lf_csum)
+    const Key ki{kwp[pk].x, kwp[pk].y};  // split(step key, n)[i] (lf_prep)
 #pragma unroll
     for (uint32_t q = 0; q < hD; ++q) {
       uint32_t w0, w1;
@@ -1995,9 +2037,9 @@ template <class Model, int D, int DY, bool GRAD>
 __global__ __launch_bounds__(LT) void lf_step_kernel(LfArgs a, int64_t t, int cend_slots) {
   __shared__ LfScratch s;
   __shared__ Model model;
-  __shared__ uint64_t win[kSearchWin];
+  __shared__ uint64_t win[kSearchWin], off[kOffsets];
   extern __shared__ uint64_t cend[];  // cend_slots entries (launch-time size)
-  lf_step_chunk<Model, D, DY, GRAD>(a, t, cend_slots, blockIdx.x, s, model, win, cend);
+  lf_step_chunk<Model, D, DY, GRAD>(a, t, cend_slots, blockIdx.x, s, model, win, cend, off);
 }
 
 // ---------------------------------------------------------------- the one-launch step (n <= kSmallMax)
@@ -2338,18 +2380,15 @@ template <bool GRAD>
 MOCAT_DEV void lf_prep_call(const LfArgs& a, int64_t t, int64_t c, LfScratch& s) {
   lf_prep_chunk<GRAD>(a, t, c, s);
 }
-MOCAT_DEV void lf_csum_call(const LfArgs& a, int64_t t, int64_t c, LfScratch& s, uint64_t* cs) {
-  lf_csum_chunk(a, t, c, s, cs);
-}
 template <class Model, int D, int DY, bool GRAD>
 MOCAT_DEV void lf_step_call(const LfArgs& a, int64_t t, int cend_slots, int64_t c, LfScratch& s,
-                                          Model& model, uint64_t* win, uint64_t* cend) {
-  lf_step_chunk<Model, D, DY, GRAD>(a, t, cend_slots, c, s, model, win, cend);
+                                          Model& model, uint64_t* win, uint64_t* cend, uint64_t* off) {
+  lf_step_chunk<Model, D, DY, GRAD>(a, t, cend_slots, c, s, model, win, cend, off);
 }
 
 // launch_mode 2: steps 1 .. max_T - 1 (after lf_init_kernel) as one persistent kernel of gridDim.x
-// workgroups. Each step runs the three phases of the per-step launches (prep, prefix sums, step), a
-// grid barrier after each; in a phase workgroup b takes chunks b, b + G, b + 2G, ... of the chunks
+// workgroups. Each step runs the phases of the per-step launches (prep, if needed the categorical rows or the large
+// filters' offsets, step), a grid barrier after each; in a phase workgroup b takes chunks b, b + G, b + 2G, ... of the chunks
 // still running. The filters are laid out in order of decreasing length, so the chunks running at
 // step t are the first act[t] (act[t] = chunks of filters with T > t). The chunk functions are those
 // of the per-step kernels, so the results are the same bit for bit.
@@ -2358,9 +2397,8 @@ __global__ __launch_bounds__(LT) void lf_persist_kernel(LfArgs a, int64_t max_T,
                                                         const int32_t* __restrict__ act, uint32_t max_polls) {
   __shared__ LfScratch s;
   __shared__ Model model;
-  __shared__ uint64_t buf[kSearchWin];  // the prefix-sum phase's chunk sums, then the step's window
+  __shared__ uint64_t win[kSearchWin], off[kOffsets];
   extern __shared__ uint64_t cend[];
-  static_assert(kSearchWin >= CH, "the LDS buffer holds a chunk of prefix sums");
   const int64_t G = gridDim.x;
   uint32_t k = 0;
   for (int64_t t = 1; t < max_T; ++t) {
@@ -2370,16 +2408,17 @@ __global__ __launch_bounds__(LT) void lf_persist_kernel(LfArgs a, int64_t max_T,
       lf_prep_call<GRAD>(a, t, c, s);
     }
     if (!lf_grid_sync(a.bar, ++k, max_polls)) return;
-    for (int64_t c = blockIdx.x; c < as; c += G) {
-      __syncthreads();
-      lf_csum_call(a, t, c, s, buf);
-    }
     if (a.resampling == 2)
       for (int64_t k = blockIdx.x; k < as * kCatBlocks; k += G) lf_cat_block(a, t, k / kCatBlocks, (int)(k % kCatBlocks));
-    if (!lf_grid_sync(a.bar, ++k, max_polls)) return;
+    if (a.big)
+      for (int64_t f = blockIdx.x; f < a.n_large; f += G) {
+        __syncthreads();
+        lf_offsets_filter(a, t, f, s);
+      }
+    if ((a.resampling == 2 || a.big) && !lf_grid_sync(a.bar, ++k, max_polls)) return;
     for (int64_t c = blockIdx.x; c < as; c += G) {
       __syncthreads();
-      lf_step_call<Model, D, DY, GRAD>(a, t, cend_slots, c, s, model, buf, cend);
+      lf_step_call<Model, D, DY, GRAD>(a, t, cend_slots, c, s, model, win, cend, off);
     }
     if (!lf_grid_sync(a.bar, ++k, max_polls)) return;
   }
@@ -2545,7 +2584,7 @@ int launch_pf_large(const LfArgs& a, int64_t max_T, int cend_slots, const int32_
     hipLaunchKernelGGL((lf_init_kernel<Model, D, DY, GRAD, PPT>), chunks, blk, 0, q, a);
     for (int64_t t = 1; t < max_T; ++t) {
       hipLaunchKernelGGL((lf_prep_kernel<GRAD>), grid(t - 1), blk, 0, q, a, t);
-      hipLaunchKernelGGL(lf_csum_kernel, grid(t), blk, 0, q, a, t);
+      if (a.big) hipLaunchKernelGGL(lf_offsets_kernel, dim3(a.n_large), blk, 0, q, a, t);
       if (a.resampling == 2) hipLaunchKernelGGL(lf_cat_kernel, dim3(grid(t).x, kCatBlocks), blk, 0, q, a, t);
       hipLaunchKernelGGL((lf_step_kernel<Model, D, DY, GRAD>), grid(t), blk, cend_bytes, q, a, t, cend_slots);
     }
@@ -2592,8 +2631,9 @@ struct LfLayout {
   int n_large = 0;
   int cend_slots = 1;  // SG-block end sums the step kernel stages: the largest filter's, up to kChunkEnds
   int64_t n_chunks = 0, max_T = 0;
+  int64_t most_chunks = 0;  // of one filter
   int64_t n_tk = 0;  // step-key slots: the sum of T over the flagged filters
-  int64_t o_desc, o_cf, o_m, o_s1, o_s2, o_g, o_tot, o_st, o_cend, o_bnd, o_keys, o_act, o_bar, o_pk, o_anc, bytes;
+  int64_t o_desc, o_cf, o_m, o_s1, o_s2, o_g, o_tot, o_st, o_cend, o_coff, o_keys, o_act, o_bar, o_pk, o_anc, bytes;
 };
 
 int64_t lf_align(int64_t v) { return (v + 255) / 256 * 256; }
@@ -2612,6 +2652,7 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters, bool small) {
     if (!(filters[f].flags & kPfLarge)) continue;
     ++L.n_large;
     L.n_chunks += (filters[f].n + ch - 1) / ch;
+    L.most_chunks = std::max<int64_t>(L.most_chunks, (filters[f].n + ch - 1) / ch);
     L.max_T = std::max<int64_t>(L.max_T, filters[f].T);
     L.n_tk += std::max<int64_t>(filters[f].T, 0);
     L.cend_slots = (int)std::min<int64_t>(kChunkEnds, std::max<int64_t>(L.cend_slots, (filters[f].n + SG - 1) / SG));
@@ -2635,7 +2676,7 @@ LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters, bool small) {
   o = lf_align(o + (int64_t)L.n_large * (int64_t)sizeof(LfState));
   L.o_cend = o;
   o = lf_align(o + L.n_chunks * (ch / SG) * 8);
-  L.o_bnd = o;
+  L.o_coff = o;
   o = lf_align(o + L.n_chunks * 8);
   L.o_keys = o;
   o = lf_align(o + L.n_tk * (int64_t)sizeof(StepKey));
@@ -2860,9 +2901,10 @@ int mocat_pf_run_large(int model, int d, int dy, const mocat_pf_filter* host_fil
            reinterpret_cast<float*>(ws + L.o_m), reinterpret_cast<double*>(ws + L.o_s1),
            reinterpret_cast<double*>(ws + L.o_s2), reinterpret_cast<double*>(ws + L.o_g),
            reinterpret_cast<uint64_t*>(ws + L.o_tot), reinterpret_cast<LfState*>(ws + L.o_st),
-           reinterpret_cast<uint64_t*>(ws + L.o_cend), reinterpret_cast<int64_t*>(ws + L.o_bnd),
+           reinterpret_cast<uint64_t*>(ws + L.o_cend), reinterpret_cast<uint64_t*>(ws + L.o_coff),
            reinterpret_cast<StepKey*>(ws + L.o_keys), reinterpret_cast<uint32_t*>(ws + L.o_bar),
-           reinterpret_cast<int32_t*>(ws + L.o_anc), model == 2 ? nullptr : reinterpret_cast<uint32_t*>(ws + L.o_pk)};
+           reinterpret_cast<int32_t*>(ws + L.o_anc), model == 2 ? nullptr : reinterpret_cast<uint32_t*>(ws + L.o_pk),
+           resampling != 2 && L.most_chunks > kOffsets};
   if (model == 1) {
     if (d != dy) return MOCAT_ERR_ARG;
     if (d != 1 && out_grad) return MOCAT_ERR_ARG;

@@ -3,7 +3,7 @@
 A batch of independent filters of uneven sizes is split between two launch structures: filters below
 a particle-count threshold run one workgroup each in a single persistent launch; the others run on the
 chunked path (1024-particle chunks spread over the GPU, three grid-wide phases per time step), either
-as three launches per step queued one by one ("stream"), those launches captured into one HIP graph
+as the launches per step queued one by one ("stream"), those launches captured into one HIP graph
 ("graph"), or one persistent kernel with grid barriers between the phases ("persistent"). Which split
 and which launch mode is fastest depends on the batch (its size distribution and lengths), so the
 tuner times every candidate schedule on the batch itself, keeps the fastest, and records it under the
