@@ -955,7 +955,7 @@ __global__ __launch_bounds__(256) void categorical_kernel(const float* __restric
 // The weights are shifted by float(lse) and quantised with the shift of the largest weight exactly as
 // in pf_kernel, so for the same log-weights and key the ancestors are the same.
 //
-// Calls whose largest flagged filter has at most kSmallMax particles take one launch per step instead
+// Calls whose largest flagged filter has at most kSmallMax particles, unless they are many, take one launch per step instead
 // (lf_small_kernel, 256-particle chunks): every workgroup redoes the statistics and the prefix sums of its
 // whole filter, which costs less than two more dependent launches.
 constexpr int LT = 256;          // threads per workgroup
@@ -2638,11 +2638,19 @@ struct LfLayout {
 
 int64_t lf_align(int64_t v) { return (v + 255) / 256 * 256; }
 
-// Whether the flagged filters of a call take the one-launch step.
+// Whether the flagged filters of a call take the one-launch step: none is above kSmallMax, and the work that its
+// workgroups repeat, n weights for each of n / SCH of them, is small enough (50 steps, d = 4, one-launch / chunked: 64
+// filters of 4096 particles 1.83 / 2.30 ms, 128 2.99 / 2.84, 256 5.23 / 4.21; stochastic volatility 1.62 / 1.81, 2.60 /
+// 2.26, 4.74 / 3.59; 512 of 2048 particles 6.1 / 6.3).
+constexpr int64_t kSmallWork = 1500000000;  // sum of n^2
 bool lf_small(const mocat_pf_filter* filters, int n_filters) {
-  for (int f = 0; f < n_filters; ++f)
-    if ((filters[f].flags & kPfLarge) && filters[f].n > kSmallMax) return false;
-  return true;
+  int64_t work = 0;
+  for (int f = 0; f < n_filters; ++f) {
+    if (!(filters[f].flags & kPfLarge)) continue;
+    if (filters[f].n > kSmallMax) return false;
+    work += filters[f].n * filters[f].n;
+  }
+  return work <= kSmallWork;
 }
 
 LfLayout lf_layout(const mocat_pf_filter* filters, int n_filters, bool small) {

@@ -25,3 +25,15 @@ def test_chunk_offsets(ns, method, launch):
             assert torch.equal(a.value, b.value) and torch.equal(a.log_weight, b.log_weight)
             np.testing.assert_allclose(a.ess.cpu().numpy(), b.ess.cpu().numpy(), rtol=1e-6)
             np.testing.assert_allclose(a.log_likelihood.item(), b.log_likelihood.item(), rtol=1e-10)
+
+
+@pytest.mark.parametrize("count", [89, 90])  # either side of the work up to which the steps take one launch
+def test_many_small_filters(count):
+    import mocat_amd as m
+    model = m.ssm.StochasticVolatility(1, 0.0, 1.0, 0.95, 0.04, 0.6)
+    y = np.random.default_rng(3).normal(size=(3, 1)).astype(np.float32)
+    keys, ns = list(m.random.split(m.random.PRNGKey(8), count)), [4096] * count
+    run = lambda n: m.ssm.run_particle_filters([model] * count, [y] * count, keys, ns, 1.0, "systematic", store=True, large_n=n)
+    for a, b in zip(run(1 << 40), run(1)):
+        assert torch.equal(a.ancestors, b.ancestors)
+        assert torch.equal(a.value, b.value) and torch.equal(a.log_weight, b.log_weight)
