@@ -363,12 +363,14 @@ struct Bf16Engine {
   // caller before a barrier); each wave returns its partial gradients and leaves its potential partials in
   // s.ured[w]. Two compiled passes (the potential terms are needed after the last leapfrog step only), so that
   // each block's row functions and MFMAs form one straight-line region the scheduler can interleave.
-  template <bool WANT_POT>
-  static MOCAT_DEV void partials(Smem& s, const void* packed, int n, Acc& acc) {
+  // SPLIT: the workgroup is number `part` of `parts` that share the blocks, wave w takes rb = part NW + w + parts NW j.
+  template <bool WANT_POT, bool SPLIT = false>
+  static MOCAT_DEV void partials(Smem& s, const void* packed, int n, Acc& acc, int part = 0, int parts = 1) {
     const int t = threadIdx.x;
     const int lane = t & (kWave - 1), w = t / kWave, g = lane >> 5, col = lane & 31;
     const int nrb = (n + 31) / 32;
-    const int nmine = nrb > w ? (nrb - w + NW - 1) / NW : 0;  // blocks rb = w + j * NW, j < nmine
+    const int rb0 = SPLIT ? part * NW + w : w, stride = SPLIT ? parts * NW : NW;
+    const int nmine = nrb > rb0 ? (nrb - rb0 + stride - 1) / stride : 0;  // blocks rb = rb0 + j * stride, j < nmine
     const char* base = reinterpret_cast<const char*>(packed);
     bf16x8 th[kThetaRegs ? KB : 1], tl[kThetaRegs ? KB : 1];
     if constexpr (kThetaRegs) {
@@ -387,7 +389,7 @@ struct Bf16Engine {
         for (int r = 0; r < 16; ++r) acc.g[ct][nb][r] = 0.f;
     }
 
-    auto blk = [&](int j) { return base + (int64_t)(w + j * NW) * L::BLOCK_BYTES; };
+    auto blk = [&](int j) { return base + (int64_t)(rb0 + j * stride) * L::BLOCK_BYTES; };
     auto load_a = [&](ABuf& a, int j) {
       const bf16x8* A = reinterpret_cast<const bf16x8*>(blk(j));
 #pragma unroll
@@ -493,7 +495,7 @@ struct Bf16Engine {
     if constexpr (WANT_POT) {
       // padding rows of the last block (x = 0, y = 0.5: z = 0) each added the same term
       const int rbl = nrb - 1;
-      if (rbl % NW == w) {
+      if (rbl % stride == rb0) {
         float cpad;
         lr_row_full_hw(0.f, 0.5f, cpad);
         int npad = 0;
@@ -697,10 +699,18 @@ __global__ __launch_bounds__(NT) void lr_eval_kernel(LrArgs a, const float* __re
 
 // The evaluation with the bf16x3 engine: thread t owns chain c = t % 32 of each of the NCT tiles and the columns
 // k0 = EPT (t / 32) .. of it, whose values stay in registers.
-template <int DP, int NT, int NCT>
+// SPLIT: gridDim.y workgroups share the rows of X; lik_pot and grad_lik then hold each one's partial sums, [gridDim.y]
+// times the arrays (lr_eval_sum_kernel adds them), and the first of them writes the prior's.
+template <int DP, int NT, int NCT, bool SPLIT = false>
 __global__ __launch_bounds__(NT) void lr_eval_bf16_kernel(LrArgs a, const float* __restrict__ theta, int64_t C,
                                                           float* prior_pot, float* lik_pot, float* grad_prior,
                                                           float* grad_lik) {
+  const int part = SPLIT ? (int)blockIdx.y : 0, parts = SPLIT ? (int)gridDim.y : 1;
+  if constexpr (SPLIT) {
+    if (part != 0) prior_pot = grad_prior = nullptr;
+    lik_pot += part * C;
+    grad_lik += part * C * a.d;
+  }
   using E = Bf16Engine<DP, NT, NCT>;
   constexpr int NG = NT / CT, EPT = DP / NG;
   static_assert(NG * EPT == DP && EPT % 4 == 0, "thread ownership");
@@ -722,8 +732,8 @@ __global__ __launch_bounds__(NT) void lr_eval_bf16_kernel(LrArgs a, const float*
   }
   __syncthreads();
   typename E::Acc acc;
-  if (lik_pot)
-    E::template partials<true>(es, a.packed, a.n, acc);
+  if (SPLIT || lik_pot)
+    E::template partials<true, SPLIT>(es, a.packed, a.n, acc, part, parts);
   else
     E::template partials<false>(es, a.packed, a.n, acc);
 #pragma unroll
@@ -752,6 +762,24 @@ __global__ __launch_bounds__(NT) void lr_eval_bf16_kernel(LrArgs a, const float*
         prior_pot[chain] = a.prior_prec > 0.f
                                ? fmaf(0.5f * (float)d, kLog2Pi - logf(a.prior_prec), 0.5f * a.prior_prec * s2)
                                : 0.f;
+    }
+  }
+}
+
+// The sums of the row parts, in their order.
+__global__ __launch_bounds__(256) void lr_eval_sum_kernel(const float* __restrict__ lik, const float* __restrict__ grad,
+                                                          int parts, int64_t C, int64_t d, float* lik_pot,
+                                                          float* grad_lik) {
+  for (int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x; e < C * d; e += (int64_t)gridDim.x * 256) {
+    float g = 0.f;
+#pragma unroll 8
+    for (int p = 0; p < parts; ++p) g += grad[p * C * d + e];
+    if (grad_lik) grad_lik[e] = g;
+    if (e < C && lik_pot) {
+      float l = 0.f;
+#pragma unroll 8
+      for (int p = 0; p < parts; ++p) l += lik[p * C + e];
+      lik_pot[e] = l;
     }
   }
 }
@@ -1465,6 +1493,31 @@ int launch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, 
   return MOCAT_OK;
 }
 
+// Parts the rows of X are split into for C points: few points (one workgroup per 32 of them) leave the other CUs idle. At
+// least four 32-row blocks per wave are left, and nothing is split below twelve, where the second launch costs
+// more than it saves. A call unsplit / split, us: X 1505x100, 40 points 26.5 / 20.2, 4096 points 29.5 / 27.0; X 3100x64, 40
+// points 26.9 / 18.6; X 20000x100, 1 point 254 / 19, 1024 259 / 56, 4096 263 / 159 (about 15 us of each is the host's).
+constexpr int kMaxParts = 32;
+int eval_parts(int64_t n, int64_t d, int64_t C) {
+  const int64_t nw = (d <= 64 ? kBf16Threads64 : kBf16Threads128) / kWave, nrb = (n + 31) / 32, tile = (C + CT - 1) / CT;
+  if (nrb < 12 * nw || tile > 128) return 1;
+  return (int)std::min<int64_t>(std::min<int64_t>(kMaxParts, 256 / tile), nrb / (4 * nw));
+}
+
+template <int DP>
+int launch_eval_split(const LrArgs& a, const float* theta, int64_t C, int parts, float* ws, float* pp, float* lp, float* gp,
+                      float* gl, hipStream_t st) {
+  constexpr int NT = DP == 64 ? kBf16Threads64 : kBf16Threads128;
+  float *lik = ws, *grad = ws + parts * C;
+  hipLaunchKernelGGL((lr_eval_bf16_kernel<DP, NT, 1, true>), dim3(tiles(C, 1), parts), dim3(NT), 0, st, a, theta, C, pp, lik,
+                     gp, grad);
+  const int64_t blocks = (C * a.d + 255) / 256;
+  hipLaunchKernelGGL(lr_eval_sum_kernel, dim3((unsigned)std::min<int64_t>(blocks, 65535)), dim3(256), 0, st, (const float*)lik,
+                     (const float*)grad, parts, C, (int64_t)a.d, lp, gl);
+  MOCAT_LAUNCH_CHECK();
+  return MOCAT_OK;
+}
+
 int dispatch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, float* lp, float* gp, float* gl,
                        hipStream_t st) {
   return a.d <= 64 ? launch_eval_bf16<64>(a, theta, C, pp, lp, gp, gl, st)
@@ -1535,6 +1588,34 @@ int mocat_lr_potential_grad(const float* X, const float* y, const void* packed, 
     return dispatch_eval<Fp64Engine>(a, theta, C, prior_pot, lik_pot, grad_prior, grad_lik, stream);
   return precision == 0 ? dispatch_eval<Fp32Engine>(a, theta, C, prior_pot, lik_pot, grad_prior, grad_lik, stream)
                         : dispatch_eval_bf16(a, theta, C, prior_pot, lik_pot, grad_prior, grad_lik, stream);
+}
+
+int mocat_lr_eval_workspace_bytes(int64_t n, int64_t d, int precision, int64_t C, int64_t* bytes) {
+  if (!bytes || n <= 0 || d <= 0 || d > 128 || C < 0) return MOCAT_ERR_ARG;
+  const int parts = precision == 1 && C > 0 ? eval_parts(n, d, C) : 1;
+  *bytes = parts > 1 ? parts * C * (d + 1) * (int64_t)sizeof(float) : 0;
+  return MOCAT_OK;
+}
+
+int mocat_lr_potential_grad_split(const float* X, const float* y, const void* packed, int64_t n, int64_t d, int precision,
+                                  float prior_prec, float temperature, const float* theta, int64_t C, float* prior_pot,
+                                  float* lik_pot, float* grad_prior, float* grad_lik, void* workspace,
+                                  int64_t workspace_bytes, hipStream_t stream) {
+  int rc = check_lr(X, y, packed, n, d, precision);
+  if (rc) return rc;
+  if (C < 0 || (C > 0 && !theta)) return MOCAT_ERR_ARG;
+  int64_t need = 0;
+  rc = mocat_lr_eval_workspace_bytes(n, d, precision, C, &need);
+  if (rc) return rc;
+  if (need == 0)
+    return mocat_lr_potential_grad(X, y, packed, n, d, precision, prior_prec, temperature, theta, C, prior_pot, lik_pot,
+                                   grad_prior, grad_lik, stream);
+  if (!workspace || workspace_bytes < need) return MOCAT_ERR_SIZE;
+  LrArgs a{X, y, packed, (int)n, (int)d, prior_prec, temperature};
+  const int parts = eval_parts(n, d, C);
+  float* ws = static_cast<float*>(workspace);
+  return d <= 64 ? launch_eval_split<64>(a, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream)
+                 : launch_eval_split<128>(a, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream);
 }
 
 int mocat_hmc_lr_iterate(const float* X, const float* y, const void* packed, int64_t n, int64_t d, int precision,

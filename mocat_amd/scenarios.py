@@ -19,6 +19,7 @@ from .core import Scenario
 
 PRECISIONS = {"fp32": 0, "bf16x3": 1, "fp64": 3}
 ENGINE_GAUSSIAN = 2
+SPLIT_MIN_ROWS = 1505  # fewer rows are never split over workgroups (mocat_lr_eval_workspace_bytes)
 
 _lib.register("mocat_gmm_potential_grad", [_lib.c_ptr, _lib.c_i64, _lib.c_i64, _lib.c_i32, _lib.c_ptr, _lib.c_ptr,
                                            _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr])
@@ -26,9 +27,12 @@ _lib.register("mocat_gmm_full_potential_grad", [_lib.c_ptr, _lib.c_i64, _lib.c_i
                                                 _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr])
 _lib.register("mocat_lr_packed_bytes", [_lib.c_i64, _lib.c_i64, _lib.c_ptr])
 _lib.register("mocat_lr_pack", [_lib.c_ptr, _lib.c_ptr, _lib.c_i64, _lib.c_i64, _lib.c_ptr, _lib.c_ptr])
+_lib.register("mocat_lr_eval_workspace_bytes", [_lib.c_i64, _lib.c_i64, _lib.c_i32, _lib.c_i64, _lib.c_ptr])
 _lib.register("mocat_lr_potential_grad",
               [_lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_i64, _lib.c_i64, _lib.c_i32, _lib.c_f32, _lib.c_f32,
                _lib.c_ptr, _lib.c_i64, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr])
+_lib.register("mocat_lr_potential_grad_split",
+              _lib.SIGNATURES["mocat_lr_potential_grad"][:-1] + [_lib.c_ptr, _lib.c_i64, _lib.c_ptr])
 
 
 class FusedPotential(torch.autograd.Function):
@@ -120,6 +124,15 @@ class LogisticRegression(Scenario):
         gp = torch.empty_like(x)
         gl = torch.empty_like(x)
         X, y, packed, n, d, prec, pprec = self.kernel_args()
+        if prec == PRECISIONS["bf16x3"] and n >= SPLIT_MIN_ROWS:
+            nbytes = _lib.c_i64(0)
+            _lib.call("mocat_lr_eval_workspace_bytes", n, d, prec, C, _lib.ctypes.byref(nbytes))
+            if nbytes.value:
+                ws = torch.empty(nbytes.value // 4, dtype=torch.float32, device=x.device)
+                _lib.call("mocat_lr_potential_grad_split", X, y, packed, n, d, prec, pprec, float(temperature),
+                          _lib.ptr(x), C, _lib.ptr(pp), _lib.ptr(lp), _lib.ptr(gp), _lib.ptr(gl), _lib.ptr(ws),
+                          nbytes.value, _lib.stream_handle())
+                return pp, lp, gp, gl
         _lib.call("mocat_lr_potential_grad", X, y, packed, n, d, prec, pprec, float(temperature), _lib.ptr(x), C,
                   _lib.ptr(pp), _lib.ptr(lp), _lib.ptr(gp), _lib.ptr(gl), _lib.stream_handle())
         return pp, lp, gp, gl
