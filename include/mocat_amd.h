@@ -69,8 +69,8 @@ int mocat_lr_potential_grad(const float* X, const float* y, const void* packed, 
                             int precision, float prior_prec, float temperature, const float* theta, int64_t C,
                             float* prior_pot, float* lik_pot, float* grad_prior, float* grad_lik,
                             hipStream_t stream);
-/* The same with the rows of X shared by several workgroups where few points leave most of the GPU idle (bf16x3 over
- * many rows; the sums over rows are then added in another order). workspace: as many bytes as
+/* The same with the rows of X shared by several workgroups where few points leave most of the GPU idle (bf16x3 and
+ * FP32; the sums over rows are then added in another order). workspace: as many bytes as
  * mocat_lr_eval_workspace_bytes says for the call (0: not split, workspace may be NULL), 4-byte aligned. */
 int mocat_lr_eval_workspace_bytes(int64_t n, int64_t d, int precision, int64_t C, int64_t* bytes);
 int mocat_lr_potential_grad_split(const float* X, const float* y, const void* packed, int64_t n, int64_t d,

@@ -670,10 +670,20 @@ MOCAT_DEV void tile_eval(typename Engine::Smem& es, TileState<DP>& ts, const LrA
   __syncthreads();
 }
 
-template <class Engine, int DP, int NT>
+// SPLIT: gridDim.y workgroups share the rows of X, `rows` each, and write partial sums as lr_eval_bf16_kernel does.
+template <class Engine, int DP, int NT, bool SPLIT = false>
 __global__ __launch_bounds__(NT) void lr_eval_kernel(LrArgs a, const float* __restrict__ theta, int64_t C,
                                                      float* prior_pot, float* lik_pot, float* grad_prior,
-                                                     float* grad_lik) {
+                                                     float* grad_lik, int rows = 0) {
+  if constexpr (SPLIT) {
+    const int part = (int)blockIdx.y, r0 = part * rows;
+    a.X += (int64_t)r0 * a.d;
+    a.y += r0;
+    a.n = a.n - r0 < rows ? a.n - r0 : rows;
+    if (part != 0) prior_pot = grad_prior = nullptr;
+    lik_pot += part * C;
+    grad_lik += part * C * a.d;
+  }
   __shared__ TileState<DP> ts;
   __shared__ typename Engine::Smem es;
   const int t = threadIdx.x;
@@ -1432,10 +1442,10 @@ int dispatch_eval(const LrArgs& a, const float* theta, int64_t C, float* pp, flo
   const unsigned blocks = (unsigned)((C + CT - 1) / CT);
   if (a.d <= 64)
     hipLaunchKernelGGL((lr_eval_kernel<E<64, kThreads>, 64, kThreads>), dim3(blocks), dim3(kThreads), 0, st, a,
-                       theta, C, pp, lp, gp, gl);
+                       theta, C, pp, lp, gp, gl, 0);
   else
     hipLaunchKernelGGL((lr_eval_kernel<E<128, kThreads>, 128, kThreads>), dim3(blocks), dim3(kThreads), 0, st, a,
-                       theta, C, pp, lp, gp, gl);
+                       theta, C, pp, lp, gp, gl, 0);
   MOCAT_LAUNCH_CHECK();
   return MOCAT_OK;
 }
@@ -1497,20 +1507,37 @@ int launch_eval_bf16(const LrArgs& a, const float* theta, int64_t C, float* pp, 
 // least four 32-row blocks per wave are left, and nothing is split below twelve, where the second launch costs
 // more than it saves. A call unsplit / split, us: X 1505x100, 40 points 26.5 / 20.2, 4096 points 29.5 / 27.0; X 3100x64, 40
 // points 26.9 / 18.6; X 20000x100, 1 point 254 / 19, 1024 259 / 56, 4096 263 / 159 (about 15 us of each is the host's).
-constexpr int kMaxParts = 32;
-int eval_parts(int64_t n, int64_t d, int64_t C) {
-  const int64_t nw = (d <= 64 ? kBf16Threads64 : kBf16Threads128) / kWave, nrb = (n + 31) / 32, tile = (C + CT - 1) / CT;
-  if (nrb < 12 * nw || tile > 128) return 1;
-  return (int)std::min<int64_t>(std::min<int64_t>(kMaxParts, 256 / tile), nrb / (4 * nw));
+// FP32: blocks of 64 rows, from four on: X 193x64, 1 point 21.1 / 19.9, 285x100 41 / 20, 1390x100 166 / 20, 20000x100 3060 / 85; 4096
+// points 37 / 28 (193x100), 172 / 98 (1390x100), 3008 / 1520 (20000x100).
+constexpr int kMaxParts = 32, kFp32Rows = 64;
+int eval_parts(int precision, int64_t n, int64_t d, int64_t C) {
+  const int64_t tile = (C + CT - 1) / CT;
+  if (tile < 1 || tile > 128) return 1;
+  const int64_t most = std::min<int64_t>(kMaxParts, 256 / tile);
+  if (precision == 0) {
+    const int64_t blocks = (n + kFp32Rows - 1) / kFp32Rows;
+    if (blocks < 4) return 1;
+    const int64_t per = (blocks + most - 1) / most;
+    return (int)((blocks + per - 1) / per);
+  }
+  if (precision != 1) return 1;
+  const int64_t nw = (d <= 64 ? kBf16Threads64 : kBf16Threads128) / kWave, nrb = (n + 31) / 32;
+  return nrb < 12 * nw ? 1 : (int)std::min<int64_t>(most, nrb / (4 * nw));
 }
 
 template <int DP>
-int launch_eval_split(const LrArgs& a, const float* theta, int64_t C, int parts, float* ws, float* pp, float* lp, float* gp,
-                      float* gl, hipStream_t st) {
+int launch_eval_split(const LrArgs& a, int precision, const float* theta, int64_t C, int parts, float* ws, float* pp,
+                      float* lp, float* gp, float* gl, hipStream_t st) {
   constexpr int NT = DP == 64 ? kBf16Threads64 : kBf16Threads128;
   float *lik = ws, *grad = ws + parts * C;
-  hipLaunchKernelGGL((lr_eval_bf16_kernel<DP, NT, 1, true>), dim3(tiles(C, 1), parts), dim3(NT), 0, st, a, theta, C, pp, lik,
-                     gp, grad);
+  if (precision == 0) {
+    const int blocks = (a.n + kFp32Rows - 1) / kFp32Rows, rows = (blocks + parts - 1) / parts * kFp32Rows;
+    hipLaunchKernelGGL((lr_eval_kernel<Fp32Engine<DP, kThreads>, DP, kThreads, true>), dim3(tiles(C, 1), parts),
+                       dim3(kThreads), 0, st, a, theta, C, pp, lik, gp, grad, rows);
+  } else {
+    hipLaunchKernelGGL((lr_eval_bf16_kernel<DP, NT, 1, true>), dim3(tiles(C, 1), parts), dim3(NT), 0, st, a, theta, C, pp,
+                       lik, gp, grad);
+  }
   const int64_t blocks = (C * a.d + 255) / 256;
   hipLaunchKernelGGL(lr_eval_sum_kernel, dim3((unsigned)std::min<int64_t>(blocks, 65535)), dim3(256), 0, st, (const float*)lik,
                      (const float*)grad, parts, C, (int64_t)a.d, lp, gl);
@@ -1592,7 +1619,7 @@ int mocat_lr_potential_grad(const float* X, const float* y, const void* packed, 
 
 int mocat_lr_eval_workspace_bytes(int64_t n, int64_t d, int precision, int64_t C, int64_t* bytes) {
   if (!bytes || n <= 0 || d <= 0 || d > 128 || C < 0) return MOCAT_ERR_ARG;
-  const int parts = precision == 1 && C > 0 ? eval_parts(n, d, C) : 1;
+  const int parts = eval_parts(precision, n, d, C);
   *bytes = parts > 1 ? parts * C * (d + 1) * (int64_t)sizeof(float) : 0;
   return MOCAT_OK;
 }
@@ -1612,10 +1639,10 @@ int mocat_lr_potential_grad_split(const float* X, const float* y, const void* pa
                                    grad_prior, grad_lik, stream);
   if (!workspace || workspace_bytes < need) return MOCAT_ERR_SIZE;
   LrArgs a{X, y, packed, (int)n, (int)d, prior_prec, temperature};
-  const int parts = eval_parts(n, d, C);
+  const int parts = eval_parts(precision, n, d, C);
   float* ws = static_cast<float*>(workspace);
-  return d <= 64 ? launch_eval_split<64>(a, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream)
-                 : launch_eval_split<128>(a, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream);
+  return d <= 64 ? launch_eval_split<64>(a, precision, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream)
+                 : launch_eval_split<128>(a, precision, theta, C, parts, ws, prior_pot, lik_pot, grad_prior, grad_lik, stream);
 }
 
 int mocat_hmc_lr_iterate(const float* X, const float* y, const void* packed, int64_t n, int64_t d, int precision,

@@ -19,7 +19,8 @@ from .core import Scenario
 
 PRECISIONS = {"fp32": 0, "bf16x3": 1, "fp64": 3}
 ENGINE_GAUSSIAN = 2
-SPLIT_MIN_ROWS = 1505  # fewer rows are never split over workgroups (mocat_lr_eval_workspace_bytes)
+# by precision, the rows below which an evaluation is never split over workgroups (mocat_lr_eval_workspace_bytes)
+SPLIT_MIN_ROWS = {PRECISIONS["bf16x3"]: 1505, PRECISIONS["fp32"]: 193}
 
 _lib.register("mocat_gmm_potential_grad", [_lib.c_ptr, _lib.c_i64, _lib.c_i64, _lib.c_i32, _lib.c_ptr, _lib.c_ptr,
                                            _lib.c_ptr, _lib.c_ptr, _lib.c_ptr, _lib.c_ptr])
@@ -124,7 +125,7 @@ class LogisticRegression(Scenario):
         gp = torch.empty_like(x)
         gl = torch.empty_like(x)
         X, y, packed, n, d, prec, pprec = self.kernel_args()
-        if prec == PRECISIONS["bf16x3"] and n >= SPLIT_MIN_ROWS:
+        if n >= SPLIT_MIN_ROWS.get(prec, math.inf):
             nbytes = _lib.c_i64(0)
             _lib.call("mocat_lr_eval_workspace_bytes", n, d, prec, C, _lib.ctypes.byref(nbytes))
             if nbytes.value:
