@@ -46,9 +46,11 @@ DEFAULT_STACK = ("value", "potential", "alpha", "stepsize", "momenta")
 
 def evaluate(scenario, x, temperature, random_key=None):
     """(prior_potential, likelihood_potential, grad_prior, grad_likelihood) at x (C, d): the fused
-    kernel of a compiled scenario, or a user scenario's torch potentials (their keys as mocat passes
-    them: `random_key` [C][2] per chain, or None)."""
+    kernel of a compiled scenario, its sums in the order of the fused iterations, or a user scenario's torch
+    potentials (their keys as mocat passes them: `random_key` [C][2] per chain, or None)."""
     if getattr(scenario, "_fused_kernel", False):
+        if getattr(scenario.evaluate, "takes_split", False):
+            return scenario.evaluate(x, temperature, split=False)
         return scenario.evaluate(x, temperature)
     return scenario.evaluate(x, temperature, random_key)
 

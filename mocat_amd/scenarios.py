@@ -113,8 +113,12 @@ class LogisticRegression(Scenario):
         return (_lib.ptr(self.X), _lib.ptr(self.y), _lib.ptr(self.packed), self.n, self.dim,
                 PRECISIONS[self.precision], float(self.prior_precision))
 
-    def evaluate(self, x: torch.Tensor, temperature: float = 1.0):
-        """(prior_potential, likelihood_potential, grad_prior, grad_likelihood) for x (..., d)."""
+    def evaluate(self, x: torch.Tensor, temperature: float = 1.0, split: bool = True):
+        """(prior_potential, likelihood_potential, grad_prior, grad_likelihood) for x (..., d). split: at few
+        points the rows of X may be shared by several workgroups, which adds the sums over rows in an order that
+        depends on the number of points. Samplers take split=False (mcmc.evaluate), the order of the
+        fused iterations: a chain started from a gradient 2e-7 away ends up to 1e-4 away (360 leapfrog steps,
+        X 3700 x 7)."""
         x = _dev_tensor(x)
         if x.shape[-1] != self.dim:
             raise ValueError(f"expected trailing dimension {self.dim}, got {tuple(x.shape)}")
@@ -125,7 +129,7 @@ class LogisticRegression(Scenario):
         gp = torch.empty_like(x)
         gl = torch.empty_like(x)
         X, y, packed, n, d, prec, pprec = self.kernel_args()
-        if n >= SPLIT_MIN_ROWS.get(prec, math.inf):
+        if split and n >= SPLIT_MIN_ROWS.get(prec, math.inf):
             nbytes = _lib.c_i64(0)
             _lib.call("mocat_lr_eval_workspace_bytes", n, d, prec, C, _lib.ctypes.byref(nbytes))
             if nbytes.value:
@@ -137,6 +141,8 @@ class LogisticRegression(Scenario):
         _lib.call("mocat_lr_potential_grad", X, y, packed, n, d, prec, pprec, float(temperature), _lib.ptr(x), C,
                   _lib.ptr(pp), _lib.ptr(lp), _lib.ptr(gp), _lib.ptr(gl), _lib.stream_handle())
         return pp, lp, gp, gl
+
+    evaluate.takes_split = True  # a subclass's own evaluate need not
 
     # differentiable potentials: torch.autograd reaches the kernel's adjoint through FusedPotential
     def prior_potential(self, x, random_key=None):
