@@ -211,13 +211,9 @@ __global__ __launch_bounds__(256) void ffbsi_step_kernel(const float* __restrict
       wi[w] = bi;
     }
     __syncthreads();
-    best = wbest[0];
-    bi = wi[0];
-    for (int k = 1; k < W; ++k)
-      if (wi[k] != kNoIndex && (bi == kNoIndex || wbest[k] > best || (wbest[k] == best && wi[k] < bi))) {
-        best = wbest[k];
-        bi = wi[k];
-      }
+    GumbelRow all;
+    for (int k = 0; k < W; ++k) all.take(wbest[k], wi[k]);
+    bi = all.bi;
     if (w != 0) return;
   }
   if (lane == 0 && idx) idx[m] = (int32_t)bi;
