@@ -869,19 +869,27 @@ def _on_device(parts):
     return torch.from_numpy(np.concatenate([p.reshape(-1) for p in parts])).to(mr.default_device())
 
 
+def _has_shapes(lgssm, **shapes):
+    """Whether these attributes have these shapes. The models do not compare theirs, and packed arrays of other
+    shapes would be read as another model (or past their end): the torch operations raise, or broadcast."""
+    return all(np.shape(getattr(lgssm, name)) == shape for name, shape in shapes.items())
+
+
 def _kalman_filter_kernel(lgssm, yn):
-    """The filter in one launch, or None when the dimensions have no kernel or an innovation covariance has no
-    Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
+    """The filter in one launch, or None when the dimensions or shapes have no kernel or an innovation covariance
+    has no Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
     observations H = 0, R = 1, y = 0."""
     T, dy = yn.shape
-    d = int(np.shape(lgssm.transition_matrix)[0])
+    d = int(np.prod(np.shape(lgssm.initial_mean)))
     k = max(d, dy)
-    if not T or k > KALMAN_MAX_DIM or np.shape(lgssm.likelihood_matrix) != (dy, d):
+    if not T or min(d, dy) < 1 or k > KALMAN_MAX_DIM or not _has_shapes(
+            lgssm, initial_mean=(d,), initial_covariance=(d, d), transition_matrix=(d, d),
+            transition_covariance=(d, d), likelihood_matrix=(dy, d), likelihood_covariance=(dy, dy)):
         return None
     model = _on_device([_padded(lgssm.transition_matrix, k), _padded(lgssm.transition_covariance, k, 1.0),
                         _padded(lgssm.likelihood_matrix, k), _padded(lgssm.likelihood_covariance, k, 1.0),
                         _padded(lgssm.initial_covariance, k, 1.0),
-                        np.pad(np.asarray(lgssm.initial_mean, np.float64).reshape(-1), (0, k - d)),
+                        np.pad(np.asarray(lgssm.initial_mean, np.float64), (0, k - d)),
                         np.pad(yn, ((0, 0), (0, k - dy)))])
     out = torch.empty(T * (d + d * d + k + 1) + 2, dtype=torch.float64, device=model.device)
     means, covs, ll, scratch, info = torch.split(out, [T * d, T * d * d, 1, T * (k + 1), 1])
@@ -899,7 +907,7 @@ def run_kalman_filter_for_marginals(lgssm, y, t=None):
     the same for the identity). FP64 on the GPU: one kernel up to dimension KALMAN_MAX_DIM, else (and where
     an innovation covariance is not positive definite, which raises) torch operations step by step."""
     yn = np.asarray(y.detach().cpu() if isinstance(y, torch.Tensor) else y, np.float64)
-    yn = yn.reshape(len(yn), -1)
+    yn = yn.reshape(len(yn), -1 if yn.size else 0)
     out = _kalman_filter_kernel(lgssm, yn)
     if out is not None:
         return out
@@ -926,10 +934,13 @@ def run_kalman_filter_for_marginals(lgssm, y, t=None):
 
 
 def _kalman_smoother_kernel(lgssm, f_mus, f_covs):
-    """The smoother in three launches, or None when the dimension has no kernel or a predicted covariance has
-    no Cholesky factor."""
+    """The smoother in three launches, or None when the dimension or shapes have no kernel or a predicted
+    covariance has no Cholesky factor."""
+    if f_mus.dim() != 2:
+        return None
     T, d = f_mus.shape
-    if not T or d > KALMAN_MAX_DIM or f_covs.shape != (T, d, d) or np.shape(lgssm.transition_matrix) != (d, d):
+    if not T or not 1 <= d <= KALMAN_MAX_DIM or f_covs.shape != (T, d, d) or not _has_shapes(
+            lgssm, transition_matrix=(d, d), transition_covariance=(d, d)):
         return None
     model = _on_device([_padded(lgssm.transition_matrix, d), _padded(lgssm.transition_covariance, d)])
     out = torch.empty(T * (d + d * d) + (T - 1) * 3 * d * d + 1, dtype=torch.float64, device=model.device)
@@ -953,7 +964,7 @@ def run_kalman_smoother_for_marginals_and_lag_ones(lgssm, y, t=None, filter_outp
     f_mus = torch.as_tensor(f_mus, dtype=torch.float64, device=dev)
     f_covs = torch.as_tensor(f_covs, dtype=torch.float64, device=dev)
     T = f_mus.shape[0]
-    out = _kalman_smoother_kernel(lgssm, f_mus.contiguous(), f_covs.contiguous()) if f_mus.dim() == 2 else None
+    out = _kalman_smoother_kernel(lgssm, f_mus.contiguous(), f_covs.contiguous())
     if out is not None:
         return out
     A, Q, _, _, _, _, dev = _kalman_mats(lgssm)
