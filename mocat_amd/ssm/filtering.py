@@ -933,10 +933,18 @@ def run_kalman_filter_for_marginals(lgssm, y, t=None):
     return KalmanOutput(torch.stack(means), torch.stack(covs), ll)
 
 
+def _recorded(*tensors):
+    """Whether a gradient, a tangent, a functorch transform (vmap, grad, jvp) or a trace follows these: the kernels
+    leave nothing for them to record."""
+    return torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0 or any(
+        t.requires_grad and torch.is_grad_enabled() or torch._C._functorch.is_functorch_wrapped_tensor(t)
+        or torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def _kalman_smoother_kernel(lgssm, f_mus, f_covs):
-    """The smoother in three launches, or None when the dimension or shapes have no kernel or a predicted
-    covariance has no Cholesky factor."""
-    if f_mus.dim() != 2:
+    """The smoother in three launches, or None when the dimension or shapes have no kernel, the filter's moments are
+    differentiated or traced, or a predicted covariance has no Cholesky factor."""
+    if f_mus.dim() != 2 or _recorded(f_mus, f_covs):
         return None
     T, d = f_mus.shape
     if not T or not 1 <= d <= KALMAN_MAX_DIM or f_covs.shape != (T, d, d) or not _has_shapes(
@@ -958,7 +966,7 @@ def run_kalman_smoother_for_marginals_and_lag_ones(lgssm, y, t=None, filter_outp
     gain J = P_t A^T (A P_t A^T + Q)^-1, m_t = f_t + J (m_t+1 - A f_t), P_t = F_t + J (P_t+1 - A F_t A^T - Q) J^T,
     and mocat's lag-one term written as it is there, f_t . m_t+1 + J (P_t+1 + (m_t+1 - f_t+1) . m_t+1)
     (dot products of the mean vectors, as jnp's @ on 1-D arrays evaluates them). Returns
-    (means (T, d), covs (T, d, d), lag_ones (T-1, d, d))."""
+    (means (T, d), covs (T, d, d), lag_ones (T-1, d, d)). Differentiable in filter_output (then step by step)."""
     dev = mr.default_device()
     f_mus, f_covs = filter_output if filter_output is not None else run_kalman_filter_for_marginals(lgssm, y, t)
     f_mus = torch.as_tensor(f_mus, dtype=torch.float64, device=dev)

@@ -86,3 +86,37 @@ def test_mismatched_smoother():
     A = torch.as_tensor(_model(3, 2).transition_matrix)
     J = fc @ A.T @ torch.linalg.inv(A @ fc @ A.T + 0.2)
     assert torch.allclose(one[1][1], fc + J @ (f[1][2] - A @ fc @ A.T - 0.2) @ J.T, rtol=1e-12, atol=1e-13)
+
+
+def _smooth(md, means, covs):
+    return filtering.run_kalman_smoother_for_marginals_and_lag_ones(md, np.zeros((3, 2)), filter_output=(means, covs))
+
+
+def test_smoother_is_differentiable_in_the_filter():
+    md = _model(2, 2)
+    g = torch.Generator().manual_seed(0)
+    means = torch.randn((3, 2), dtype=torch.float64, generator=g)
+    covs = torch.eye(2, dtype=torch.float64).expand(3, 2, 2).contiguous()
+    with pytest.raises(_Kernel):
+        _smooth(md, means, covs)
+    f = lambda m, c: sum(t.sum() for t in _smooth(md, m, c))
+    inputs = (means.clone().requires_grad_(), covs.clone().requires_grad_())
+    assert torch.autograd.gradcheck(f, inputs, check_forward_ad=True)
+    with torch.no_grad(), pytest.raises(_Kernel):  # no graph asked for
+        _smooth(md, *inputs)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(means, torch.ones_like(means))
+        assert torch.autograd.forward_ad.unpack_dual(_smooth(md, dual, covs)[0]).tangent is not None
+
+
+def test_smoother_under_vmap_and_tracing():
+    md = _model(2, 2)
+    means = torch.randn((4, 3, 2), dtype=torch.float64, generator=torch.Generator().manual_seed(1))
+    covs = torch.eye(2, dtype=torch.float64).expand(3, 2, 2).contiguous()
+    many = torch.func.vmap(lambda m: _smooth(md, m, covs)[0])(means)
+    for k in range(4):
+        one = _smooth(md, means[k].requires_grad_(), covs)[0]
+        assert torch.allclose(many[k], one, rtol=1e-12, atol=1e-13)
+    from torch.fx.experimental.proxy_tensor import make_fx
+    traced = make_fx(lambda m: _smooth(md, m, covs)[0])(means[0].detach())
+    assert torch.allclose(traced(means[1].detach()), many[1], rtol=1e-12, atol=1e-13)
