@@ -449,13 +449,13 @@ int mocat_ksd_batch_rows(const float* x, const float* grad_potential, const floa
  * (m_pad x m_pad each), m0 (m_pad), y (T x m_pad), both dimensions padded to m_pad = max(d, dy) <= 8 (padding
  * states A = 0, Q = P0 = 1, padding observations H = 0, R = 1, y = 0). means [T][d], covs [T][d][d], loglik: one
  * value; scratch: T (m_pad + 1) doubles; *info (device) = 1 when an innovation covariance is not positive
- * definite (the outputs are then not defined), else 0. */
+ * definite or P0 or Q is not symmetric (the outputs are then not defined), else 0. */
 int mocat_kalman_filter(const double* model, int m_pad, int64_t T, int d, int dy, double* means, double* covs,
                         double* loglik, double* scratch, int* info, hipStream_t stream);
 /* Rauch-Tung-Striebel smoother with mocat's lag-one terms (kalman.py:60-98) from filter means [T][d] and
  * covariances [T][d][d]: means, covs, lag_ones [T-1][d][d]; scratch: 2 (T - 1) m_pad^2 doubles; model: A, Q
  * (m_pad x m_pad, padded as above); *info (device, zeroed by the caller) is set to 1 when a predicted covariance is not
- * positive definite. */
+ * positive definite or Q or a filter covariance is not symmetric. */
 int mocat_kalman_smoother(const double* model, int m_pad, int64_t T, int d, const double* filter_means,
                           const double* filter_covs, double* means, double* covs, double* lag_ones, double* scratch,
                           int* info, hipStream_t stream);

@@ -30,6 +30,16 @@ MOCAT_DEV void each(F f) {
   }
 }
 
+// Whether each lane's elements of a covariance (LDS) equal their mirror images but for rounding.
+template <int M>
+MOCAT_DEV bool symmetric(const double* s) {
+  bool ok = true;
+  each<M>([&](int i, int j, int e) {
+    ok = ok && !(fabs(s[e] - s[j * M + i]) > 1e-9 * (fabs(s[i * M + i]) + fabs(s[j * M + j])));
+  });
+  return ok;
+}
+
 // Lower Cholesky factor of the symmetric matrix s (LDS, lower triangle read) in registers, diagonal as
 // its reciprocal too; false if it is not positive definite (or not a number).
 template <int M>
@@ -73,7 +83,8 @@ MOCAT_DEV void solve(const double (&L)[M][M], const double (&inv)[M], double (&x
 }
 
 // stats: [T][M + 1] scratch (the factors' diagonals and the innovations' quadratic forms, whose logarithms are
-// summed at the end, off the serial path); info: set to 1 when an innovation covariance has no Cholesky factor.
+// summed at the end, off the serial path); info: set to 1 when an innovation covariance has no Cholesky factor, and when
+// P0 or Q, whose symmetry the gain uses, is not symmetric.
 template <int M>
 __global__ __launch_bounds__(kWave) void kalman_filter_kernel(KfModel g, int64_t T, int d, int dy, double* means,
                                                               double* covs, double* loglik, double* stats, int* info) {
@@ -88,7 +99,8 @@ __global__ __launch_bounds__(kWave) void kalman_filter_kernel(KfModel g, int64_t
     P[e] = g.P0[e];
   });
   if (lane < M) m[lane] = g.m0[lane];
-  bool ok = true;
+  __syncthreads();
+  bool ok = symmetric<M>(P) && symmetric<M>(Q);
   double yt = lane < M ? g.y[lane] : 0.0;
   for (int64_t t = 0; t < T; ++t) {
     const double ynext = (lane < M && t + 1 < T) ? g.y[(t + 1) * M + lane] : 0.0;
@@ -184,6 +196,7 @@ __global__ __launch_bounds__(kWave) void kalman_filter_kernel(KfModel g, int64_t
     ll -= 0.5 * q;
   }
   ll = wave_sum(ll);
+  ok = __all(ok);
   if (lane == 0) {
     *loglik = ll;
     *info = ok ? 0 : 1;
@@ -191,14 +204,17 @@ __global__ __launch_bounds__(kWave) void kalman_filter_kernel(KfModel g, int64_t
 }
 
 // One wave per time point t < T - 1: pred = A F_t A^T + Q and the gain J = F_t A^T pred^-1, to [T - 1][M][M] each.
+// J uses F_t = F_t^T and pred = pred^T, and the filter covariances are the caller's: info is also set where F_t or Q is
+// not symmetric.
 template <int M>
 __global__ __launch_bounds__(kWave) void kalman_gain_kernel(KfModel g, int d, const double* f_covs, double* gains,
                                                             double* preds, int* info) {
-  __shared__ double A[M * M], F[M * M], B[M * M], S[M * M];
+  __shared__ double A[M * M], Q[M * M], F[M * M], B[M * M], S[M * M];
   const int lane = threadIdx.x;
   const int64_t t = blockIdx.x;
   each<M>([&](int i, int j, int e) {
     A[e] = g.A[e];
+    Q[e] = g.Q[e];
     F[e] = (i < d && j < d) ? f_covs[(t * d + i) * d + j] : 0.0;
   });
   __syncthreads();
@@ -213,14 +229,14 @@ __global__ __launch_bounds__(kWave) void kalman_gain_kernel(KfModel g, int d, co
     double v = 0.0;
 #pragma unroll
     for (int k = 0; k < M; ++k) v += B[i * M + k] * A[j * M + k];
-    v += g.Q[e];
+    v += Q[e];
     S[e] = v;
     preds[t * M * M + e] = v;
   });
   __syncthreads();
   double L[M][M], inv[M], x[M];
   const bool ok = cholesky<M>(S, L, inv);
-  if (lane == 0 && !ok) *info = 1;
+  if (!ok || !symmetric<M>(F) || !symmetric<M>(Q)) *info = 1;
   if (lane < M) {
 #pragma unroll
     for (int k = 0; k < M; ++k) x[k] = B[k * M + lane];

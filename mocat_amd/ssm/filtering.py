@@ -876,8 +876,8 @@ def _has_shapes(lgssm, **shapes):
 
 
 def _kalman_filter_kernel(lgssm, yn):
-    """The filter in one launch, or None when the dimensions or shapes have no kernel or an innovation covariance
-    has no Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
+    """The filter in one launch, or None when the dimensions or shapes have no kernel or the kernel finds a covariance
+    that is not symmetric or an innovation covariance without a Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
     observations H = 0, R = 1, y = 0."""
     T, dy = yn.shape
     d = int(np.prod(np.shape(lgssm.initial_mean)))
@@ -934,16 +934,17 @@ def run_kalman_filter_for_marginals(lgssm, y, t=None):
 
 
 def _recorded(*tensors):
-    """Whether a gradient, a tangent, a functorch transform (vmap, grad, jvp) or a trace follows these: the kernels
-    leave nothing for them to record."""
-    return torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0 or any(
-        t.requires_grad and torch.is_grad_enabled() or torch._C._functorch.is_functorch_wrapped_tensor(t)
-        or torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+    """Whether a gradient, forward mode, a functorch transform (vmap, grad, jvp) or a trace may follow these: the
+    kernels leave nothing for them to record."""
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0)
 
 
 def _kalman_smoother_kernel(lgssm, f_mus, f_covs):
     """The smoother in three launches, or None when the dimension or shapes have no kernel, the filter's moments are
-    differentiated or traced, or a predicted covariance has no Cholesky factor."""
+    differentiated or traced, or the kernels find a covariance that is not symmetric or a predicted one without a
+    Cholesky factor."""
     if f_mus.dim() != 2 or _recorded(f_mus, f_covs):
         return None
     T, d = f_mus.shape
