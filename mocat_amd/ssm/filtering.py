@@ -826,7 +826,8 @@ def run_particle_filters(ssm_scenarios, ys, random_keys, ns, ess_threshold: floa
         if schedule == "auto":
             run = lambda c: _launch(models, ys, keys, ns, ess_threshold, resampling, store, grad, c["large_n"],
                                     particle_filter, launch_mode=sched.launch_mode(c), ts=ts)
-            choice = sched.choose(sched.signature(models, ys, ns, resampling, grad, store, particle_filter), run)
+            sig = sched.signature(models, ys, ns, resampling, grad, store, particle_filter, ess_threshold)
+            choice = sched.choose(sig, run)
         elif isinstance(schedule, dict):
             choice = schedule
         else:

@@ -2,12 +2,12 @@
 
 A batch of independent filters of uneven sizes is split between two launch structures: filters below
 a particle-count threshold run one workgroup each in a single persistent launch; the others run on the
-chunked path (1024-particle chunks spread over the GPU, three grid-wide phases per time step), either
-as the launches per step queued one by one ("stream"), those launches captured into one HIP graph
+chunked path (1024-particle chunks spread over the GPU, two grid-wide phases per time step, or one over 256-particle
+chunks when all of them are small), either as the launches per step queued one by one ("stream"), those launches captured into one HIP graph
 ("graph"), or one persistent kernel with grid barriers between the phases ("persistent"). Which split
 and which launch mode is fastest depends on the batch (its size distribution and lengths), so the
 tuner times every candidate schedule on the batch itself, keeps the fastest, and records it under the
-batch's shape signature: in memory for the process and in a JSON file ($MOCAT_AMD_SCHEDULE_CACHE, else
+batch's signature (sizes, outputs, kernels, device): in memory for the process and in a JSON file ($MOCAT_AMD_SCHEDULE_CACHE, else
 ~/.cache/mocat_amd/pf_schedule.json) for later processes. Results do not depend on the schedule (the
 filters' key trees and arithmetic are the same on both paths), so tuning changes only the time.
 """
@@ -28,6 +28,9 @@ CANDIDATE_LARGE_N = (1, 1024, 2048, 4096, 8192, 16384)  # 1: every filter on the
 CANDIDATE_LAUNCH = ("stream", "graph")
 LAUNCH_MODES = {"stream": 0, "graph": 1, "persistent": 2}
 
+# counts the changes of the filters' step kernels or launches, so that a record is used with the launches it was timed on
+KERNEL_VERSION = 2
+
 _MEMO: dict = {}
 
 
@@ -45,13 +48,23 @@ def cache_path() -> Path:
     return Path(p) if p else Path.home() / ".cache" / "mocat_amd" / "pf_schedule.json"
 
 
-def signature(models, ys, ns, resampling, grad, store, particle_filter) -> str:
-    """Model class and dimensions, resampling, outputs, and the sorted (n, T) pairs of the batch."""
+def _device() -> str:
+    """Name and compute units (fewer in a partition) of the current device."""
+    if not torch.cuda.is_available():
+        return "cpu"
+    p = torch.cuda.get_device_properties(torch.cuda.current_device())
+    return f"{p.name}/{p.multi_processor_count}"
+
+
+def signature(models, ys, ns, resampling, grad, store, particle_filter, ess_threshold: float = 1.0) -> str:
+    """Kernel version, device, model class and dimensions, resampling (how often, too), outputs, and the sorted
+    (n, T) pairs of the batch."""
     m0 = models[0]
     shapes = np.asarray(sorted((int(n), int(np.asarray(y).shape[0])) for n, y in zip(ns, ys)), np.int64)
     h = hashlib.sha1(shapes.tobytes()).hexdigest()[:16]
     pf = "default" if particle_filter is None else getattr(particle_filter, "__name__", type(particle_filter).__name__)
-    return f"{m0.kernel_model}-{m0.dim}-{m0.dim_obs}-{pf}-{resampling}-g{int(bool(grad))}-s{int(bool(store))}-{h}"
+    return (f"k{KERNEL_VERSION}-{_device()}-{m0.kernel_model}-{m0.dim}-{m0.dim_obs}-{pf}-{resampling}"
+            f"-e{float(ess_threshold):g}-g{int(bool(grad))}-s{int(bool(store))}-{h}")
 
 
 def _load() -> dict:
