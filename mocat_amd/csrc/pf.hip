@@ -1046,17 +1046,6 @@ struct LfScratch {
 };
 
 // chunk-level reductions in a fixed order (wave butterflies, then waves in order)
-MOCAT_DEV uint64_t lf_block_sum(uint64_t v, LfScratch& s) {
-  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-  v = wave_sum(v);
-  __syncthreads();
-  if (lane == 0) s.u[w] = v;
-  __syncthreads();
-  uint64_t r = 0;
-  for (int i = 0; i < LW; ++i) r += s.u[i];
-  return r;
-}
-
 MOCAT_DEV uint64_t lf_block_inclusive_scan(uint64_t v, LfScratch& s) {
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const uint64_t incl = wave_inclusive_scan(v);
@@ -1900,10 +1889,7 @@ MOCAT_DEV void lf_step_chunk(const LfArgs& a, int64_t t, int cend_slots, int64_t
         m[pk] = in[pk] ? ((kc[pk] + 1) * SG < n ? (kc[pk] + 1) * SG : n) - 1 - b[pk] : 0;
       }
       int64_t p[PPT];
-      if (staged)
-        upper_bound_lockstep<PPT>([&](int64_t k) { return win[k - lo]; }, b, m, tg, in, p);
-      else
-        upper_bound_lockstep<PPT>(sum_at, b, m, tg, in, p);
+      upper_bound_lockstep<PPT>(sum_at, b, m, tg, in, p);
 #pragma unroll
       for (int pk = 0; pk < PPT; ++pk)
         if (live[pk]) srcs[pk] = in[pk] ? p[pk] : n - 1;

@@ -30,7 +30,6 @@ from .mcmc import Metropolis, check_correction, evaluate
 from .sample import Sampler
 
 _P = _lib.c_ptr
-_lib.register("mocat_gather_rows", [_P, _P, _lib.c_i64, _lib.c_i64, _P, _P])
 _lib.register("mocat_smc_temper", [_P, _P, _lib.c_i64, _lib.c_f64, _lib.c_f64, _lib.c_f64, _lib.c_f64, _lib.c_f64,
                                    _lib.c_i32, _lib.c_i32, _lib.c_f64, _P, _lib.c_i32, _lib.c_f64, _lib.c_f64,
                                    _lib.c_f64, _P, _P, _P])
@@ -43,18 +42,6 @@ _lib.register("mocat_smc_move", [_P, _P, _P, _lib.c_i64, _lib.c_i64, _lib.c_i32,
               + [_lib.c_i32, _lib.c_i32, _lib.c_f32, _P, _P] + [_lib.c_f64] * 7 + [_lib.c_i32, _lib.c_i32]
               + [_lib.c_f64] * 3 + [_P, _P, _P, _lib.c_i64, _lib.c_i32, _P])
 TEMPER_POLLS = 1 << 22  # polls of one wait between the workgroups of the temperature search
-
-
-def gather_rows(t: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
-    """t[idx] along the first axis (4-byte element types)."""
-    t = t.contiguous()
-    if t.element_size() != 4:
-        raise TypeError("gather_rows handles 4-byte element types")
-    out = torch.empty((idx.shape[0], *t.shape[1:]), dtype=t.dtype, device=t.device)
-    width = int(t[0].numel()) if t.dim() > 1 else 1
-    _lib.call("mocat_gather_rows", _lib.ptr(t), _lib.ptr(idx), int(idx.shape[0]), width, _lib.ptr(out),
-              _lib.stream_handle())
-    return out
 
 
 class TransportSampler(Sampler):
