@@ -861,6 +861,8 @@ KALMAN_MAX_DIM = 8  # the Kalman kernels' largest state or observation dimension
 def _padded(a, m_pad, diag=0.0):
     """a in the upper left of an m_pad x m_pad FP64 matrix, diag on the diagonal below its rows."""
     a = np.asarray(a, np.float64)
+    if a.shape == (m_pad, m_pad):
+        return a
     out = np.diag(np.where(np.arange(m_pad) < a.shape[0], 0.0, diag))
     out[:a.shape[0], :a.shape[1]] = a
     return out
@@ -878,8 +880,8 @@ def _has_shapes(lgssm, **shapes):
 
 def _kalman_filter_kernel(lgssm, yn):
     """The filter in one launch, or None when the dimensions or shapes have no kernel or the kernel finds a covariance
-    that is not symmetric or an innovation covariance without a Cholesky factor. Both dimensions are padded to the larger: padding states A = 0, Q = P0 = 1, padding
-    observations H = 0, R = 1, y = 0."""
+    that is not symmetric or an innovation covariance without a Cholesky factor. Both dimensions are padded to the
+    larger: padding states A = 0, Q = P0 = 1, padding observations H = 0, R = 1, y = 0."""
     T, dy = yn.shape
     d = int(np.prod(np.shape(lgssm.initial_mean)))
     k = max(d, dy)
