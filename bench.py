@@ -587,7 +587,7 @@ def main():
         "error_vs_fp64": err,
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                      "frac": achieved / peak, "traffic": traffic,
-                     "kernel": "hmc_lr_bf16_kernel<64,512>" if a.precision == "bf16x3"
+                     "kernel": "hmc_lr_bf16_kernel<64,512,1>" if a.precision == "bf16x3"
                      else "hmc_lr_kernel<Fp32Engine<64,512>>",
                      "kernel_ms_per_iteration": kernel_ms, "flop_per_iteration": flop_per_launch,
                      "iterations_per_launch": ITERATIONS,

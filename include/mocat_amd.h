@@ -189,13 +189,14 @@ int mocat_pf_run(int model, int d, int dy, const mocat_pf_filter* host_filters, 
                  float* tan_ws1, double* out_grad, hipStream_t stream);
 
 /* The same filters (same run_particle_filter_for_marginals semantics, outputs and workspaces as
- * mocat_pf_run) for those flagged MOCAT_PF_LARGE, spread over the whole GPU: per time step three
+ * mocat_pf_run) for those flagged MOCAT_PF_LARGE, spread over the whole GPU: per time step two
  * grid-wide launches over 1024-particle chunks, all flagged filters batched in each (the previous
- * step's statistics, resampling decision and quantised weight totals; exact prefix sums; ancestor
- * search, propagation and weighting), or one over 256-particle chunks when no flagged filter has more
- * than 4096 particles (launch modes 0 and 1); categorical resampling adds a launch of its draws. For the same log-weights and key the ancestors equal mocat_pf_run's. host_filters is a
- * host array (the launch sequence depends on n and T); workspace holds
- * mocat_pf_large_workspace_bytes bytes, including T step-key slots per flagged filter (independent of
+ * step's statistics, resampling decision and each chunk's quantised prefix sums; ancestor search,
+ * propagation and weighting), with one more for the chunk offsets when a filter has more than 1024 chunks;
+ * or one over 256-particle chunks when no flagged filter has more than 4096 particles and the sum of their
+ * n^2 is at most 1.5e9 (launch modes 0 and 1). Categorical resampling adds a launch of its draws. For the
+ * same log-weights and key the ancestors equal mocat_pf_run's. host_filters is a host array (the launch
+ * sequence depends on n and T); workspace holds mocat_pf_large_workspace_bytes bytes, including T step-key slots per flagged filter (independent of
  * t_offset, which only places out_ess / out_loglik_t and must be >= 0 when either is given).
  * launch_mode 0 queues the per-step launches on the stream; 1 captures them into one HIP graph,
  * launches it on the stream and returns after it has run (when the stream is already being captured

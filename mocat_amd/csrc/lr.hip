@@ -310,12 +310,15 @@ MOCAT_DEV void split_bf16(float v, __bf16& hi, __bf16& lo) {
 // the 32-row blocks rb = w + NW j; two waves per SIMD (NW = 8) let one wave's row functions on the
 // vector ALU overlap the other's MFMAs.
 //
-// A workgroup takes NCT tiles of 32 chains. What bounds one tile is the first-level cache: every wave streams its
+// A workgroup takes NCT tiles of 32 chains. What bounds one tile most is the first-level cache: every wave streams its
 // blocks' operands through it at 64 B per clock, 32 KB per 32 rows at d > 64 (2050 clocks for four waves, their
-// MFMAs 1540) and 16 KB at d <= 64 (2050 clocks for eight waves, the MFMAs 1540); leaving out the transcendentals or
-// taking the operands from a hot line changes little there, and neither do two blocks at once per wave (slower) or
-// waves out of phase. Two tiles use each operand twice and are bound by the matrix cores: 309 TFLOP/s algorithmic at
-// d = 100 is 1190 TFLOP/s issued, where a large bf16 product reaches 1344. (One MFMA for the last columns' three
+// MFMAs 1540) and 16 KB at d <= 64 (2050 clocks for eight waves, the MFMAs 1540), and each block's labels another quarter
+// of that at d <= 64 (16 bytes a lane, four times). Counters of the moves at d = 50: 0.8 accesses of 64 B a clock in
+// the block loop, the return path busy 83% of all clocks, vector ALU 50%, matrix pipe 43%. Leaving out the
+// transcendentals or taking the operands from a hot line changes little there, and neither do two blocks at once per wave
+// (slower) or waves out of phase. Two tiles use each operand twice (0.39 accesses a clock); then the one wave per SIMD takes
+// turns between the vector ALU (52% of the clocks) and the matrix pipe (50%), one of them busy in 83%: 288-309 TFLOP/s
+// algorithmic at d = 100, 1105-1190 issued, where a large bf16 product reaches 1320-1344. (One MFMA for the last columns' three
 // products, at d = 50 and 100 10 instead of 12 and 19 instead of 24 per block, would give another 6%, but sums them in
 // another order: chains of 200 leapfrog steps then end up to 3e-5 from where they ended before.)
 template <int DP, int NT, int NCT>

@@ -520,7 +520,7 @@ def _launch(models, ys, keys, ns, ess_threshold, resampling, store, grad=False, 
             initial=None, extra_flags=0, launch_mode=0, ts=None):
     """Runs len(models) filters (same model class and dims): filters below large_n particles in one
     persistent launch (a workgroup per filter), the others through the chunked per-step path
-    (launch_mode 0: three stream launches per step; 1: those launches captured into one HIP graph;
+    (launch_mode 0: stream launches, one to three per step; 1: those launches captured into one HIP graph;
     2: one persistent kernel for all steps)."""
     m0 = models[0]
     d, dy, kind = m0.dim, m0.dim_obs, m0.kernel_model

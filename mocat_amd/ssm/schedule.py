@@ -2,12 +2,13 @@
 
 A batch of independent filters of uneven sizes is split between two launch structures: filters below
 a particle-count threshold run one workgroup each in a single persistent launch; the others run on the
-chunked path (1024-particle chunks spread over the GPU, two grid-wide phases per time step, or one over 256-particle
-chunks when all of them are small), either as the launches per step queued one by one ("stream"), those launches captured into one HIP graph
-("graph"), or one persistent kernel with grid barriers between the phases ("persistent"). Which split
-and which launch mode is fastest depends on the batch (its size distribution and lengths), so the
-tuner times every candidate schedule on the batch itself, keeps the fastest, and records it under the
-batch's signature (sizes, outputs, kernels, device): in memory for the process and in a JSON file ($MOCAT_AMD_SCHEDULE_CACHE, else
+chunked path (1024-particle chunks spread over the GPU, two grid-wide phases per time step, or one over
+256-particle chunks when all of them are small), either as the launches per step queued one by one
+("stream"), those launches captured into one HIP graph ("graph"), or one persistent kernel with grid
+barriers between the phases ("persistent"). Which split and which launch mode is fastest depends on the
+batch (its size distribution and lengths), so the tuner times every candidate schedule on the batch
+itself, keeps the fastest, and records it under the batch's signature (sizes, outputs, kernels, device):
+in memory for the process and in a JSON file ($MOCAT_AMD_SCHEDULE_CACHE, else
 ~/.cache/mocat_amd/pf_schedule.json) for later processes. Results do not depend on the schedule (the
 filters' key trees and arithmetic are the same on both paths), so tuning changes only the time.
 """
